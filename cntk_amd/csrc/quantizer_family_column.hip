@@ -67,10 +67,10 @@ struct StripeColLauncher
 
 template <bool ZT, int PER>
 inline void launch_quantize_col(hipStream_t s, LaunchEvents ev, const float* g, const float* r_in, float* r_out, char* q, uint32_t cols,
-                                uint64_t qcol)
+                                uint64_t qcol, bool runs)
 {
     hipExtLaunchKernelGGL((quantize_col_kernel<ZT, PER>), dim3(cols), dim3(kColThreads), col_lds_bytes<PER>(), s, ev.start, ev.stop, 0, g,
-                          r_in, r_out, q, qcol);
+                          r_in, r_out, q, qcol, runs ? 1u : 0u);
 }
 
 template <bool ZT, int PER>
@@ -92,14 +92,14 @@ hipError_t family_col_stripe(size_t nbits, bool zt, hipStream_t s, LaunchEvents 
     return dispatch_nbits<StripeColLauncher>(nbits, zt, s, ev, src, stripe_res, q_out, agg_out, cols, c);
 }
 
-hipError_t family_col_quantize_unrolled(bool zt, int per, hipStream_t s, LaunchEvents ev, const float* g, const float* r_in, float* r_out, char* q, uint32_t cols, uint64_t qcol)
+hipError_t family_col_quantize_unrolled(bool zt, int per, hipStream_t s, LaunchEvents ev, const float* g, const float* r_in, float* r_out, char* q, uint32_t cols, uint64_t qcol, bool runs)
 {
     if (per == 1)
-        zt ? launch_quantize_col<true, 1>(s, ev, g, r_in, r_out, q, cols, qcol) : launch_quantize_col<false, 1>(s, ev, g, r_in, r_out, q, cols, qcol);
+        zt ? launch_quantize_col<true, 1>(s, ev, g, r_in, r_out, q, cols, qcol, runs) : launch_quantize_col<false, 1>(s, ev, g, r_in, r_out, q, cols, qcol, runs);
     else if (per == 2)
-        zt ? launch_quantize_col<true, 2>(s, ev, g, r_in, r_out, q, cols, qcol) : launch_quantize_col<false, 2>(s, ev, g, r_in, r_out, q, cols, qcol);
+        zt ? launch_quantize_col<true, 2>(s, ev, g, r_in, r_out, q, cols, qcol, runs) : launch_quantize_col<false, 2>(s, ev, g, r_in, r_out, q, cols, qcol, runs);
     else if (per == 4)
-        zt ? launch_quantize_col<true, 4>(s, ev, g, r_in, r_out, q, cols, qcol) : launch_quantize_col<false, 4>(s, ev, g, r_in, r_out, q, cols, qcol);
+        zt ? launch_quantize_col<true, 4>(s, ev, g, r_in, r_out, q, cols, qcol, runs) : launch_quantize_col<false, 4>(s, ev, g, r_in, r_out, q, cols, qcol, runs);
     else
         return hipErrorInvalidValue;
     return hipGetLastError();

@@ -197,25 +197,10 @@ __device__ __forceinline__ void quantize_col_body(const float* __restrict__ g, c
 
 template <bool ZT, int PER>
 __global__ __launch_bounds__(kColThreads) void quantize_col_kernel(const float* __restrict__ g, const float* r_in, float* r_out,
-                                                                   char* __restrict__ q, uint64_t qcol)
+                                                                   char* __restrict__ q, uint64_t qcol, uint32_t runs)
 {
     extern __shared__ f32x4 smem_v4[];
-    quantize_col_body<ZT, PER>(g, r_in, r_out, q, qcol, blockIdx.x, smem_v4);
-}
-
-// Consecutive workgroups go to the device's eight dies in turn, each die with an L2 of its own. A packed column record is
-// not a whole number of 128-byte lines (264 bytes at 2048 rows), so neighbouring columns share lines, and neighbours on
-// different dies fetch such a line into two L2s (2048 x 9304, eight workers: 29 MB read for 19.6 MB of packed stripes).
-// Runs of 16 consecutive columns therefore go to one die; the eight dies still walk through memory side by side, a
-// megabyte of residual at a time. Maps workgroup b of n to its column (the last n % 128 keep their index).
-__device__ __forceinline__ uint32_t column_of_workgroup(uint32_t b, uint32_t n)
-{
-    constexpr uint32_t RUN = 16, DIES = 8;
-    const uint32_t whole = n - n % (RUN * DIES);
-    if (b >= whole)
-        return b;
-    const uint32_t die = b % DIES, slot = b / DIES;
-    return ((slot / RUN) * DIES + die) * RUN + slot % RUN;
+    quantize_col_body<ZT, PER>(g, r_in, r_out, q, qcol, runs != 0 ? column_of_workgroup(blockIdx.x, gridDim.x) : blockIdx.x, smem_v4);
 }
 
 // Stripe reduction in the same shape, up to eight workers: the sum of an element is one of 256 values, picked by the

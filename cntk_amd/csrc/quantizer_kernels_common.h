@@ -31,6 +31,26 @@ constexpr uint32_t kTileScratchFloats = 12;
 constexpr uint32_t kTileMaxCols = 32;
 constexpr uint32_t kTilePrefixFloats = kTileScratchFloats + 2 * kTileMaxCols; // 76 floats = 304 B (16-B multiple)
 
+// Consecutive workgroups go to the device's eight dies in turn, each die with an L2 of its own. A packed column record is
+// not a whole number of 128-byte lines (264 bytes at 2048 rows), so neighbouring columns share lines, and neighbours on
+// different dies fetch such a line into two L2s (2048 x 9304, eight workers: 29 MB read for 19.6 MB of packed stripes).
+// Runs of 16 consecutive columns therefore go to one die; the eight dies still walk through memory side by side, a
+// megabyte of residual at a time. Maps workgroup b of n to its column (the last n % 128 keep their index).
+__device__ __forceinline__ uint32_t column_of_workgroup(uint32_t b, uint32_t n)
+{
+    constexpr uint32_t RUN = 16, DIES = 8;
+    const uint32_t whole = n - n % (RUN * DIES);
+    if (b >= whole)
+        return b;
+    const uint32_t die = b % DIES, slot = b / DIES;
+    return ((slot / RUN) * DIES + die) * RUN + slot % RUN;
+}
+// A packed matrix in host memory: the quantize kernels with a workgroup per column deal their columns in these runs too. The
+// L2 puts the pieces of a line that two neighbours write together before the line crosses the bus, if both write to the same
+// L2 (2048 x 9304 at 1 bit, 2.46 MB: 82 us with neighbours on different dies, 64 us so; 2049 x 9304 77 and 73 us; into
+// device memory 36 and 37 us, so there a workgroup's index stays its column. Tiles of short columns and columns of doubles,
+// whose records or runs of records are several lines, measured the same either way).
+
 // A QWord is assembled from work items of at most 8 bit positions each, so that a tile with few QWords
 // still keeps every thread busy; the partial words meet in LDS (atomic OR). WORD_BITS: 32 for float columns, 64 for double.
 template <int NBITS, int WORD_BITS>

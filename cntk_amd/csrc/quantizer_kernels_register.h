@@ -22,6 +22,7 @@ struct RegGeom
     uint32_t step_k; // (4 * T) / nq: a thread's next piece lies this many bit positions ...
     uint32_t step_w; // (4 * T) % nq: ... and this many QWords further on
     uint32_t line_shift; // non-zero: slots are dealt so that wavefronts cover whole 128-byte lines (see column_shift)
+    uint32_t runs;   // non-zero: columns are dealt by column_of_workgroup (packed matrix in host memory)
     uint64_t qcol;
 };
 
@@ -287,7 +288,7 @@ __global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(reg_waves<T, 
     const float* __restrict__ g, const float* r_in, float* r_out, char* __restrict__ q, RegGeom c)
 {
     extern __shared__ f32x4 smem_v4[];
-    quantize_reg_body<NBITS, ZT, T, PER, EDGE>(g, r_in, r_out, q, c, blockIdx.x, smem_v4);
+    quantize_reg_body<NBITS, ZT, T, PER, EDGE>(g, r_in, r_out, q, c, c.runs != 0 ? column_of_workgroup(blockIdx.x, gridDim.x) : blockIdx.x, smem_v4);
 }
 
 // Stripe reduction for tall columns (above the LDS kernels' 14336 rows), in the register kernel's shape: 1024 threads per

@@ -69,6 +69,7 @@ struct LaunchTuning
     uint32_t unq_slots = 0; // 0 = default; else bit positions per thread in unquantize
     int unq_mode = 0; // 0 automatic, 1 QWord-major with 4-byte stores, 2 / 4 / 5 tile / row-major / LDS-free row-major decoder wherever it can run, 3 automatic without the tile decoder
     bool unq_member = false; // the matrix is decoded as a member of a gradient-set launch
+    bool packed_on_host = false; // the packed matrix is written to or read out of pinned host memory
 };
 
 // Events tied to the kernel dispatch itself (its completion signal), not recorded as separate stream
@@ -161,7 +162,7 @@ hipError_t family_col_quantize(size_t nbits, bool zt, hipStream_t s, LaunchEvent
                                uint32_t cols, ColGeom c);
 // per: 1, 2 or 4 pieces per thread (1024, 2048, 4096 rows at 1 bit)
 hipError_t family_col_quantize_unrolled(bool zt, int per, hipStream_t s, LaunchEvents ev, const float* g, const float* r_in, float* r_out, char* q,
-                                        uint32_t cols, uint64_t qcol);
+                                        uint32_t cols, uint64_t qcol, bool runs);
 hipError_t family_col_stripe(size_t nbits, bool zt, hipStream_t s, LaunchEvents ev, const StripeSources& src, float* stripe_res, char* q_out,
                              float* agg_out, uint32_t cols, ColGeom c);
 hipError_t family_col_stripe_unrolled(bool zt, int per, hipStream_t s, LaunchEvents ev, const StripeSources& src, float* stripe_res, char* q_out,
@@ -263,6 +264,7 @@ inline RegGeom make_reg_geom(size_t rows, size_t nbits, uint32_t threads, bool l
     c.step_k = (4 * threads) / c.nq;
     c.step_w = (4 * threads) % c.nq;
     c.line_shift = line_shift ? 1u : 0u;
+    c.runs = 0;
     c.qcol = qcol_bytes(nbits, rows);
     return c;
 }
@@ -640,6 +642,7 @@ inline hipError_t launch_quantize(hipStream_t s, LaunchEvents ev, const float* g
 {
     zt = zt && (nbits == 1);
     char* qc = static_cast<char*>(q);
+    const uint32_t runs = tune.packed_on_host ? 1u : 0u;
     int path = tune.quantize_path;
     if (path == kPathAuto)
     {
@@ -661,14 +664,16 @@ inline hipError_t launch_quantize(hipStream_t s, LaunchEvents ev, const float* g
                 return hipErrorInvalidValue;
             const uint32_t threads = reg_edge_threads(rows);
             RegGeom c = make_reg_geom(rows, nbits, threads, true); // always dealt by the residual's lines
+            c.runs = runs;
             return family_reg_edge_quantize(nbits, zt, s, ev, g, r_in, r_out, qc, (uint32_t) cols, c, threads);
         }
         const uint32_t threads = reg_threads(rows);
         // up to 14336 rows the shift is part of the summation order all column kernels share; above, it is used where
         // the registers allow
         const bool line_shift = quantize_line_shift(g, r_in, r_out, rows) && (threads == 256 || rows / 4 + 7 <= 1024 * (size_t) kRegMaxShiftPer);
-        return family_reg_quantize(nbits, zt, s, ev, g, r_in, r_out, qc, (uint32_t) cols,
-                                           make_reg_geom(rows, nbits, threads, line_shift), threads);
+        RegGeom c = make_reg_geom(rows, nbits, threads, line_shift);
+        c.runs = runs;
+        return family_reg_quantize(nbits, zt, s, ev, g, r_in, r_out, qc, (uint32_t) cols, c, threads);
     }
     if (path == kPathStrip)
         return launch_strip_quantize<float>(s, ev, g, r_in, r_out, qc, rows, cols, nbits, zt, tune);
@@ -693,7 +698,7 @@ inline hipError_t launch_quantize(hipStream_t s, LaunchEvents ev, const float* g
             return family_col_quantize(nbits, zt, s, ev, g, r_in, r_out, qc, (uint32_t) cols, make_col_geom(rows, nbits, line_shift));
         const uint64_t qcol = qcol_bytes(nbits, rows);
         const uint32_t c = (uint32_t) cols;
-        return family_col_quantize_unrolled(zt, rows == 1024 ? 1 : (rows == 2048 ? 2 : 4), s, ev, g, r_in, r_out, qc, c, qcol);
+        return family_col_quantize_unrolled(zt, rows == 1024 ? 1 : (rows == 2048 ? 2 : 4), s, ev, g, r_in, r_out, qc, c, qcol, runs != 0);
     }
     if (path == kPathTile)
     {
@@ -910,6 +915,16 @@ inline UnquantizePlan plan_unquantize(const void* q, const float* out, size_t ro
     const bool direct_auto = direct_can && (rows >= 16384 || (!vec_ideal && nbits >= 2 && rows >= 8192 && direct_full) ||
                                             (vec_ideal && nbits <= 2 && rows % direct_chunk == 0 && rows <= 8192 && !tune.unq_member));
     bool vec = false, rowmajor = false, tile = false, seg_allowed = true, direct = false;
+    // A packed matrix in host memory: every 128-byte line crosses the bus as often as a workgroup or a wavefront asks for it
+    // (no cache of the device holds host memory), so the decoder is the one that asks once. From 256 QWords per column on,
+    // a wavefront's 16-byte loads of the LDS-free row-major decoder meet no QWord twice; below, the tile decoder takes the
+    // records of several columns into LDS as one run (a record alone is not a whole number of lines), given columns enough
+    // for a workgroup per compute unit. Decoded out of host memory, against the decoder that the same matrix gets in device
+    // memory: 2048 x 9304 at 1 bit 97 -> 60 us (2.46 MB, 48 us on the bus), 9304 x 2048 245 -> 55 us, 1000 x 20000
+    // 106 -> 63 us, 1152 x 10378 at 8 bits 322 -> 247 us (12 MB).
+    const bool host_auto = tune.packed_on_host && mode == 0 && slots_free;
+    const bool host_direct = host_auto && direct_can && nq >= 256;
+    const bool host_tile = host_auto && !host_direct && tile_can && (rows < kUnqRowsMinRows || cols >= 4 * 256);
     // The LDS-free decoder for short columns, wherever it can run below 10000 rows: in a launch of its
     // own it measured 4 to 24 % faster than the tile, row-major and QWord-major decoders it replaces (512 x 100000: 38.3 ->
     // 33.7 us, 576 x 16384 at 2 bits 9.1 -> 7.0 us, 64 x 400000 at 8 bits 22.9 -> 19.4 us, 1536 x 12288 13.4 -> 12.1 us,
@@ -917,7 +932,7 @@ inline UnquantizePlan plan_unquantize(const void* q, const float* out, size_t ro
     // even at 512 x 40000 and 2304 x 4096 at 4 bits). As a member of a gradient-set launch only a large matrix (4 M elements)
     // gains (the LSTM set's decode with its 512 x 100000 and 1024 x 4096 members: 80.6 -> 69.4 us); ResNet-50's 161 members
     // and the 2048 x 1163 stripes of the all-reduce measured 5 to 7 % slower with it and keep their decoders.
-    const bool flat_auto = mode == 0 && !direct_auto && rows < 10000 && // (9304 x 2048: 14.4 -> 13.7 us; even from 10000 rows on)
+    const bool flat_auto = mode == 0 && !host_direct && !host_tile && !direct_auto && rows < 10000 && // (9304 x 2048: 14.4 -> 13.7 us; even from 10000 rows on)
                            (!tune.unq_member || (uint64_t) rows * cols >= ((uint64_t) 1 << 22));
     if ((mode == 6 || flat_auto) && slots_free && out16 && make_unq_flat_geom(p.flat, rows, cols, nq, qcol_bytes(nbits, rows), 4))
     {
@@ -928,6 +943,10 @@ inline UnquantizePlan plan_unquantize(const void* q, const float* out, size_t ro
     }
     if (mode == 5 && direct_can)
         direct = true;
+    else if (host_direct)
+        direct = true;
+    else if (host_tile)
+        tile = true;
     else if (mode == 0 && direct_auto)
         direct = true;
     else if (mode == 1)

@@ -147,6 +147,7 @@ inline RegGeom make_reg_geom(size_t rows, size_t nbits, bool line_shift)
     c.step_k = (2 * kRegThreads) / c.nq;
     c.step_w = (2 * kRegThreads) % c.nq;
     c.line_shift = line_shift ? 1u : 0u;
+    c.runs = 0;
     c.qcol = qcol_bytes(nbits, rows);
     return c;
 }
@@ -469,7 +470,11 @@ inline UnquantizePlan64 plan_unquantize(const double* out, size_t rows, size_t c
     // is 13 % slower with it than with the packed column in LDS)
     // (QWord counts that are odd stay with the tile and row-major decoders here: 1000 x 10000 at 8 bits and 200 x 100000 at 2
     // bits were 11 % slower with it, 576 x 16384 at 1 bit 10 % faster)
-    const bool flat_auto = mode == 0 && !direct_auto && rows <= 2048 && nq % 2 == 0 &&
+    // (a packed matrix in host memory: the rule of the float side, by the bytes of a QWord)
+    const bool host_auto = tune.packed_on_host && mode == 0 && tune.unq_slots == 0;
+    const bool host_direct = host_auto && direct_can && nq >= 128;
+    const bool host_tile = host_auto && !host_direct && tile_can && (rows < kUnqRowsMinRows64 || cols >= 4 * 256);
+    const bool flat_auto = mode == 0 && !host_direct && !host_tile && !direct_auto && rows <= 2048 && nq % 2 == 0 &&
                            (!tune.unq_member || (uint64_t) rows * cols >= ((uint64_t) 1 << 22));
     if ((mode == 6 || flat_auto) && tune.unq_slots == 0 && out16 && make_unq_flat_geom(p.flat, rows, cols, nq, qcol_bytes(nbits, rows), 2))
     {
@@ -479,7 +484,7 @@ inline UnquantizePlan64 plan_unquantize(const double* out, size_t rows, size_t c
         return p;
     }
     bool use_rows = false, use_tile = false;
-    if ((mode == 5 && direct_can) || (mode == 0 && direct_auto))
+    if ((mode == 5 && direct_can) || host_direct || (mode == 0 && !host_tile && direct_auto))
     {
         if (make_unq_direct_geom(p.rowg, rows, cols, nq, qcol_bytes(nbits, rows), 2))
         {
@@ -489,7 +494,7 @@ inline UnquantizePlan64 plan_unquantize(const double* out, size_t rows, size_t c
             return p;
         }
     }
-    else if (mode == 2 && tile_can)
+    else if ((mode == 2 && tile_can) || host_tile)
         use_tile = true;
     else if (mode == 4 && rows_can)
         use_rows = true;

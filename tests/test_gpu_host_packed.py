@@ -1,0 +1,70 @@
+"""Packed matrices in host memory: pinned memory is written and read by the kernels where it lies, pageable memory goes through
+the handle's staging buffer. Either way the bytes are those of a packed matrix in device memory (whose parity with the oracle
+the other files check), and nothing outside the packed matrix is touched."""
+import pytest
+import torch
+
+import cntk_amd
+from cntk_amd import Matrix, MatrixQuantizerImpl, QuantizedMatrix, qcol_bytes
+
+pytestmark = pytest.mark.gpu
+
+# (rows, columns, bits): what decides the kernels -- 255 / 256 QWords per column, columns in runs of 16 x 8 (127 / 128 / 129 /
+# 260), tile decoder against row-major one (1023 / 1024 columns from 1664 rows on), short columns, one column, strips
+SHAPES = [(512, 512, 1), (2048, 127, 1), (2048, 128, 1), (2048, 260, 1), (2048, 1025, 1), (2049, 129, 2), (1664, 1023, 1),
+          (8160, 40, 1), (8192, 40, 1), (1023, 130, 8), (1024, 130, 8), (1, 1, 1), (7, 5000, 4), (147, 999, 1), (20001, 9, 2),
+          (110000, 3, 1), (33, 40, 32)]
+SHAPES_F64 = [(2048, 130, 1), (511, 1025, 1), (8128, 20, 1), (8192, 20, 1), (3, 700, 4), (9001, 17, 8)]
+
+
+def pinned_slice(size, before):
+    """A byte tensor in pinned memory inside a larger allocation, and that allocation."""
+    whole = torch.full((before + size + 256,), 0x5A, dtype=torch.uint8, pin_memory=True)
+    return whole[before:before + size], whole
+
+
+@pytest.mark.parametrize("dedicated", [False, True], ids=["main_stream", "dedicated_stream"])
+@pytest.mark.parametrize("shape", SHAPES, ids=["%dx%d_%dbit" % s for s in SHAPES])
+def test_float(shape, dedicated):
+    check(*shape, torch.float32, dedicated)
+
+
+@pytest.mark.parametrize("shape", SHAPES_F64, ids=["%dx%d_%dbit" % s for s in SHAPES_F64])
+def test_double(shape):
+    check(*shape, torch.float64, False)
+
+
+def check(rows, cols, nbits, dtype, dedicated):
+    qz = MatrixQuantizerImpl.Create(0, dedicated)
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(rows * 131 + cols)
+    size = qcol_bytes(nbits, rows, dtype) * cols
+    n = rows * cols
+    g = torch.randn(n, generator=gen, device="cuda:0", dtype=dtype)
+    G = Matrix(rows, cols, 0, g)
+    before = 8 * 13
+    pinned, whole = pinned_slice(size, before)
+    pageable = torch.zeros(size, dtype=torch.uint8)
+    places = {"device": QuantizedMatrix(rows, cols, nbits, 0, dtype=dtype),
+              "pinned": QuantizedMatrix(rows, cols, nbits, cntk_amd.CPUDEVICE, pinned, dtype=dtype),
+              "pageable": QuantizedMatrix(rows, cols, nbits, cntk_amd.CPUDEVICE, pageable, dtype=dtype)}
+    res = {k: Matrix(rows, cols, dtype=dtype) for k in places}
+    out = {k: Matrix(rows, cols, dtype=dtype) for k in places}
+    torch.cuda.synchronize()
+    for step in range(2):  # the residual carried once, the second result added to the first
+        for k, q in places.items():
+            qz.QuantizeAsync(G, res[k], q, res[k], False)
+            qz.WaitQuantizeAsyncDone()
+            if k == "pinned":
+                # the host may read, move and write back what it was waited for
+                copy = q.buffer.clone()
+                q.buffer.fill_(0)
+                q.buffer.copy_(copy)
+            qz.UnquantizeAsync(q, out[k], add=step > 0)
+            qz.WaitUnquantizeAsyncDone()
+        torch.cuda.synchronize()
+        for k in ("pinned", "pageable"):
+            assert torch.equal(places[k].buffer, places["device"].buffer.cpu()), k
+            assert torch.equal(res[k].data, res["device"].data), k
+            assert torch.equal(out[k].data, out["device"].data), k
+    assert bool((whole[:before] == 0x5A).all()) and bool((whole[before + size:] == 0x5A).all())
