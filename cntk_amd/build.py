@@ -26,7 +26,8 @@ HIPCC_FLAGS = [
 SOURCES = ["quantizer_api.hip", "quantizer_family_tile.hip", "quantizer_family_column.hip", "quantizer_family_register_256.hip",
            "quantizer_family_register_1024.hip", "quantizer_family_register_edge.hip", "quantizer_family_strip.hip",
            "quantizer_family_stripe_register_256.hip", "quantizer_family_stripe_register_1024.hip", "quantizer_family_unquantize.hip",
-           "quantizer_family_batch_quantize.hip", "quantizer_family_batch_stripe.hip", "quantizer_api_f64.hip"]
+           "quantizer_family_batch_quantize.hip", "quantizer_family_batch_stripe.hip", "quantizer_family_batch_register.hip",
+           "quantizer_api_f64.hip"]
 # compilers running at once (a source file takes up to 3 GB while it is compiled)
 JOBS = max(1, min(16, os.cpu_count() or 1, int(os.environ.get("MAX_JOBS", "16"))))
 

@@ -54,6 +54,49 @@ struct BatchAbi<float>
     static BatchTable& unquantize_table(cntkq_quantizer* h) { return h->unquantize_table; }
     static BatchTable& stripe_table(cntkq_quantizer* h) { return h->stripe_table; }
 
+    // The kind of a register grid's member by its pieces per thread; 0: more than the grid's kernels hold.
+    static uint32_t register_kind(uint32_t per, uint32_t threads)
+    {
+        const int* most = threads == 1024 ? kRegBatchPer1024 : kRegBatchPer256;
+        for (uint32_t i = 0; i < 3; ++i)
+            if (per <= (uint32_t) most[i])
+                return 8 + i;
+        return 0;
+    }
+    // Fills the geometry of a member of one of the register grids and names the grid; kBatchOwnLaunch: none of theirs. The slots
+    // are dealt as launch_quantize deals them. few_tall: also a few tall columns that the general grid would stage in memory.
+    static int quantize_register_member(const QItem& it, size_t nbits, QEntry& e, size_t& lds, uint64_t& blocks, bool few_tall)
+    {
+        if (quantize_auto_path(it.in, it.res_in, it.res_out, it.qbuf, it.rows, nbits) != kPathReg)
+            return kBatchOwnLaunch;
+        const bool whole = reg_applicable(it.in, it.res_in, it.res_out, it.qbuf, it.rows, nbits);
+        const uint32_t threads = whole ? reg_threads(it.rows) : reg_edge_threads(it.rows);
+        bool line_shift = true;
+        if (whole)
+            line_shift = quantize_line_shift(it.in, it.res_in, it.res_out, it.rows) &&
+                         (threads == 256 || it.rows / 4 + 7 <= 1024 * (size_t) kRegMaxShiftPer);
+        const RegGeom r = make_reg_geom(it.rows, nbits, threads, line_shift);
+        const uint32_t per = (r.pieces + (r.line_shift ? 7u : 0u) + threads - 1) / threads;
+        // Whole pieces on 256 threads: up to six per thread they are members of the general grid, a few tall columns may be its
+        // members staged in memory, and a large matrix keeps the plain kernel.
+        if (whole && threads == 256 &&
+            (per <= 6 || (it.cols <= kStagedInResidualMaxCols && !few_tall) || it.rows * it.cols >= kOwnLaunchElements))
+            return kBatchOwnLaunch;
+        e.kind = register_kind(per, threads);
+        if (e.kind == 0)
+            return kBatchOwnLaunch;
+        e.r = r;
+        lds = reg_lds_bytes(r);
+        blocks = it.cols;
+        return threads == 256 ? kBatchReg256 : kBatchReg1024;
+    }
+    static bool quantize_entry_wide(const QEntry& e) { return e.kind == 10; }
+    static hipError_t launch_quantize_register_members(hipStream_t s, LaunchEvents ev, const QEntry* de, const uint32_t* db, uint32_t members,
+                                                       uint32_t blocks, size_t lds, size_t nbits, bool zt, uint32_t threads, bool wide)
+    {
+        return family_batch_reg_quantize(nbits, zt && nbits == 1, s, ev, de, db, members, blocks, lds, threads, wide);
+    }
+
     // Fills the geometry of a member of the quantize grid; false: the matrix gets a launch of its own.
     static bool quantize_member(const QItem& it, size_t nbits, QEntry& e, size_t& lds, uint64_t& blocks)
     {
@@ -105,7 +148,7 @@ struct BatchAbi<float>
         }
         return false;
     }
-    static bool first_in_grid(const QEntry& e) { return e.kind == 5; }
+    static bool first_in_grid(const QEntry& e) { return e.kind == 5 || e.kind >= 9; }
     static hipError_t launch_quantize_members(hipStream_t s, LaunchEvents ev, const QEntry* de, const uint32_t* db, uint32_t members,
                                               uint32_t blocks, size_t lds, size_t nbits, bool zt)
     {
@@ -203,9 +246,52 @@ struct BatchAbi<float>
         }
         return true;
     }
+    // Fills the geometry of a member of one of the register grids and names the grid; kBatchOwnLaunch: none of theirs. The slots
+    // are dealt as launch_stripe_reduce deals them.
+    static int stripe_register_member(const SItem& it, size_t workers, size_t nbits, SEntry& e, size_t& lds, uint64_t& blocks)
+    {
+        if (nbits >= 32 || it.rows > stripe_reduce_max_rows(nbits) || (nbits == 1 && workers > 8))
+            return kBatchOwnLaunch;
+        const bool whole = it.rows % 4 == 0 && (reinterpret_cast<uintptr_t>(it.stripe_res) & 15u) == 0;
+        bool line_shift = whole ? !columns_start_on_lines(it.stripe_res, it.rows) : true;
+        uint32_t threads = 256;
+        if (stripe_uses_reg(it.rows, it.stripe_res, nbits))
+        {
+            if (whole && it.rows / 4 + 7 > 1024 * (size_t) kRegMaxShiftPer)
+                line_shift = false;
+            threads = it.rows > kTileMaxRows ? 1024u : reg_edge_threads(it.rows);
+        }
+        else if (!stripe_auto_col(it.rows, it.stripe_res) || stripe_lookup_per(it.rows, line_shift) <= 6 ||
+                 (nbits == 1 ? !stripe_looks_up(it.rows, nbits, workers) : workers > 2 && it.stripe_cols > 64))
+            return kBatchOwnLaunch; // (a member of the general grids)
+        const RegGeom r = make_reg_geom(it.rows, nbits, threads, line_shift);
+        e.kind = register_kind((r.pieces + (r.line_shift ? 7u : 0u) + threads - 1) / threads, threads);
+        if (e.kind == 0)
+            return kBatchOwnLaunch;
+        e.r = r;
+        if (nbits == 1)
+            lds = stripe_lut_lds_bytes(r);
+        else
+        {
+            // as many workers together as leave room for four workgroups of 256 threads, two of 1024, in a compute unit's LDS
+            // (the order of the additions does not depend on it)
+            e.group = stripe_reg_group(r, (uint32_t) workers, threads == 256 ? 40 * 1024 : 80 * 1024);
+            lds = stripe_reg_lds_bytes(r, e.group);
+        }
+        if (lds > kRegMaxLdsBytes)
+            return kBatchOwnLaunch;
+        blocks = it.stripe_cols;
+        return threads == 256 ? kBatchReg256 : kBatchReg1024;
+    }
+    static hipError_t launch_stripe_register_members(hipStream_t s, LaunchEvents ev, const SEntry* de, const uint32_t* db, uint32_t members,
+                                                     uint32_t blocks, size_t lds, size_t nbits, bool zt, uint32_t threads, bool wide)
+    {
+        return family_batch_reg_stripe(nbits, zt && nbits == 1, s, ev, de, db, members, blocks, lds, threads, wide);
+    }
     // members that look their sums up need 76 registers where the others need 44: a launch without them keeps eight
     // wavefronts per SIMD
-    static bool stripe_entry_wide(const SEntry& e) { return e.kind >= 4; }
+    // (register grids: more than 8 pieces per thread)
+    static bool stripe_entry_wide(const SEntry& e) { return e.kind == 4 || e.kind == 5 || e.kind == 10; }
     // he / hb: the host's copy of the entries and first workgroups that de / db hold on the device
     static hipError_t launch_stripe_members(hipStream_t s, LaunchEvents ev, const SEntry* de, const uint32_t* db, const SEntry* he,
                                             const uint32_t* hb, uint32_t members, uint32_t blocks, size_t lds, size_t nbits, bool zt, bool wide)

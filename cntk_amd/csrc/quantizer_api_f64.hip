@@ -68,6 +68,13 @@ struct BatchAbi<double>
         blocks = (e.t.cols + e.t.cols_per_tile - 1) / e.t.cols_per_tile;
         return true;
     }
+    static int quantize_register_member(const QItem&, size_t, QEntry&, size_t&, uint64_t&, bool) { return kBatchOwnLaunch; }
+    static bool quantize_entry_wide(const QEntry&) { return false; }
+    static hipError_t launch_quantize_register_members(hipStream_t, LaunchEvents, const QEntry*, const uint32_t*, uint32_t, uint32_t, size_t, size_t,
+                                                       bool, uint32_t, bool)
+    {
+        return hipErrorInvalidValue; // no member is of these classes
+    }
     static bool first_in_grid(const QEntry&) { return false; }
     static hipError_t launch_quantize_members(hipStream_t s, LaunchEvents ev, const QEntry* de, const uint32_t* db, uint32_t members,
                                               uint32_t blocks, size_t lds, size_t nbits, bool zt)
@@ -130,6 +137,12 @@ struct BatchAbi<double>
         lds = f64::tile_lds_bytes(e.t, (uint32_t) workers);
         blocks = (e.t.cols + e.t.cols_per_tile - 1) / e.t.cols_per_tile;
         return lds <= f64::kMaxLdsBytes;
+    }
+    static int stripe_register_member(const SItem&, size_t, size_t, SEntry&, size_t&, uint64_t&) { return kBatchOwnLaunch; }
+    static hipError_t launch_stripe_register_members(hipStream_t, LaunchEvents, const SEntry*, const uint32_t*, uint32_t, uint32_t, size_t, size_t,
+                                                     bool, uint32_t, bool)
+    {
+        return hipErrorInvalidValue; // no member is of these classes
     }
     static bool stripe_entry_wide(const SEntry&) { return false; }
     static hipError_t launch_stripe_members(hipStream_t s, LaunchEvents ev, const SEntry* de, const uint32_t* db, const SEntry*, const uint32_t*,

@@ -94,6 +94,18 @@ bool aligned_for(const void* p)
 
 } // namespace cntkq_api
 
+// Members of a gradient-set call that share a grid: workgroups of 256 threads with little / much LDS, and columns in registers
+// on 256 / 1024 threads.
+enum BatchClass : int
+{
+    kBatchSmall = 0,
+    kBatchLarge = 1,
+    kBatchReg256 = 2,
+    kBatchReg1024 = 3,
+    kBatchClasses = 4,
+    kBatchOwnLaunch = kBatchClasses // a launch of its own
+};
+
 struct BatchTable
 {
     std::vector<char> key;   // the item list and parameters the table was built for
@@ -114,13 +126,13 @@ struct BatchTable
     // fresh ones.
     bool captured = false;
     std::vector<std::pair<char*, char*>> retired;
-    // launch parameters of the two LDS classes and the matrices that get a launch of their own
-    size_t members[2] = {0, 0};
-    uint32_t blocks[2] = {0, 0};
-    size_t lds[2] = {0, 0};
-    bool wide[2] = {false, false}; // a member of the class needs the kernel variant compiled for more registers
-    size_t first_entry[2] = {0, 0};
-    size_t first_begin[2] = {0, 0};
+    // launch parameters of the classes of members that share a grid, and the matrices that get a launch of their own
+    size_t members[kBatchClasses] = {};
+    uint32_t blocks[kBatchClasses] = {};
+    size_t lds[kBatchClasses] = {};
+    bool wide[kBatchClasses] = {}; // a member of the class needs the kernel variant compiled for more registers
+    size_t first_entry[kBatchClasses] = {};
+    size_t first_begin[kBatchClasses] = {};
     size_t entries_bytes = 0;
     std::vector<size_t> own;
 };

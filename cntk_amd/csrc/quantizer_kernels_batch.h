@@ -2,6 +2,7 @@
 #pragma once
 
 #include "quantizer_kernels_column.h"
+#include "quantizer_kernels_register.h"
 #include "quantizer_kernels_unquantize.h"
 
 namespace cntkq {
@@ -42,7 +43,8 @@ struct QuantizeBatchEntry
     char* q;
     // 0: tiles (t), 1: columns (c), 2 / 3 / 4: 1-bit columns of 1024 / 2048 / 4096 rows (the unrolled body; c.qcol),
     // 5: columns staged in the residual's memory instead of LDS (c), 6 / 7: columns in registers, up to 3 / 6 pieces per
-    // thread (r; below 32 bits)
+    // thread (r; below 32 bits); 8 / 9 / 10: members of the register grids (quantize_reg_batch_kernel), up to 4 / 8 / 15 pieces
+    // for each of 256 threads, up to 3 / 4 / 6 for each of 1024 (r)
     uint32_t kind;
     uint32_t pad;
     union // the geometry of the entry's kind
@@ -102,6 +104,40 @@ __global__ __launch_bounds__(kTileThreads) void quantize_batch_kernel(const Quan
     }
 }
 
+// The members whose columns the plain call keeps in registers with edge elements or on 1024 threads, and columns of whole
+// pieces too tall for the grid above to hold in 64 registers: one grid for those on T = 256 threads, one for those on 1024.
+// Launched one by one, each such matrix took at least the 4.4 us of a launch, and its last workgroups ran alone on the device:
+// a network of 20 matrices at 2 bits (755 to 14336 rows, 4 workers) spent 16 launches and 240 us on them. The body with
+// edge elements serves whole columns too (it then has none), so the bytes are the plain call's. A column of few pieces per thread does not
+// execute the slots of the taller members: the bodies differ in PER only.
+constexpr int kRegBatchPer256[3] = {4, 8, 15};
+constexpr int kRegBatchPer1024[3] = {3, 4, 6};
+
+// WIDE (T = 256): also members of more than 8 pieces per thread (five wavefronts per SIMD instead of six)
+template <int T, bool WIDE>
+constexpr int reg_batch_waves() // (seven for eight pieces would cost a few spilled registers)
+{
+    return T == 1024 ? 8 : (WIDE ? 5 : 6);
+}
+
+template <int NBITS, bool ZT, int T, bool WIDE>
+__global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(reg_batch_waves<T, WIDE>(), reg_batch_waves<T, WIDE>()))) void
+quantize_reg_batch_kernel(const QuantizeBatchEntry* __restrict__ entries, const uint32_t* __restrict__ begins, uint32_t count)
+{
+    extern __shared__ f32x4 smem_v4[];
+    const uint32_t e = batch_find(begins, count, blockIdx.x);
+    const uint32_t column = blockIdx.x - begins[e];
+    const QuantizeBatchEntry& en = entries[e];
+    const RegGeom c = en.r;
+    constexpr const int(&P)[3] = T == 1024 ? kRegBatchPer1024 : kRegBatchPer256;
+    if (en.kind == 8)
+        quantize_reg_body<NBITS, ZT, T, P[0], true>(en.g, en.r_in, en.r_out, en.q, c, column, smem_v4);
+    else if ((T == 256 && !WIDE) || en.kind == 9)
+        quantize_reg_body<NBITS, ZT, T, P[1], true>(en.g, en.r_in, en.r_out, en.q, c, column, smem_v4);
+    else if constexpr (T == 1024 || WIDE)
+        quantize_reg_body<NBITS, ZT, T, P[2], true>(en.g, en.r_in, en.r_out, en.q, c, column, smem_v4);
+}
+
 // The owner's stripe reductions of a whole gradient set in one launch: same grid construction as quantize_batch_kernel.
 struct StripeBatchEntry
 {
@@ -110,9 +146,10 @@ struct StripeBatchEntry
     char* q_out;
     float* agg_out;
     // 0: tiles (t), 1: columns (c), 2 / 3: 1-bit columns of 1024 / 2048 rows (the unrolled body; c.qcol),
-    // 4 / 5: 1-bit columns of up to eight workers, sums looked up, up to 3 / 6 pieces per thread (r)
+    // 4 / 5: 1-bit columns of up to eight workers, sums looked up, up to 3 / 6 pieces per thread (r);
+    // 8 / 9 / 10: members of the register grids, pieces as QuantizeBatchEntry has them (r, group)
     uint32_t kind;
-    uint32_t pad;
+    uint32_t group; // workers whose packed columns are in LDS together
     TileGeom t;
     ColGeom c;
     RegGeom r;
@@ -179,6 +216,40 @@ __global__ __launch_bounds__(kTileThreads) void stripe_reduce_batch_lookup_kerne
     stripe_reduce_batch_body<1, ZT, true>(entries, begins, count);
 }
 
+// Stripes whose sums the plain call keeps in registers (with edge elements or on 1024 threads), in one grid per workgroup size:
+// see quantize_reg_batch_kernel. 1 bit: up to eight workers, sums looked up; otherwise decoded worker by worker.
+template <int NBITS, bool ZT, int T, int PER>
+__device__ __forceinline__ void stripe_reduce_reg_member(const StripeBatchEntry& en, const RegGeom& c, uint32_t column, f32x4* smem_v4)
+{
+    if constexpr (NBITS == 1)
+        stripe_reduce_lut_body<ZT, PER, T>(en.src, en.stripe_res, en.q_out, en.agg_out, c, column, smem_v4);
+    else
+        stripe_reduce_reg_body<NBITS, ZT, PER, T>(en.src, en.stripe_res, en.q_out, en.agg_out, c, en.group, column, smem_v4);
+}
+
+template <int NBITS, int T, bool WIDE>
+constexpr int stripe_reg_batch_waves()
+{
+    return T == 1024 ? 8 : (WIDE ? (NBITS == 1 ? 5 : 4) : 7);
+}
+
+template <int NBITS, bool ZT, int T, bool WIDE>
+__global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(stripe_reg_batch_waves<NBITS, T, WIDE>(), stripe_reg_batch_waves<NBITS, T, WIDE>()))) void
+stripe_reduce_reg_batch_kernel(const StripeBatchEntry* __restrict__ entries, const uint32_t* __restrict__ begins, uint32_t count)
+{
+    extern __shared__ f32x4 smem_v4[];
+    const uint32_t e = batch_find(begins, count, blockIdx.x);
+    const uint32_t column = blockIdx.x - begins[e];
+    const StripeBatchEntry& en = entries[e];
+    const RegGeom c = en.r;
+    constexpr const int(&P)[3] = T == 1024 ? kRegBatchPer1024 : kRegBatchPer256;
+    if (en.kind == 8)
+        stripe_reduce_reg_member<NBITS, ZT, T, P[0]>(en, c, column, smem_v4);
+    else if ((T == 256 && !WIDE) || en.kind == 9)
+        stripe_reduce_reg_member<NBITS, ZT, T, P[1]>(en, c, column, smem_v4);
+    else if constexpr (T == 1024 || WIDE)
+        stripe_reduce_reg_member<NBITS, ZT, T, P[2]>(en, c, column, smem_v4);
+}
 
 // Many matrices in one launch (see quantize_batch_kernel): the 256-thread blocks of all matrices form one grid.
 enum UnqKind : uint32_t

@@ -319,22 +319,21 @@ __host__ __device__ inline uint32_t stripe_reg_group(const RegGeom& c, uint32_t 
     return (uint32_t) (g < workers ? g : workers);
 }
 
-template <int NBITS, bool ZT, int PER, int TT = 1024>
-__global__ __launch_bounds__(TT) __attribute__((amdgpu_waves_per_eu(reg_waves<TT, PER>(), reg_waves<TT, PER>()))) void stripe_reduce_reg_kernel(
-    StripeSources src, float* stripe_res, char* q_out, float* agg_out, RegGeom c, uint32_t group)
+template <int NBITS, bool ZT, int PER, int TT>
+__device__ __forceinline__ void stripe_reduce_reg_body(const StripeSources& src, float* stripe_res, char* q_out, float* agg_out, const RegGeom& c,
+                                                       uint32_t group, uint32_t column, f32x4* smem_v4)
 {
     using PS = PackShape<NBITS>;
     static_assert(NBITS < 32, "32-bit codes are whole QWords: nothing to assemble");
     constexpr uint32_t T = TT, NW = T / 64;
-    extern __shared__ f32x4 smem_v4[];
     float* red = reinterpret_cast<float*>(smem_v4);
     uint32_t* red_u = reinterpret_cast<uint32_t*>(red + 2 * NW);
     uint32_t* words = reinterpret_cast<uint32_t*>(red + kRegRedSlots);
     float* dec = reinterpret_cast<float*>(words + c.nq); // per worker of the group: 1 bit -> the two levels, else (ufactor, lower)
     uint32_t* pw = words + c.nq + 2 * group;             // the group's packed columns, nq QWords each
     const uint32_t tid = threadIdx.x;
-    const size_t base = (size_t) blockIdx.x * c.rows;
-    const size_t rec = (size_t) blockIdx.x * c.qcol;
+    const size_t base = (size_t) column * c.rows;
+    const size_t rec = (size_t) column * c.qcol;
     for (uint32_t x = tid; x < c.nq; x += T)
         words[x] = 0u;
     // the column as the quantize kernel would see it: head elements, aligned pieces, tail elements
@@ -532,6 +531,21 @@ __global__ __launch_bounds__(TT) __attribute__((amdgpu_waves_per_eu(reg_waves<TT
         }
     }
     reg_stats_pack<NBITS, ZT, T, PER>(a, edge, has_edge, edge_at, head, pieces, shift, c, red, red_u, words, sres, q_out + rec);
+}
+
+// (eight pieces for each of 256 threads: a few registers more than seven wavefronts per SIMD leave)
+template <int T, int PER>
+constexpr int stripe_reg_waves()
+{
+    return T == 256 && PER == 8 ? 6 : reg_waves<T, PER>();
+}
+
+template <int NBITS, bool ZT, int PER, int TT = 1024>
+__global__ __launch_bounds__(TT) __attribute__((amdgpu_waves_per_eu(stripe_reg_waves<TT, PER>(), stripe_reg_waves<TT, PER>()))) void stripe_reduce_reg_kernel(
+    StripeSources src, float* stripe_res, char* q_out, float* agg_out, RegGeom c, uint32_t group)
+{
+    extern __shared__ f32x4 smem_v4[];
+    stripe_reduce_reg_body<NBITS, ZT, PER, TT>(src, stripe_res, q_out, agg_out, c, group, blockIdx.x, smem_v4);
 }
 
 // The 1-bit tall stripe reduction with up to eight workers decoded together from a worker-minor table in LDS. The kernel

@@ -199,6 +199,11 @@ hipError_t family_batch_quantize(size_t nbits, bool zt, hipStream_t s, LaunchEve
                                  uint32_t count, uint32_t total_blocks, size_t lds);
 hipError_t family_batch_stripe(size_t nbits, bool zt, hipStream_t s, LaunchEvents ev, const StripeBatchEntry* entries, const uint32_t* begins,
                                uint32_t count, uint32_t total_blocks, size_t lds, bool wide);
+// members of the register grids: threads 256 or 1024; wide: some of more than 8 pieces per thread
+hipError_t family_batch_reg_quantize(size_t nbits, bool zt, hipStream_t s, LaunchEvents ev, const QuantizeBatchEntry* entries, const uint32_t* begins,
+                                     uint32_t count, uint32_t total_blocks, size_t lds, uint32_t threads, bool wide);
+hipError_t family_batch_reg_stripe(size_t nbits, bool zt, hipStream_t s, LaunchEvents ev, const StripeBatchEntry* entries, const uint32_t* begins,
+                                   uint32_t count, uint32_t total_blocks, size_t lds, uint32_t threads, bool wide);
 hipError_t launch_unquantize_batch(hipStream_t s, LaunchEvents ev, const UnquantizeBatchEntry* entries, const uint32_t* begins, uint32_t count,
                                    uint32_t total_blocks, size_t nbits, bool add, size_t lds);
 

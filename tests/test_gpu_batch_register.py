@@ -1,0 +1,97 @@
+"""The register grids of the gradient-set calls (columns kept in registers on 256 or 1024 threads, many matrices per launch):
+the bytes are those of one call per matrix, whose parity with the oracle the other tests hold. Needs an MI355X."""
+import numpy as np
+import pytest
+import torch
+
+import datagen
+import parity
+from cntk_amd import Matrix, MatrixQuantizerImpl, QuantizedMatrix
+
+pytestmark = pytest.mark.gpu
+
+# heights on both sides of every line between the kernels: edge elements on 256 threads (2049 .. 7168 rows not a multiple of 4) and
+# on 1024 (up to 24576 rows by pieces per thread, 102368 in launches of their own), whole pieces on 256 threads with more
+# than six pieces each (6148 .. 14336 rows) and on 1024
+EDGE = [(2049, 40), (4071, 5), (4099, 3), (7166, 9), (7169, 3), (9305, 7), (12258, 2), (16359, 2), (16361, 3), (24547, 2), (24555, 1)]
+WHOLE = [(6148, 70), (8192, 40), (9304, 33), (14308, 36), (14336, 34), (14340, 3), (16384, 2), (24576, 2), (24580, 1)]
+SMALL = [(64, 64), (429, 37), (21, 960), (2048, 1), (9280, 1), (13000, 2)]
+
+
+def _matrices(shapes, nbits, seed):
+    # slices of one allocation at odd offsets: the columns of a matrix start anywhere within 16 bytes, the same in both runs
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(datagen.case_seed(seed))
+    out = []
+    for i, (r, c) in enumerate(shapes):
+        off = 0 if r % 4 == 0 else i % 4
+        g, res = [(torch.randn(r * c + 4, generator=gen, device="cuda:0") * s)[off:off + r * c] for s in (0.01, 0.002)]
+        out.append((Matrix(r, c, 0, g), Matrix(r, c, 0, res), QuantizedMatrix(r, c, nbits, 0)))
+    return out
+
+
+@pytest.mark.parametrize("nbits,zt", [(1, False), (1, True), (2, False), (8, False), (16, False)])
+@pytest.mark.parametrize("shapes", [EDGE, WHOLE, EDGE[:2] + SMALL, EDGE + WHOLE + SMALL], ids=["edge", "whole", "few", "all"])
+def test_quantize(shapes, nbits, zt):
+    qz = MatrixQuantizerImpl.Create(0, False)
+    one, many = _matrices(shapes, nbits, nbits), _matrices(shapes, nbits, nbits)
+    for _ in range(2):
+        for g, r, q in one:
+            qz.QuantizeAsync(g, r, q, r, zt)
+        qz.QuantizeBatchAsync([(g, r, q, r) for g, r, q in many], zt)
+        qz.WaitQuantizeAsyncDone()
+        torch.cuda.synchronize()
+        for (_, r1, q1), (_, r2, q2), shape in zip(one, many, shapes):
+            assert np.array_equal(q1.to_numpy(), q2.to_numpy()), ("packed", shape)
+            assert parity.bits_equal(r1.to_numpy(), r2.to_numpy()), ("residual", shape)
+
+
+def _stripes(qz, shapes, nbits, zt, k):
+    workers = [_matrices(shapes, nbits, 20 * w + nbits) for w in range(k)]
+    for ms in workers:
+        for g, r, q in ms:
+            qz.QuantizeAsync(g, r, q, r, zt)
+    sres = [r for _, r, _ in _matrices(shapes, nbits, 999)]
+    agg = [Matrix(r, c) for r, c in shapes]
+    return [[ms[i][2] for ms in workers] for i in range(len(shapes))], sres, agg
+
+
+@pytest.mark.parametrize("nbits,zt,k", [(1, False, 1), (1, True, 8), (1, False, 9), (2, False, 3), (8, False, 1), (8, False, 8), (16, False, 2)])
+@pytest.mark.parametrize("shapes", [EDGE, WHOLE, EDGE[:2] + SMALL, EDGE + WHOLE + SMALL], ids=["edge", "whole", "few", "all"])
+def test_stripe_reduction(shapes, nbits, zt, k):
+    qz = MatrixQuantizerImpl.Create(0, False)
+    owner = k // 2
+    q1, s1, a1 = _stripes(qz, shapes, nbits, zt, k)
+    q2, s2, a2 = _stripes(qz, shapes, nbits, zt, k)
+    for q, s, a in zip(q1, s1, a1):
+        qz.StripeReduceAsync(q, owner, s, q[owner], zt, agg_out=a)
+    qz.StripeReduceBatchAsync([(q, s, q[owner], a) for q, s, a in zip(q2, s2, a2)], owner, zt)
+    qz.WaitStripeReduceDone()
+    torch.cuda.synchronize()
+    for i, shape in enumerate(shapes):
+        assert np.array_equal(q1[i][owner].to_numpy(), q2[i][owner].to_numpy()), ("packed", shape)
+        assert parity.bits_equal(s1[i].to_numpy(), s2[i].to_numpy()), ("stripe residual", shape)
+        assert parity.bits_equal(a1[i].to_numpy(), a2[i].to_numpy()), ("aggregate", shape)
+
+
+def test_recorded_stripes_without_a_table():
+    """Stripes that each had a launch of their own could always be recorded without an eager call before; they still can."""
+    qz = MatrixQuantizerImpl.Create(0, False)
+    shapes = [(9305, 3), (7169, 2), (4099, 2)]
+    q1, s1, a1 = _stripes(qz, shapes, 2, False, 2)
+    q2, s2, a2 = _stripes(qz, shapes, 2, False, 2)
+    torch.cuda.synchronize()
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    qz.SetMainStream(side.cuda_stream)
+    with torch.cuda.graph(graph, stream=side):
+        qz.StripeReduceBatchAsync([(q, s, q[0], a) for q, s, a in zip(q2, s2, a2)], 0, False)
+    qz.SetMainStream(torch.cuda.current_stream().cuda_stream)
+    for _ in range(3):
+        for q, s, a in zip(q1, s1, a1):
+            qz.StripeReduceAsync(q, 0, s, q[0], False, agg_out=a)
+        qz.WaitStripeReduceDone()
+        graph.replay()
+        torch.cuda.synchronize()
+        for i, shape in enumerate(shapes):
+            assert np.array_equal(q1[i][0].to_numpy(), q2[i][0].to_numpy()), ("packed", shape)
+            assert parity.bits_equal(s1[i].to_numpy(), s2[i].to_numpy()), ("stripe residual", shape)
