@@ -101,6 +101,14 @@ struct BatchAbi<float>
     static bool quantize_member(const QItem& it, size_t nbits, QEntry& e, size_t& lds, uint64_t& blocks)
     {
         const int path = quantize_auto_path(it.in, it.res_in, it.res_out, it.qbuf, it.rows, nbits);
+        if (path == kPathTile && short_applicable(it.rows))
+        {
+            e.kind = 11;
+            e.s = make_short_geom(it.rows, it.cols, qwords_per_col(it.rows, nbits), qcol_bytes(nbits, it.rows), sizeof(float));
+            lds = short_lds_bytes(e.s, sizeof(float));
+            blocks = short_blocks(e.s);
+            return true;
+        }
         if (path == kPathTile)
         {
             e.kind = 0;
@@ -148,7 +156,7 @@ struct BatchAbi<float>
         }
         return false;
     }
-    static bool first_in_grid(const QEntry& e) { return e.kind == 5 || e.kind >= 9; }
+    static bool first_in_grid(const QEntry& e) { return e.kind == 5 || e.kind == 9 || e.kind == 10; }
     static hipError_t launch_quantize_members(hipStream_t s, LaunchEvents ev, const QEntry* de, const uint32_t* db, uint32_t members,
                                               uint32_t blocks, size_t lds, size_t nbits, bool zt)
     {
@@ -236,6 +244,13 @@ struct BatchAbi<float>
                 e.kind = stripe_lookup_per(it.rows, line_shift) <= 3 ? 4 : 5;
                 lds = stripe_lut_lds_bytes(e.r);
             }
+        }
+        else if (short_applicable(it.rows))
+        {
+            e.kind = 11;
+            e.s = make_short_geom(it.rows, it.stripe_cols, qwords_per_col(it.rows, nbits), qcol_bytes(nbits, it.rows), sizeof(float));
+            lds = short_lds_bytes(e.s, sizeof(float));
+            blocks = short_blocks(e.s);
         }
         else
         {

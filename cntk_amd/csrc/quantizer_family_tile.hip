@@ -54,6 +54,40 @@ hipError_t family_tile_stripe(size_t nbits, bool zt, hipStream_t s, LaunchEvents
     return dispatch_nbits<StripeLauncher>(nbits, zt, s, ev, src, stripe_res, q_out, agg_out, t);
 }
 
+template <int NBITS, bool ZT>
+struct ShortLauncher
+{
+    static hipError_t run(hipStream_t s, LaunchEvents ev, const float* g, const float* r_in, float* r_out, char* q, ShortGeom t)
+    {
+        hipExtLaunchKernelGGL((quantize_short_kernel<NBITS, ZT, float>), dim3(short_blocks(t)), dim3(kShortThreads), short_lds_bytes(t, sizeof(float)), s,
+                              ev.start, ev.stop, 0, g, r_in, r_out, q, t);
+        return hipGetLastError();
+    }
+};
+
+template <int NBITS, bool ZT>
+struct StripeShortLauncher
+{
+    static hipError_t run(hipStream_t s, LaunchEvents ev, const StripeSources& src, float* stripe_res, char* q_out, float* agg_out,
+                          ShortGeom t)
+    {
+        hipExtLaunchKernelGGL((stripe_reduce_short_kernel<NBITS, ZT>), dim3(short_blocks(t)), dim3(kShortThreads), short_lds_bytes(t, sizeof(float)), s,
+                              ev.start, ev.stop, 0, src, stripe_res, q_out, agg_out, t);
+        return hipGetLastError();
+    }
+};
+
+hipError_t family_short_quantize(size_t nbits, bool zt, hipStream_t s, LaunchEvents ev, const float* g, const float* r_in, float* r_out, char* q, ShortGeom t)
+{
+    return dispatch_nbits<ShortLauncher>(nbits, zt, s, ev, g, r_in, r_out, q, t);
+}
+
+hipError_t family_short_stripe(size_t nbits, bool zt, hipStream_t s, LaunchEvents ev, const StripeSources& src, float* stripe_res, char* q_out,
+                               float* agg_out, ShortGeom t)
+{
+    return dispatch_nbits<StripeShortLauncher>(nbits, zt, s, ev, src, stripe_res, q_out, agg_out, t);
+}
+
 hipError_t family_tall_quantize(size_t nbits, bool zt, hipStream_t s, LaunchEvents ev, const float* g, const float* r_in, float* r_out, char* q, uint32_t rows, uint32_t cols, uint32_t nq, uint64_t qcol)
 {
     return dispatch_nbits<TallLauncher>(nbits, zt, s, ev, g, r_in, r_out, q, rows, cols, nq, qcol);

@@ -4,6 +4,7 @@
 
 #include "quantizer_kernels_common.h"
 #include "quantizer_kernels_tile.h"
+#include "quantizer_kernels_short.h"
 #include "quantizer_kernels_column.h"
 #include "quantizer_kernels_register.h"
 #include "quantizer_kernels_tall.h"

@@ -2,6 +2,7 @@
 #pragma once
 
 #include "quantizer_kernels_column.h"
+#include "quantizer_kernels_short.h"
 #include "quantizer_kernels_register.h"
 #include "quantizer_kernels_unquantize.h"
 
@@ -44,7 +45,8 @@ struct QuantizeBatchEntry
     // 0: tiles (t), 1: columns (c), 2 / 3 / 4: 1-bit columns of 1024 / 2048 / 4096 rows (the unrolled body; c.qcol),
     // 5: columns staged in the residual's memory instead of LDS (c), 6 / 7: columns in registers, up to 3 / 6 pieces per
     // thread (r; below 32 bits); 8 / 9 / 10: members of the register grids (quantize_reg_batch_kernel), up to 4 / 8 / 15 pieces
-    // for each of 256 threads, up to 3 / 4 / 6 for each of 1024 (r)
+    // for each of 256 threads, up to 3 / 4 / 6 for each of 1024 (r);
+    // 11: columns of at most 16 rows, one thread each (s)
     uint32_t kind;
     uint32_t pad;
     union // the geometry of the entry's kind
@@ -52,12 +54,13 @@ struct QuantizeBatchEntry
         TileGeom t;
         ColGeom c;
         RegGeom r;
+        ShortGeom s;
     };
     uint32_t reserved[6]; // (keeps the entry at the size the no-allocation call's fixed array is laid out for)
 };
 
 template <int NBITS, bool ZT>
-__global__ __launch_bounds__(kTileThreads) void quantize_batch_kernel(const QuantizeBatchEntry* __restrict__ entries,
+__global__ __launch_bounds__(kTileThreads) CNTKQ_SGPRS_FOR_8_WAVES void quantize_batch_kernel(const QuantizeBatchEntry* __restrict__ entries,
                                                                       const uint32_t* __restrict__ begins, uint32_t count)
 {
     extern __shared__ f32x4 smem_v4[];
@@ -69,12 +72,17 @@ __global__ __launch_bounds__(kTileThreads) void quantize_batch_kernel(const Quan
         const TileGeom t = entries[e].t;
         quantize_tile_body<NBITS, ZT>(entries[e].g, entries[e].r_in, entries[e].r_out, entries[e].q, t, index);
     }
+    else if (entries[e].kind == 11)
+    {
+        const ShortGeom t = entries[e].s;
+        quantize_short_body<NBITS, ZT>(entries[e].g, entries[e].r_in, entries[e].r_out, entries[e].q, t, index, reinterpret_cast<float*>(smem_v4));
+    }
     else if (entries[e].kind == 5)
     {
         const ColGeom c = entries[e].c;
         quantize_colg_body<NBITS, ZT, true>(entries[e].g, entries[e].r_in, entries[e].r_out, entries[e].q, c, index, smem_v4);
     }
-    else if (NBITS < 32 && entries[e].kind >= 6)
+    else if (NBITS < 32 && entries[e].kind >= 6) // (6 or 7)
     {
         // the column in registers: the bytes of the LDS column body, a fifth faster from 2304 rows up
         if constexpr (NBITS < 32)
@@ -147,12 +155,14 @@ struct StripeBatchEntry
     float* agg_out;
     // 0: tiles (t), 1: columns (c), 2 / 3: 1-bit columns of 1024 / 2048 rows (the unrolled body; c.qcol),
     // 4 / 5: 1-bit columns of up to eight workers, sums looked up, up to 3 / 6 pieces per thread (r);
-    // 8 / 9 / 10: members of the register grids, pieces as QuantizeBatchEntry has them (r, group)
+    // 8 / 9 / 10: members of the register grids, pieces as QuantizeBatchEntry has them (r, group);
+    // 11: columns of at most 16 rows (s)
     uint32_t kind;
     uint32_t group; // workers whose packed columns are in LDS together
     TileGeom t;
     ColGeom c;
     RegGeom r;
+    ShortGeom s;
 };
 
 // LOOKUP: the variant that also runs members of kinds 4 and 5 (76 registers instead of 44: a launch without such members
@@ -169,6 +179,11 @@ __device__ __forceinline__ void stripe_reduce_batch_body(const StripeBatchEntry*
     {
         const TileGeom t = en.t;
         stripe_reduce_tile_body<NBITS, ZT>(en.src, en.stripe_res, en.q_out, en.agg_out, t, index);
+    }
+    else if (en.kind == 11)
+    {
+        const ShortGeom t = en.s;
+        stripe_reduce_short_body<NBITS, ZT>(en.src, en.stripe_res, en.q_out, en.agg_out, t, index, reinterpret_cast<float*>(smem_v4));
     }
     else if (NBITS != 1 || en.kind == 1)
     {

@@ -132,6 +132,33 @@ inline TileGeom make_tile_geom(size_t rows, size_t cols, size_t nbits, uint32_t 
     return t;
 }
 
+// Columns of at most kShortMaxRows rows: one thread per column, with the tile kernels' sums (same bytes). A thread holds the column
+// in registers; the tile kernel's share of a column grows with the height meanwhile (12 x 1.37 M: 34 us against the tile kernel's
+// 80, 15 x 836000 26 against 50, 28 x 939000 62 with the tile kernel, whose bytes take 53).
+inline bool short_applicable(size_t rows)
+{
+    return rows <= kShortMaxRows;
+}
+
+// A workgroup takes kShortTileBytes of values, or 256 columns where those are more, or fewer columns where the device would
+// otherwise have less than two workgroups per compute unit.
+inline ShortGeom make_short_geom(size_t rows, size_t cols, size_t nq, size_t qcol, size_t element)
+{
+    ShortGeom t;
+    t.rows = (uint32_t) rows;
+    t.cols = (uint32_t) cols;
+    t.nq = (uint32_t) nq;
+    const size_t most = kShortTileBytes / element / rows / kShortThreads, wanted = cols / (512 * kShortThreads);
+    t.cpt = kShortThreads * (uint32_t) std::max<size_t>(1, std::min(most, wanted));
+    t.qcol = qcol;
+    return t;
+}
+
+inline uint32_t short_blocks(const ShortGeom& t)
+{
+    return (t.cols - 1) / t.cpt + 1;
+}
+
 template <template <int, bool> class Launcher, typename... Args>
 inline hipError_t dispatch_nbits(size_t nbits, bool zt, Args... args)
 {
@@ -156,6 +183,10 @@ struct UnquantizePlan;
 hipError_t family_tile_quantize(size_t nbits, bool zt, hipStream_t s, LaunchEvents ev, const float* g, const float* r_in, float* r_out, char* q, TileGeom t);
 hipError_t family_tile_stripe(size_t nbits, bool zt, hipStream_t s, LaunchEvents ev, const StripeSources& src, float* stripe_res, char* q_out,
                               float* agg_out, TileGeom t);
+hipError_t family_short_quantize(size_t nbits, bool zt, hipStream_t s, LaunchEvents ev, const float* g, const float* r_in, float* r_out, char* q,
+                                 ShortGeom t);
+hipError_t family_short_stripe(size_t nbits, bool zt, hipStream_t s, LaunchEvents ev, const StripeSources& src, float* stripe_res, char* q_out,
+                               float* agg_out, ShortGeom t);
 hipError_t family_tall_quantize(size_t nbits, bool zt, hipStream_t s, LaunchEvents ev, const float* g, const float* r_in, float* r_out, char* q,
                                 uint32_t rows, uint32_t cols, uint32_t nq, uint64_t qcol);
 hipError_t family_col_quantize(size_t nbits, bool zt, hipStream_t s, LaunchEvents ev, const float* g, const float* r_in, float* r_out, char* q,
@@ -709,6 +740,8 @@ inline hipError_t launch_quantize(hipStream_t s, LaunchEvents ev, const float* g
     {
         if (rows > kTileMaxRows)
             return hipErrorInvalidValue;
+        if (tune.quantize_path == kPathAuto && short_applicable(rows))
+            return family_short_quantize(nbits, zt, s, ev, g, r_in, r_out, qc, make_short_geom(rows, cols, qwords_per_col(rows, nbits), qcol_bytes(nbits, rows), sizeof(float)));
         const TileGeom t = make_tile_geom(rows, cols, nbits, tune.tile_gs, tune.tile_stage, tune.tile_threads);
         return family_tile_quantize(nbits, zt, s, ev, g, r_in, r_out, qc, t);
     }
@@ -826,6 +859,9 @@ inline hipError_t launch_stripe_reduce(hipStream_t s, LaunchEvents ev, const Str
         char* qo = static_cast<char*>(q_out);
         return family_col_stripe_unrolled(zt, rows == 1024 ? 1 : (rows == 2048 ? 2 : 4), s, ev, src, stripe_res, qo, agg_out, c, qcol);
     }
+    if (tune.quantize_path == kPathAuto && short_applicable(rows))
+        return family_short_stripe(nbits, zt, s, ev, src, stripe_res, static_cast<char*>(q_out), agg_out,
+                                   make_short_geom(rows, cols, qwords_per_col(rows, nbits), qcol_bytes(nbits, rows), sizeof(float)));
     // Same tile geometry as launch_quantize would use for a matrix of this height, so that the statistics are summed in
     // the same order and the fused call gives the bytes of the reference's unquantize ... quantize call sequence.
     const TileGeom t = make_tile_geom(rows, cols, nbits, tune.tile_gs, tune.tile_stage, tune.tile_threads);
@@ -982,7 +1018,9 @@ inline UnquantizePlan plan_unquantize(const void* q, const float* out, size_t ro
         t.rows = (uint32_t) rows;
         t.cols = (uint32_t) cols;
         t.nq = (uint32_t) nq;
-        size_t cpt = (kUnqTileElems / rows) & ~(size_t) 3;
+        // (short columns, whose records are longer than their values: no more than leaves room for eight workgroups in a compute
+        // unit's LDS; 1 x 38 M at 4 bits, which without the limit exceeded 64 KB and went to the QWord-major decoder: 377 -> 155 us; 3 x 4.65 M at 1 bit 32 -> 22 us)
+        size_t cpt = std::min(kUnqTileElems / rows, (size_t) (20 * 1024) / ((nq + 4) * 4)) & ~(size_t) 3;
         if (cpt < 4)
             cpt = 4;
         t.cpt = (uint32_t) cpt;

@@ -76,6 +76,17 @@ inline hipError_t dispatch_nbits64(size_t nbits, bool zt, Args... args)
 }
 
 template <int NBITS, bool ZT>
+struct ShortLauncher
+{
+    static hipError_t run(hipStream_t s, LaunchEvents ev, const double* g, const double* r_in, double* r_out, char* q, ShortGeom t)
+    {
+        hipExtLaunchKernelGGL((quantize_short_kernel<NBITS, ZT, double>), dim3(short_blocks(t)), dim3(kShortThreads), short_lds_bytes(t, sizeof(double)), s,
+                              ev.start, ev.stop, 0, g, r_in, r_out, q, t);
+        return hipGetLastError();
+    }
+};
+
+template <int NBITS, bool ZT>
 struct TileLauncher
 {
     static hipError_t run(hipStream_t s, LaunchEvents ev, const double* g, const double* r_in, double* r_out, char* q, TileGeom t)
@@ -278,6 +289,9 @@ inline hipError_t launch_quantize(hipStream_t s, LaunchEvents ev, const double* 
     {
         if (rows > kTileMaxRows)
             return hipErrorInvalidValue;
+        if (tune.quantize_path == kPathAuto && short_applicable(rows))
+            return dispatch_nbits64<ShortLauncher>(nbits, zt, s, ev, g, r_in, r_out, qc,
+                                                   make_short_geom(rows, cols, qwords_per_col(rows, nbits), qcol_bytes(nbits, rows), sizeof(double)));
         const TileGeom t = make_tile_geom(rows, cols, nbits, tune.tile_gs);
         if (tile_lds_bytes(t, 0) > kMaxLdsBytes)
             return hipErrorInvalidValue;
@@ -537,7 +551,7 @@ inline UnquantizePlan64 plan_unquantize(const double* out, size_t rows, size_t c
         t.rows = (uint32_t) rows;
         t.cols = (uint32_t) cols;
         t.nq = (uint32_t) nq;
-        size_t cpt = (kUnqTileElems64 / rows) & ~(size_t) 1;
+        size_t cpt = std::min<size_t>(kUnqTileElems64 / rows, (size_t) (20 * 1024) / ((nq + 4) * 8)) & ~(size_t) 1; // (the limit: as on the float side)
         if (cpt < 2)
             cpt = 2;
         t.cpt = (uint32_t) cpt;
