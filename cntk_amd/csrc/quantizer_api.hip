@@ -228,6 +228,15 @@ struct BatchAbi<float>
             e.c = make_col_geom(it.rows, nbits, line_shift);
             lds = colg_lds_bytes_rt(e.c, nbits) + stripe_dec_bytes(nbits, workers);
             blocks = it.stripe_cols;
+            if (workers == 1 && nbits < 32)
+            {
+                // a single worker's columns: quantized again as quantize_reg_body would (the bytes of all column kernels);
+                // more than six pieces per thread are members of the register grids
+                e.r = make_reg_geom(it.rows, nbits, 256, line_shift);
+                e.kind = stripe_lookup_per(it.rows, line_shift) <= 3 ? 12 : 13;
+                lds = reg_lds_bytes(e.r);
+                return stripe_lookup_per(it.rows, line_shift) <= 6;
+            }
             // as launch_stripe_reduce chooses: the unrolled body where every packed stripe is 8-byte aligned
             bool aligned = (reinterpret_cast<uintptr_t>(it.q_out) & 7u) == 0;
             for (size_t w = 0; w < workers; ++w)
@@ -284,7 +293,9 @@ struct BatchAbi<float>
         if (e.kind == 0)
             return kBatchOwnLaunch;
         e.r = r;
-        if (nbits == 1)
+        if (workers == 1)
+            lds = reg_lds_bytes(r);
+        else if (nbits == 1)
             lds = stripe_lut_lds_bytes(r);
         else
         {
@@ -299,9 +310,9 @@ struct BatchAbi<float>
         return threads == 256 ? kBatchReg256 : kBatchReg1024;
     }
     static hipError_t launch_stripe_register_members(hipStream_t s, LaunchEvents ev, const SEntry* de, const uint32_t* db, uint32_t members,
-                                                     uint32_t blocks, size_t lds, size_t nbits, bool zt, uint32_t threads, bool wide)
+                                                     uint32_t blocks, size_t lds, size_t nbits, bool zt, uint32_t threads, bool wide, bool one)
     {
-        return family_batch_reg_stripe(nbits, zt && nbits == 1, s, ev, de, db, members, blocks, lds, threads, wide);
+        return family_batch_reg_stripe(nbits, zt && nbits == 1, s, ev, de, db, members, blocks, lds, threads, wide, one);
     }
     // members that look their sums up need 76 registers where the others need 44: a launch without them keeps eight
     // wavefronts per SIMD
@@ -313,7 +324,7 @@ struct BatchAbi<float>
     {
         // a few stripes of one shape that all run the unrolled 1-bit column body with up to eight workers (the ranks of a
         // small cluster simulated on one GPU): described in the kernel's arguments instead of the table in device memory
-        bool as_set = members <= kStripeSetMax && nbits == 1 && (he[0].kind == 2 || he[0].kind == 3) && he[0].src.workers <= kStripeSetMax;
+        bool as_set = members <= kStripeSetMax && nbits == 1 && he[0].src.workers > 1 && (he[0].kind == 2 || he[0].kind == 3) && he[0].src.workers <= kStripeSetMax;
         for (uint32_t i = 1; i < members && as_set; ++i)
             as_set = he[i].kind == he[0].kind && he[i].src.workers == he[0].src.workers;
         if (as_set)
@@ -336,7 +347,7 @@ struct BatchAbi<float>
             set.qcol = he[0].c.qcol;
             return family_col_stripe_set(zt && nbits == 1, he[0].kind == 2 ? 1 : 2, s, ev, set);
         }
-        return launch_stripe_reduce_batch(s, ev, de, db, members, blocks, lds, nbits, zt, wide);
+        return launch_stripe_reduce_batch(s, ev, de, db, members, blocks, lds, nbits, zt, wide, he[0].src.workers == 1);
     }
 };
 

@@ -140,7 +140,7 @@ struct BatchAbi<double>
     }
     static int stripe_register_member(const SItem&, size_t, size_t, SEntry&, size_t&, uint64_t&) { return kBatchOwnLaunch; }
     static hipError_t launch_stripe_register_members(hipStream_t, LaunchEvents, const SEntry*, const uint32_t*, uint32_t, uint32_t, size_t, size_t,
-                                                     bool, uint32_t, bool)
+                                                     bool, uint32_t, bool, bool)
     {
         return hipErrorInvalidValue; // no member is of these classes
     }

@@ -9,8 +9,14 @@ template <int NBITS, bool ZT>
 struct StripeBatchLauncher
 {
     static hipError_t run(hipStream_t s, LaunchEvents ev, const StripeBatchEntry* entries, const uint32_t* begins, uint32_t count,
-                          uint32_t total_blocks, size_t lds, bool wide)
+                          uint32_t total_blocks, size_t lds, bool wide, bool one)
     {
+        if (one)
+        {
+            hipExtLaunchKernelGGL((stripe_one_batch_kernel<NBITS, ZT>), dim3(total_blocks), dim3(kTileThreads), lds, s, ev.start, ev.stop, 0,
+                                  entries, begins, count);
+            return hipGetLastError();
+        }
         if constexpr (NBITS == 1)
         {
             if (wide)
@@ -26,9 +32,9 @@ struct StripeBatchLauncher
     }
 };
 
-hipError_t family_batch_stripe(size_t nbits, bool zt, hipStream_t s, LaunchEvents ev, const StripeBatchEntry* entries, const uint32_t* begins, uint32_t count, uint32_t total_blocks, size_t lds, bool wide)
+hipError_t family_batch_stripe(size_t nbits, bool zt, hipStream_t s, LaunchEvents ev, const StripeBatchEntry* entries, const uint32_t* begins, uint32_t count, uint32_t total_blocks, size_t lds, bool wide, bool one)
 {
-    return dispatch_nbits<StripeBatchLauncher>(nbits, zt, s, ev, entries, begins, count, total_blocks, lds, wide);
+    return dispatch_nbits<StripeBatchLauncher>(nbits, zt, s, ev, entries, begins, count, total_blocks, lds, wide, one);
 }
 
 } // namespace cntkq

@@ -156,7 +156,7 @@ struct StripeBatchEntry
     // 0: tiles (t), 1: columns (c), 2 / 3: 1-bit columns of 1024 / 2048 rows (the unrolled body; c.qcol),
     // 4 / 5: 1-bit columns of up to eight workers, sums looked up, up to 3 / 6 pieces per thread (r);
     // 8 / 9 / 10: members of the register grids, pieces as QuantizeBatchEntry has them (r, group);
-    // 11: columns of at most 16 rows (s)
+    // 11: columns of at most 16 rows (s); 12 / 13: columns of a single worker, up to 3 / 6 pieces per thread (r)
     uint32_t kind;
     uint32_t group; // workers whose packed columns are in LDS together
     TileGeom t;
@@ -216,6 +216,41 @@ __device__ __forceinline__ void stripe_reduce_batch_body(const StripeBatchEntry*
     }
 }
 
+// The stripes of a single worker: columns of up to six pieces per thread as quantize_reg_body has them (kinds 12 / 13: up to 3 / 6
+// pieces; r), the rest as above.
+template <int NBITS, bool ZT>
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8, 8))) CNTKQ_SGPRS_FOR_8_WAVES void stripe_one_batch_kernel(const StripeBatchEntry* __restrict__ entries,
+                                                                                                const uint32_t* __restrict__ begins, uint32_t count)
+{
+    extern __shared__ f32x4 smem_v4[];
+    const uint32_t e = batch_find(begins, count, blockIdx.x);
+    const uint32_t index = blockIdx.x - begins[e];
+    const StripeBatchEntry& en = entries[e];
+    if (en.kind == 0)
+    {
+        const TileGeom t = en.t;
+        stripe_reduce_tile_body<NBITS, ZT>(en.src, en.stripe_res, en.q_out, en.agg_out, t, index);
+    }
+    else if (en.kind == 11)
+    {
+        const ShortGeom t = en.s;
+        stripe_reduce_short_body<NBITS, ZT>(en.src, en.stripe_res, en.q_out, en.agg_out, t, index, reinterpret_cast<float*>(smem_v4));
+    }
+    else if constexpr (NBITS == 32)
+    {
+        const ColGeom c = en.c;
+        stripe_reduce_colg_body<NBITS, ZT>(en.src, en.stripe_res, en.q_out, en.agg_out, c, index, smem_v4);
+    }
+    else
+    {
+        const RegGeom c = en.r;
+        if (en.kind == 12)
+            stripe_one_reg_body<NBITS, ZT, kTileThreads, 3>(en.src.q[0], en.stripe_res, en.q_out, en.agg_out, c, index, smem_v4);
+        else
+            stripe_one_reg_body<NBITS, ZT, kTileThreads, 6>(en.src.q[0], en.stripe_res, en.q_out, en.agg_out, c, index, smem_v4);
+    }
+}
+
 template <int NBITS, bool ZT>
 __global__ __launch_bounds__(kTileThreads) CNTKQ_SGPRS_FOR_8_WAVES void stripe_reduce_batch_kernel(const StripeBatchEntry* __restrict__ entries,
                                                                                                    const uint32_t* __restrict__ begins, uint32_t count)
@@ -264,6 +299,31 @@ stripe_reduce_reg_batch_kernel(const StripeBatchEntry* __restrict__ entries, con
         stripe_reduce_reg_member<NBITS, ZT, T, P[1]>(en, c, column, smem_v4);
     else if constexpr (T == 1024 || WIDE)
         stripe_reduce_reg_member<NBITS, ZT, T, P[2]>(en, c, column, smem_v4);
+}
+
+// ... of a single worker
+template <int T, bool WIDE>
+constexpr int stripe_one_reg_batch_waves()
+{
+    return T == 1024 ? 8 : (WIDE ? 4 : 6);
+}
+
+template <int NBITS, bool ZT, int T, bool WIDE>
+__global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(stripe_one_reg_batch_waves<T, WIDE>(), stripe_one_reg_batch_waves<T, WIDE>()))) void
+stripe_one_reg_batch_kernel(const StripeBatchEntry* __restrict__ entries, const uint32_t* __restrict__ begins, uint32_t count)
+{
+    extern __shared__ f32x4 smem_v4[];
+    const uint32_t e = batch_find(begins, count, blockIdx.x);
+    const uint32_t column = blockIdx.x - begins[e];
+    const StripeBatchEntry& en = entries[e];
+    const RegGeom c = en.r;
+    constexpr const int(&P)[3] = T == 1024 ? kRegBatchPer1024 : kRegBatchPer256;
+    if (en.kind == 8)
+        stripe_one_reg_body<NBITS, ZT, T, P[0]>(en.src.q[0], en.stripe_res, en.q_out, en.agg_out, c, column, smem_v4);
+    else if ((T == 256 && !WIDE) || en.kind == 9)
+        stripe_one_reg_body<NBITS, ZT, T, P[1]>(en.src.q[0], en.stripe_res, en.q_out, en.agg_out, c, column, smem_v4);
+    else if constexpr (T == 1024 || WIDE)
+        stripe_one_reg_body<NBITS, ZT, T, P[2]>(en.src.q[0], en.stripe_res, en.q_out, en.agg_out, c, column, smem_v4);
 }
 
 // Many matrices in one launch (see quantize_batch_kernel): the 256-thread blocks of all matrices form one grid.

@@ -548,6 +548,116 @@ __global__ __launch_bounds__(TT) __attribute__((amdgpu_waves_per_eu(stripe_reg_w
     stripe_reduce_reg_body<NBITS, ZT, PER, TT>(src, stripe_res, q_out, agg_out, c, group, blockIdx.x, smem_v4);
 }
 
+// ---- one worker: its stripe quantized again --------------------------------------------------------------------------
+//
+// With a single worker (a training process on its own, or the one owner of a stripe) the sum is that worker's values, and the
+// reduction is the quantize kernel with a decoded gradient. The kernels above take the packed columns through LDS, or make a table of
+// sums, before the first value is known; here a thread that would load 16 bytes of gradient loads the four QWords that hold
+// those elements -- a column's QWords stay in the compute unit's cache -- while the residual is on its way. Statistics, codes and
+// bytes are those of the other kernels. ResNet-50's 161 stripes at 1 bit: 62.8 us with the table of sums, 57 us with the general
+// column kernel, 50.9 us so (8 bytes of residual per element: 34 us at 6 TB/s; below 1024 rows the tile kernel still goes through
+// LDS, and the coding is bound by instruction issue as much as by memory).
+template <int NBITS, bool ZT, int T, int PER>
+__device__ __forceinline__ void stripe_one_reg_body(const char* q_in, float* stripe_res, char* q_out, float* agg_out, const RegGeom& c,
+                                                    uint32_t column, f32x4* smem_v4)
+{
+    using PS = PackShape<NBITS>;
+    static_assert(NBITS < 32, "32-bit codes are whole QWords: nothing to assemble");
+    constexpr uint32_t NW = T / 64;
+    typedef u32x4 u32x4_u __attribute__((aligned(4)));
+    float* red = reinterpret_cast<float*>(smem_v4);
+    uint32_t* red_u = reinterpret_cast<uint32_t*>(red + 2 * NW);
+    uint32_t* words = reinterpret_cast<uint32_t*>(red + kRegRedSlots);
+    const uint32_t tid = threadIdx.x;
+    const size_t base = (size_t) column * c.rows;
+    const size_t rec = (size_t) column * c.qcol;
+    for (uint32_t x = tid; x < c.nq; x += T)
+        words[x] = 0u;
+    float* sres = stripe_res + base;
+    const uint32_t head = (4u - (uint32_t) ((reinterpret_cast<uintptr_t>(sres) >> 2) & 3u)) & 3u;
+    const uint32_t pieces = (c.rows - head) >> 2;
+    const uint32_t tail = c.rows - head - 4 * pieces;
+    const bool has_edge = tid < head + tail;
+    const uint32_t edge_at = tid < head ? tid : c.rows - tail + (tid - head);
+    const uint32_t shift = column_shift(sres + head, c.line_shift);
+    const uint32_t last = pieces - 1;
+    const f32x4* r4 = reinterpret_cast<const f32x4*>(sres + head);
+    f32x4 a[PER];
+    {
+        const uint32_t t = opaque(tid);
+#pragma unroll
+        for (int u = 0; u < PER; ++u)
+            a[u] = __builtin_nontemporal_load(r4 + slot_piece(t + T * u, shift, last));
+    }
+    const float* header = reinterpret_cast<const float*>(q_in + rec);
+    const uint32_t* bits = reinterpret_cast<const uint32_t*>(q_in + rec + 8);
+    const float lo = header[0];
+    const float uf = make_ufactor<NBITS>(lo, header[1]);
+    const float val0 = unquantize_value<NBITS>(uf, lo, 0u);
+    const float val1 = unquantize_value<NBITS>(uf, lo, 1u);
+    auto value_of = [&](uint32_t word, uint32_t k) -> float {
+        if constexpr (NBITS == 1)
+            return pick_level(word, k, val0, val1);
+        else
+            return unquantize_value<NBITS>(uf, lo, (word >> (k * PS::SHIFT)) & PS::CODEMASK);
+    };
+    float* ag = agg_out != nullptr ? agg_out + base : nullptr;
+    // (pieces whose QWords are in flight together: three or four measured the same and spill)
+    constexpr int B = 2;
+    const float inv_nq = small_divisor(c.nq); // (element numbers are far below the 2^20 that small_div takes)
+#pragma unroll
+    for (int u0 = 0; u0 < PER; u0 += B)
+    {
+        const uint32_t t = opaque(tid);
+        u32x4 b[B];
+        uint32_t k[B], w[B];
+#pragma unroll
+        for (int u = u0; u < u0 + B && u < PER; ++u)
+        {
+            const uint32_t e0 = head + 4 * slot_piece(t + T * u, shift, last);
+            k[u - u0] = small_div(e0, inv_nq);
+            w[u - u0] = e0 - k[u - u0] * c.nq;
+            b[u - u0] = *reinterpret_cast<const u32x4_u*>(bits + min(w[u - u0], c.nq - 4));
+        }
+#pragma unroll
+        for (int u = u0; u < u0 + B && u < PER; ++u)
+        {
+            f32x4 x;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                x[e] = value_of(b[u - u0][e], k[u - u0]);
+            if (w[u - u0] + 4 > c.nq)
+            {
+                // the piece runs past the last QWord: its later elements are the next bit position of the first ones
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                {
+                    const bool wraps = w[u - u0] + e >= c.nq;
+                    x[e] = value_of(bits[wraps ? w[u - u0] + e - c.nq : w[u - u0] + e], wraps ? k[u - u0] + 1 : k[u - u0]);
+                }
+            }
+            if (ag != nullptr && slot_valid(t + T * u, shift, pieces))
+            {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    ag[head + 4 * (t + T * u - shift) + e] = x[e];
+            }
+            a[u] = x + a[u];
+        }
+    }
+    float edge = 0.0f;
+    if (has_edge)
+    {
+        const uint32_t edge_k = edge_at / c.nq;
+        edge = value_of(bits[edge_at - edge_k * c.nq], edge_k);
+        if (ag != nullptr)
+            ag[edge_at] = edge;
+        edge = edge + sres[edge_at];
+    }
+    // (every thread has its QWords before reg_stats_pack's last barrier but one, the record is written after it: q_out may be q_in)
+    reg_stats_pack<NBITS, ZT, T, PER>(a, edge, has_edge, edge_at, head, pieces, shift, c, red, red_u, words, sres, q_out + rec);
+}
+
 // The 1-bit tall stripe reduction with up to eight workers decoded together from a worker-minor table in LDS. The kernel
 // above reads a piece's four QWords of one worker at a time (lanes 16 bytes apart, 4 bytes each: a quarter of the LDS
 // banks serve every access, and counters put the kernel at 122 us of LDS time for a 219 us run at 100000 x 512, K = 8).

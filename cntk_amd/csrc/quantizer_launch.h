@@ -228,13 +228,14 @@ hipError_t family_strip_occupancy(size_t nbits, bool zt, bool stripe, int* per_c
 hipError_t family_unquantize(size_t nbits, hipStream_t s, LaunchEvents ev, const char* q, float* out, const UnquantizePlan& p, int add);
 hipError_t family_batch_quantize(size_t nbits, bool zt, hipStream_t s, LaunchEvents ev, const QuantizeBatchEntry* entries, const uint32_t* begins,
                                  uint32_t count, uint32_t total_blocks, size_t lds);
+// one: the stripes are a single worker's
 hipError_t family_batch_stripe(size_t nbits, bool zt, hipStream_t s, LaunchEvents ev, const StripeBatchEntry* entries, const uint32_t* begins,
-                               uint32_t count, uint32_t total_blocks, size_t lds, bool wide);
+                               uint32_t count, uint32_t total_blocks, size_t lds, bool wide, bool one);
 // members of the register grids: threads 256 or 1024; wide: some of more than 8 pieces per thread
 hipError_t family_batch_reg_quantize(size_t nbits, bool zt, hipStream_t s, LaunchEvents ev, const QuantizeBatchEntry* entries, const uint32_t* begins,
                                      uint32_t count, uint32_t total_blocks, size_t lds, uint32_t threads, bool wide);
 hipError_t family_batch_reg_stripe(size_t nbits, bool zt, hipStream_t s, LaunchEvents ev, const StripeBatchEntry* entries, const uint32_t* begins,
-                                   uint32_t count, uint32_t total_blocks, size_t lds, uint32_t threads, bool wide);
+                                   uint32_t count, uint32_t total_blocks, size_t lds, uint32_t threads, bool wide, bool one);
 hipError_t launch_unquantize_batch(hipStream_t s, LaunchEvents ev, const UnquantizeBatchEntry* entries, const uint32_t* begins, uint32_t count,
                                    uint32_t total_blocks, size_t nbits, bool add, size_t lds);
 
@@ -1155,10 +1156,10 @@ inline hipError_t launch_quantize_batch(hipStream_t s, LaunchEvents ev, const Qu
 }
 
 inline hipError_t launch_stripe_reduce_batch(hipStream_t s, LaunchEvents ev, const StripeBatchEntry* entries, const uint32_t* begins,
-                                             uint32_t count, uint32_t total_blocks, size_t lds, size_t nbits, bool zt, bool wide)
+                                             uint32_t count, uint32_t total_blocks, size_t lds, size_t nbits, bool zt, bool wide, bool one)
 {
     zt = zt && (nbits == 1);
-    return family_batch_stripe(nbits, zt, s, ev, entries, begins, count, total_blocks, lds, wide);
+    return family_batch_stripe(nbits, zt, s, ev, entries, begins, count, total_blocks, lds, wide, one);
 }
 
 // which kernel family launch_stripe_reduce takes by itself for a stripe of this height: columns (true) or tiles
