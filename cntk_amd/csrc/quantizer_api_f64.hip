@@ -68,12 +68,25 @@ struct BatchAbi<double>
         blocks = (e.t.cols + e.t.cols_per_tile - 1) / e.t.cols_per_tile;
         return true;
     }
-    static int quantize_register_member(const QItem&, size_t, QEntry&, size_t&, uint64_t&, bool) { return kBatchOwnLaunch; }
-    static bool quantize_entry_wide(const QEntry&) { return false; }
-    static hipError_t launch_quantize_register_members(hipStream_t, LaunchEvents, const QEntry*, const uint32_t*, uint32_t, uint32_t, size_t, size_t,
-                                                       bool, uint32_t, bool)
+    // Fills the geometry of a member of the register grid, with the slots dealt as launch_quantize deals them; kBatchOwnLaunch: none.
+    static int quantize_register_member(const QItem& it, size_t nbits, QEntry& e, size_t& lds, uint64_t& blocks, bool)
     {
-        return hipErrorInvalidValue; // no member is of these classes
+        if (f64::quantize_auto_path(it.in, it.res_in, it.res_out, it.rows, nbits) != kPathReg ||
+            !f64::reg_applicable(it.in, it.res_in, it.res_out, it.rows, nbits))
+            return kBatchOwnLaunch;
+        e.r = f64::make_reg_geom(it.rows, nbits, f64::reg_line_shift(it.res_in, it.rows));
+        e.kind = f64::reg_batch_kind(e.r);
+        if (e.kind == 0)
+            return kBatchOwnLaunch;
+        lds = f64::reg_lds_bytes64(e.r);
+        blocks = it.cols;
+        return kBatchReg1024;
+    }
+    static bool quantize_entry_wide(const QEntry&) { return false; }
+    static hipError_t launch_quantize_register_members(hipStream_t s, LaunchEvents ev, const QEntry* de, const uint32_t* db, uint32_t members,
+                                                       uint32_t blocks, size_t lds, size_t nbits, bool zt, uint32_t, bool)
+    {
+        return f64::dispatch_nbits64<f64::RegBatchLauncher64>(nbits, zt && nbits == 1, s, ev, de, db, members, blocks, lds);
     }
     static bool first_in_grid(const QEntry&) { return false; }
     static hipError_t launch_quantize_members(hipStream_t s, LaunchEvents ev, const QEntry* de, const uint32_t* db, uint32_t members,
@@ -138,11 +151,23 @@ struct BatchAbi<double>
         blocks = (e.t.cols + e.t.cols_per_tile - 1) / e.t.cols_per_tile;
         return lds <= f64::kMaxLdsBytes;
     }
-    static int stripe_register_member(const SItem&, size_t, size_t, SEntry&, size_t&, uint64_t&) { return kBatchOwnLaunch; }
-    static hipError_t launch_stripe_register_members(hipStream_t, LaunchEvents, const SEntry*, const uint32_t*, uint32_t, uint32_t, size_t, size_t,
-                                                     bool, uint32_t, bool, bool)
+    // ... with the slots dealt as launch_stripe_reduce deals them
+    static int stripe_register_member(const SItem& it, size_t, size_t nbits, SEntry& e, size_t& lds, uint64_t& blocks)
     {
-        return hipErrorInvalidValue; // no member is of these classes
+        if (it.rows > f64::stripe_reduce_max_rows(nbits) || !f64::stripe_uses_reg(it.rows, nbits))
+            return kBatchOwnLaunch;
+        e.r = f64::make_reg_geom(it.rows, nbits, f64::reg_line_shift(it.stripe_res, it.rows));
+        e.kind = f64::reg_batch_kind(e.r);
+        if (e.kind == 0)
+            return kBatchOwnLaunch;
+        lds = f64::stripe_reg_lds_bytes64(e.r);
+        blocks = it.stripe_cols;
+        return kBatchReg1024;
+    }
+    static hipError_t launch_stripe_register_members(hipStream_t s, LaunchEvents ev, const SEntry* de, const uint32_t* db, uint32_t members,
+                                                     uint32_t blocks, size_t lds, size_t nbits, bool zt, uint32_t, bool, bool)
+    {
+        return f64::dispatch_nbits64<f64::StripeRegBatchLauncher64>(nbits, zt && nbits == 1, s, ev, de, db, members, blocks, lds);
     }
     static bool stripe_entry_wide(const SEntry&) { return false; }
     static hipError_t launch_stripe_members(hipStream_t s, LaunchEvents ev, const SEntry* de, const uint32_t* db, const SEntry*, const uint32_t*,

@@ -634,18 +634,17 @@ __device__ __forceinline__ void reg_stats_pack(f64x2 (&a)[PER], double edge, boo
 }
 
 template <int NBITS, bool ZT, int T, int PER>
-__global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(reg_waves<T, PER>(), reg_waves<T, PER>()))) void quantize_reg_kernel(
-    const double* __restrict__ g, const double* r_in, double* r_out, char* __restrict__ q, RegGeom c)
+__device__ __forceinline__ void quantize_reg_body(const double* __restrict__ g, const double* r_in, double* r_out, char* __restrict__ q,
+                                                  const RegGeom& c, uint32_t column, f32x4* smem_v4)
 {
     static_assert(NBITS < 64, "64-bit codes are whole QWords: nothing to assemble");
     constexpr uint32_t NW = T / 64;
-    extern __shared__ f32x4 smem_v4[];
     double* red = reinterpret_cast<double*>(smem_v4);
     uint32_t* red_u = reinterpret_cast<uint32_t*>(red + 2 * NW);
     unsigned long long* words = reinterpret_cast<unsigned long long*>(red + kRegRedSlots);
     const uint32_t tid = threadIdx.x;
-    const size_t base = (size_t) blockIdx.x * c.rows;
-    char* qc = q + (size_t) blockIdx.x * c.qcol;
+    const size_t base = (size_t) column * c.rows;
+    char* qc = q + (size_t) column * c.qcol;
     for (uint32_t x = tid; x < c.nq; x += T)
         words[x] = 0ull;
     // the column may start 8 bytes off a 16-byte boundary and have an odd height: one element before the first aligned
@@ -685,6 +684,14 @@ __global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(reg_waves<T, 
     reg_stats_pack<NBITS, ZT, T, PER>(a, edge, has_edge, edge_at, head, pieces, shift, c, red, red_u, words, r_out + base, qc);
 }
 
+template <int NBITS, bool ZT, int T, int PER>
+__global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(reg_waves<T, PER>(), reg_waves<T, PER>()))) void quantize_reg_kernel(
+    const double* __restrict__ g, const double* r_in, double* r_out, char* __restrict__ q, RegGeom c)
+{
+    extern __shared__ f32x4 smem_v4[];
+    quantize_reg_body<NBITS, ZT, T, PER>(g, r_in, r_out, q, c, blockIdx.x, smem_v4);
+}
+
 // Stripe reduction in the register kernel's shape (the fp32 stripe_reduce_reg_kernel on doubles): 1024 threads per owned
 // column, the running sum of the decoded stripes in registers. The workers are taken one at a time in the fixed order
 // (owner first, then ascending rank): the worker's packed record goes to LDS in one coalesced copy, each thread decodes
@@ -697,20 +704,19 @@ __host__ __device__ inline size_t stripe_reg_lds_bytes64(const RegGeom& c)
 }
 
 template <int NBITS, bool ZT, int PER>
-__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(reg_waves<1024, PER>(), reg_waves<1024, PER>()))) void stripe_reduce_reg_kernel(
-    StripeSources src, double* stripe_res, char* q_out, double* agg_out, RegGeom c)
+__device__ __forceinline__ void stripe_reduce_reg_body(const StripeSources& src, double* stripe_res, char* q_out, double* agg_out, const RegGeom& c,
+                                                       uint32_t column, f32x4* smem_v4)
 {
     using PS = PackShape<NBITS>;
     static_assert(NBITS < 64, "64-bit codes are whole QWords: nothing to assemble");
     constexpr uint32_t T = 1024, NW = T / 64;
-    extern __shared__ f32x4 smem_v4[];
     double* red = reinterpret_cast<double*>(smem_v4);
     uint32_t* red_u = reinterpret_cast<uint32_t*>(red + 2 * NW);
     unsigned long long* words = reinterpret_cast<unsigned long long*>(red + kRegRedSlots);
     unsigned long long* pw = words + c.nq; // one worker's record: lower, upper, QWords
     const uint32_t tid = threadIdx.x;
-    const size_t base = (size_t) blockIdx.x * c.rows;
-    const size_t rec = (size_t) blockIdx.x * c.qcol;
+    const size_t base = (size_t) column * c.rows;
+    const size_t rec = (size_t) column * c.qcol;
     for (uint32_t x = tid; x < c.nq; x += T)
         words[x] = 0ull;
     // the column as the quantize kernel would see it: an element before the first aligned pair, pairs, an element after
@@ -833,6 +839,14 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(reg_waves<
     reg_stats_pack<NBITS, ZT, T, PER>(a, edge, has_edge, edge_at, head, pieces, shift, c, red, red_u, words, sres, q_out + rec);
 }
 
+template <int NBITS, bool ZT, int PER>
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(reg_waves<1024, PER>(), reg_waves<1024, PER>()))) void stripe_reduce_reg_kernel(
+    StripeSources src, double* stripe_res, char* q_out, double* agg_out, RegGeom c)
+{
+    extern __shared__ f32x4 smem_v4[];
+    stripe_reduce_reg_body<NBITS, ZT, PER>(src, stripe_res, q_out, agg_out, c, blockIdx.x, smem_v4);
+}
+
 // ---- whole gradient sets in one launch (the fp32 batch kernels on doubles) ------------------------------------------
 //
 // The workgroups of all member matrices form one grid; `begins` (count + 1 entries, ascending) gives the first workgroup
@@ -845,7 +859,13 @@ struct QuantizeBatchEntry64
     const double* r_in;
     double* r_out;
     char* q;
-    TileGeom t;
+    uint32_t kind; // 8 / 9: members of the register grid, up to 4 / 6 pieces for each of 1024 threads (r); otherwise column tiles (t)
+    uint32_t pad;
+    union
+    {
+        TileGeom t;
+        RegGeom r;
+    };
 };
 
 template <int NBITS, bool ZT>
@@ -865,7 +885,13 @@ struct StripeBatchEntry64
     double* stripe_res;
     char* q_out;
     double* agg_out;
-    TileGeom t;
+    uint32_t kind; // as QuantizeBatchEntry64 has it
+    uint32_t pad;
+    union
+    {
+        TileGeom t;
+        RegGeom r;
+    };
 };
 
 template <int NBITS, bool ZT>
@@ -891,6 +917,40 @@ struct UnquantizeBatchEntry64
     UnqTileGeom tile;
     UnqFlatGeom flat;
 };
+
+// The members whose columns stay in registers on 1024 threads, in one grid (see the float side): eight workers' bias columns of
+// 6883 rows were eight launches of 7 us each.
+constexpr int kRegBatchPer[2] = {4, 6};
+
+template <int NBITS, bool ZT>
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(reg_waves<1024, kRegBatchPer[1]>(), reg_waves<1024, kRegBatchPer[1]>()))) void
+quantize_reg_batch_kernel64(const QuantizeBatchEntry64* __restrict__ entries, const uint32_t* __restrict__ begins, uint32_t count)
+{
+    extern __shared__ f32x4 smem_v4[];
+    const uint32_t e = batch_find(begins, count, blockIdx.x);
+    const uint32_t column = blockIdx.x - begins[e];
+    const QuantizeBatchEntry64& en = entries[e];
+    const RegGeom c = en.r;
+    if (en.kind == 8)
+        quantize_reg_body<NBITS, ZT, 1024, kRegBatchPer[0]>(en.g, en.r_in, en.r_out, en.q, c, column, smem_v4);
+    else
+        quantize_reg_body<NBITS, ZT, 1024, kRegBatchPer[1]>(en.g, en.r_in, en.r_out, en.q, c, column, smem_v4);
+}
+
+template <int NBITS, bool ZT>
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(reg_waves<1024, kRegBatchPer[1]>(), reg_waves<1024, kRegBatchPer[1]>()))) void
+stripe_reduce_reg_batch_kernel64(const StripeBatchEntry64* __restrict__ entries, const uint32_t* __restrict__ begins, uint32_t count)
+{
+    extern __shared__ f32x4 smem_v4[];
+    const uint32_t e = batch_find(begins, count, blockIdx.x);
+    const uint32_t column = blockIdx.x - begins[e];
+    const StripeBatchEntry64& en = entries[e];
+    const RegGeom c = en.r;
+    if (en.kind == 8)
+        stripe_reduce_reg_body<NBITS, ZT, kRegBatchPer[0]>(en.src, en.stripe_res, en.q_out, en.agg_out, c, column, smem_v4);
+    else
+        stripe_reduce_reg_body<NBITS, ZT, kRegBatchPer[1]>(en.src, en.stripe_res, en.q_out, en.agg_out, c, column, smem_v4);
+}
 
 template <int NBITS>
 __global__ __launch_bounds__(256) void unquantize_batch_kernel64(const UnquantizeBatchEntry64* __restrict__ entries,

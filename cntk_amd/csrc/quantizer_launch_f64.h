@@ -399,6 +399,47 @@ inline hipError_t launch_stripe_reduce(hipStream_t s, LaunchEvents ev, const Str
     return dispatch_nbits64<StripeLauncher>(nbits, zt, s, ev, src, stripe_res, static_cast<char*>(q_out), agg_out, t);
 }
 
+// The kind of the register grid's member of this geometry; 0: more pieces per thread than its kernels hold.
+inline uint32_t reg_batch_kind(const RegGeom& c)
+{
+    const uint32_t per = (c.pieces + (c.line_shift ? 7u : 0u) + kRegThreads - 1) / kRegThreads;
+    return per <= (uint32_t) kRegBatchPer[0] ? 8u : (per <= (uint32_t) kRegBatchPer[1] ? 9u : 0u);
+}
+
+template <int NBITS, bool ZT>
+struct RegBatchLauncher64
+{
+    static hipError_t run(hipStream_t s, LaunchEvents ev, const QuantizeBatchEntry64* entries, const uint32_t* begins, uint32_t count, uint32_t blocks,
+                          size_t lds)
+    {
+        if constexpr (NBITS >= 64)
+            return hipErrorInvalidValue;
+        else
+        {
+            hipExtLaunchKernelGGL((quantize_reg_batch_kernel64<NBITS, ZT>), dim3(blocks), dim3(kRegThreads), lds, s, ev.start, ev.stop, 0, entries, begins,
+                                  count);
+            return hipGetLastError();
+        }
+    }
+};
+
+template <int NBITS, bool ZT>
+struct StripeRegBatchLauncher64
+{
+    static hipError_t run(hipStream_t s, LaunchEvents ev, const StripeBatchEntry64* entries, const uint32_t* begins, uint32_t count, uint32_t blocks,
+                          size_t lds)
+    {
+        if constexpr (NBITS >= 64)
+            return hipErrorInvalidValue;
+        else
+        {
+            hipExtLaunchKernelGGL((stripe_reduce_reg_batch_kernel64<NBITS, ZT>), dim3(blocks), dim3(kRegThreads), lds, s, ev.start, ev.stop, 0, entries,
+                                  begins, count);
+            return hipGetLastError();
+        }
+    }
+};
+
 template <int NBITS>
 inline hipError_t launch_unquantize_n(hipStream_t s, LaunchEvents ev, const char* q, double* out, const UnqGeom& t, bool vec, int add)
 {

@@ -15,26 +15,37 @@ pytestmark = pytest.mark.gpu
 # than six pieces each (6148 .. 14336 rows) and on 1024
 EDGE = [(2049, 40), (4071, 5), (4099, 3), (7166, 9), (7169, 3), (9305, 7), (12258, 2), (16359, 2), (16361, 3), (24547, 2), (24555, 1)]
 WHOLE = [(6148, 70), (8192, 40), (9304, 33), (14308, 36), (14336, 34), (14340, 3), (16384, 2), (24576, 2), (24580, 1)]
+# doubles: from 6145 rows on 1024 threads, up to six pieces each in the shared grid
+DOUBLE = [(6145, 3), (6883, 1), (6884, 40), (8187, 2), (8192, 3), (12258, 2), (12288, 2), (12303, 2), (300, 30), (6144, 2)]
 SMALL = [(64, 64), (429, 37), (21, 960), (2048, 1), (9280, 1), (13000, 2)]
 
 
-def _matrices(shapes, nbits, seed):
+def _matrices(shapes, nbits, seed, dtype=torch.float32):
     # slices of one allocation at odd offsets: the columns of a matrix start anywhere within 16 bytes, the same in both runs
     gen = torch.Generator(device="cuda:0")
     gen.manual_seed(datagen.case_seed(seed))
     out = []
     for i, (r, c) in enumerate(shapes):
         off = 0 if r % 4 == 0 else i % 4
-        g, res = [(torch.randn(r * c + 4, generator=gen, device="cuda:0") * s)[off:off + r * c] for s in (0.01, 0.002)]
-        out.append((Matrix(r, c, 0, g), Matrix(r, c, 0, res), QuantizedMatrix(r, c, nbits, 0)))
+        g, res = [(torch.randn(r * c + 4, generator=gen, device="cuda:0") * s).to(dtype)[off:off + r * c] for s in (0.01, 0.002)]
+        out.append((Matrix(r, c, 0, g, dtype=dtype), Matrix(r, c, 0, res, dtype=dtype), QuantizedMatrix(r, c, nbits, 0, dtype=dtype)))
     return out
 
 
 @pytest.mark.parametrize("nbits,zt", [(1, False), (1, True), (2, False), (8, False), (16, False)])
 @pytest.mark.parametrize("shapes", [EDGE, WHOLE, EDGE[:2] + SMALL, EDGE + WHOLE + SMALL], ids=["edge", "whole", "few", "all"])
 def test_quantize(shapes, nbits, zt):
+    _check_quantize(shapes, nbits, zt, torch.float32)
+
+
+@pytest.mark.parametrize("nbits,zt", [(1, False), (1, True), (4, False), (32, False)])
+def test_quantize_doubles(nbits, zt):
+    _check_quantize(DOUBLE, nbits, zt, torch.float64)
+
+
+def _check_quantize(shapes, nbits, zt, dtype):
     qz = MatrixQuantizerImpl.Create(0, False)
-    one, many = _matrices(shapes, nbits, nbits), _matrices(shapes, nbits, nbits)
+    one, many = _matrices(shapes, nbits, nbits, dtype), _matrices(shapes, nbits, nbits, dtype)
     for _ in range(2):
         for g, r, q in one:
             qz.QuantizeAsync(g, r, q, r, zt)
@@ -46,23 +57,32 @@ def test_quantize(shapes, nbits, zt):
             assert parity.bits_equal(r1.to_numpy(), r2.to_numpy()), ("residual", shape)
 
 
-def _stripes(qz, shapes, nbits, zt, k):
-    workers = [_matrices(shapes, nbits, 20 * w + nbits) for w in range(k)]
+def _stripes(qz, shapes, nbits, zt, k, dtype=torch.float32):
+    workers = [_matrices(shapes, nbits, 20 * w + nbits, dtype) for w in range(k)]
     for ms in workers:
         for g, r, q in ms:
             qz.QuantizeAsync(g, r, q, r, zt)
-    sres = [r for _, r, _ in _matrices(shapes, nbits, 999)]
-    agg = [Matrix(r, c) for r, c in shapes]
+    sres = [r for _, r, _ in _matrices(shapes, nbits, 999, dtype)]
+    agg = [Matrix(r, c, dtype=dtype) for r, c in shapes]
     return [[ms[i][2] for ms in workers] for i in range(len(shapes))], sres, agg
 
 
 @pytest.mark.parametrize("nbits,zt,k", [(1, False, 1), (1, True, 8), (1, False, 9), (2, False, 3), (8, False, 1), (8, False, 8), (16, False, 2)])
 @pytest.mark.parametrize("shapes", [EDGE, WHOLE, EDGE[:2] + SMALL, EDGE + WHOLE + SMALL], ids=["edge", "whole", "few", "all"])
 def test_stripe_reduction(shapes, nbits, zt, k):
+    _check_stripe_reduction(shapes, nbits, zt, k, torch.float32)
+
+
+@pytest.mark.parametrize("nbits,zt,k", [(1, True, 1), (1, False, 8), (8, False, 3), (32, False, 2)])
+def test_stripe_reduction_doubles(nbits, zt, k):
+    _check_stripe_reduction(DOUBLE, nbits, zt, k, torch.float64)
+
+
+def _check_stripe_reduction(shapes, nbits, zt, k, dtype):
     qz = MatrixQuantizerImpl.Create(0, False)
     owner = k // 2
-    q1, s1, a1 = _stripes(qz, shapes, nbits, zt, k)
-    q2, s2, a2 = _stripes(qz, shapes, nbits, zt, k)
+    q1, s1, a1 = _stripes(qz, shapes, nbits, zt, k, dtype)
+    q2, s2, a2 = _stripes(qz, shapes, nbits, zt, k, dtype)
     for q, s, a in zip(q1, s1, a1):
         qz.StripeReduceAsync(q, owner, s, q[owner], zt, agg_out=a)
     qz.StripeReduceBatchAsync([(q, s, q[owner], a) for q, s, a in zip(q2, s2, a2)], owner, zt)
