@@ -96,22 +96,44 @@ def _check_stripe_reduction(shapes, nbits, zt, k, dtype):
 
 def test_recorded_stripes_without_a_table():
     """Stripes that each had a launch of their own could always be recorded without an eager call before; they still can."""
+    _check_recorded([(9305, 3), (7169, 2), (4099, 2)], 2, 2, eager_first=False)
+
+
+@pytest.mark.parametrize("shapes,nbits,k", [([(8192, 40), (40, 1)], 2, 1), ([(14336, 34), (64, 64)], 8, 2), ([(9304, 33), (2048, 3), (9305, 2)], 4, 1),
+                                            ([(8192, 40), (9304, 5)], 2, 2), ([(6148, 70), (429, 37), (21, 960)], 2, 1)])
+def test_recorded_stripes_after_a_call(shapes, nbits, k):
+    """A list that was called once can be recorded, whatever the call made of it: a layer of whole pieces and its bias are a member of
+    a register grid and one of the general grids, with nothing to share a grid with in either, so that the call builds no table."""
+    _check_recorded(shapes, nbits, k, eager_first=True)
+
+
+def _check_recorded(shapes, nbits, k, eager_first):
     qz = MatrixQuantizerImpl.Create(0, False)
-    shapes = [(9305, 3), (7169, 2), (4099, 2)]
-    q1, s1, a1 = _stripes(qz, shapes, 2, False, 2)
-    q2, s2, a2 = _stripes(qz, shapes, 2, False, 2)
+    q1, s1, a1 = _stripes(qz, shapes, nbits, False, k)
+    q2, s2, a2 = _stripes(qz, shapes, nbits, False, k)
+
+    def one_by_one():
+        for q, s, a in zip(q1, s1, a1):
+            qz.StripeReduceAsync(q, 0, s, q[0], False, agg_out=a)
+        qz.WaitStripeReduceDone()
+
+    def as_a_set():
+        qz.StripeReduceBatchAsync([(q, s, q[0], a) for q, s, a in zip(q2, s2, a2)], 0, False)
+
+    if eager_first:
+        one_by_one()
+        as_a_set()
     torch.cuda.synchronize()
     side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
     qz.SetMainStream(side.cuda_stream)
     with torch.cuda.graph(graph, stream=side):
-        qz.StripeReduceBatchAsync([(q, s, q[0], a) for q, s, a in zip(q2, s2, a2)], 0, False)
+        as_a_set()
     qz.SetMainStream(torch.cuda.current_stream().cuda_stream)
     for _ in range(3):
-        for q, s, a in zip(q1, s1, a1):
-            qz.StripeReduceAsync(q, 0, s, q[0], False, agg_out=a)
-        qz.WaitStripeReduceDone()
+        one_by_one()
         graph.replay()
         torch.cuda.synchronize()
         for i, shape in enumerate(shapes):
             assert np.array_equal(q1[i][0].to_numpy(), q2[i][0].to_numpy()), ("packed", shape)
             assert parity.bits_equal(s1[i].to_numpy(), s2[i].to_numpy()), ("stripe residual", shape)
+            assert parity.bits_equal(a1[i].to_numpy(), a2[i].to_numpy()), ("aggregate", shape)
