@@ -985,6 +985,11 @@ unsigned cntkq_debug_strip_max_strips_f64(cntkq_quantizer* h, size_t nbits, int 
     return strip_max_strips<double>(nbits, zero_threshold_for_1bit != 0 && nbits == 1);
 }
 
+size_t cntkq_debug_staging_bytes(const cntkq_quantizer* h)
+{
+    return h != nullptr ? h->staging_bytes : 0;
+}
+
 int cntkq_debug_attach_events(cntkq_quantizer* h, void* start_event, void* stop_event)
 {
     if (h == nullptr)

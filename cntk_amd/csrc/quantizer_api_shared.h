@@ -187,7 +187,7 @@ struct cntkq_quantizer
     bool quantize_included_fetch = false;
     bool fetch_pending = false;   // a device-to-host copy out of the staging buffer may still be running
     bool staging_read_pending = false; // a kernel reading the staging buffer may still be running
-    char* staging = nullptr;      // device buffer used when the packed matrix lives in host memory
+    char* staging = nullptr;      // device buffer used when the packed matrix lives in host memory that the kernels do not take
     size_t staging_bytes = 0;
     // entry tables of the batched calls, one for quantize and one for unquantize. A gradient set is the same list of
     // matrices step after step, so the table built for a list is kept (host key, pinned host copy, device copy, launch
@@ -267,20 +267,31 @@ inline int ensure_staging(cntkq_quantizer* h, size_t bytes)
     return CNTKQ_OK;
 }
 
-// Whether the device reaches a host-resident packed matrix at the address the host has it at (pinned memory: hipHostMalloc,
-// registered memory, torch's pin_memory), from its first byte to its last. Kernels then write and read it where it lies.
-// hipPointerGetAttributes cannot tell about the end of the range, so both ends are asked for.
-inline bool device_reaches_host(const void* p, size_t bytes)
+// Whether the kernels may write and read a host-resident packed matrix where it lies: pinned memory that the device reaches at the
+// address the host has it at, from its first byte to its last (hipPointerGetAttributes cannot tell about the end of the range, so
+// both ends are asked for), and that is coherent. Nothing makes the device's caches give up a line of non-coherent memory between
+// the quantize step and the decode of what the host has received into it, and events that do not release to the system leave
+// what a kernel wrote there invisible to the host; copies give both guarantees, so such memory is staged like pageable memory. By its
+// flags memory is coherent that was allocated hipHostMallocDefault (as torch's pin_memory does), Mapped or Coherent and with none
+// of the flags that say otherwise; the runtime's pool flags name the same allocations fine-grained, Portable or WriteCombined ones
+// by themselves coarse-grained, with HIP_HOST_COHERENT unset or 0.
+inline bool kernels_take_host_memory(const void* p, size_t bytes)
 {
-    char* first = static_cast<char*>(const_cast<void*>(p));
-    void* d[2] = {nullptr, nullptr};
-    for (int i = 0; i < 2; ++i)
-        if (hipHostGetDevicePointer(&d[i], first + (i == 0 ? 0 : bytes - 1), 0) != hipSuccess)
+    char* ends[2] = {static_cast<char*>(const_cast<void*>(p)), static_cast<char*>(const_cast<void*>(p)) + (bytes - 1)};
+    for (char* end : ends)
+    {
+        void* d = nullptr;
+        unsigned flags = 0;
+        if (hipHostGetDevicePointer(&d, end, 0) != hipSuccess || hipHostGetFlags(&flags, end) != hipSuccess)
         {
             (void) hipGetLastError(); // pageable memory is no error of the call: it goes through the staging buffer
             return false;
         }
-    return d[0] == first && d[1] == first + (bytes - 1);
+        if (d != end || (flags & ~(unsigned) (hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent)) != 0 ||
+            (flags != hipHostMallocDefault && (flags & (hipHostMallocMapped | hipHostMallocCoherent)) == 0))
+            return false;
+    }
+    return true;
 }
 
 // Whether work issued on `s` is being recorded into a graph instead of executed.
@@ -496,10 +507,10 @@ int quantize_async_impl(cntkq_quantizer* h, const E* in, const E* res_in, size_t
     if (capturing && qbuf_on_host)
         return fail(CNTKQ_INVALID_ARGUMENT, "cntkq_quantize_async: a host-resident packed matrix needs copies on other streams and cannot "
                                             "be recorded into a graph");
-    // Pinned host memory is written by the kernel itself while it runs: the transfer needs no stream of its own, no copy after
+    // Coherent pinned host memory is written by the kernel itself while it runs: the transfer needs no stream of its own, no copy after
     // the kernel and none of the events that order the two (512 x 512 at 1 bit, quantize, wait, unquantize, wait: 95 us
     // through the staging buffer, 33 us so; 2048 x 9304: 214 and 150 us).
-    const bool staged = qbuf_on_host && !device_reaches_host(qbuf, need);
+    const bool staged = qbuf_on_host && !kernels_take_host_memory(qbuf, need);
     if (staged)
     {
         int rc = ensure_staging(h, need);
@@ -570,7 +581,7 @@ int unquantize_async_impl(cntkq_quantizer* h, const void* qbuf, size_t qbuf_byte
     if (qbuf_on_host && stream_capturing(s))
         return fail(CNTKQ_INVALID_ARGUMENT, "cntkq_unquantize_async: a host-resident packed matrix needs copies on other streams and "
                                             "cannot be recorded into a graph");
-    const bool reached = qbuf_on_host && device_reaches_host(qbuf, need);
+    const bool reached = qbuf_on_host && kernels_take_host_memory(qbuf, need);
     if (qbuf_on_host && !reached)
     {
         int rc = ensure_staging(h, need);

@@ -41,6 +41,10 @@ int cntkq_debug_set_strip_spin_limit(cntkq_quantizer* h, unsigned limit);
 unsigned cntkq_debug_strip_max_strips(cntkq_quantizer* h, size_t nbits, int zero_threshold_for_1bit);
 unsigned cntkq_debug_strip_max_strips_f64(cntkq_quantizer* h, size_t nbits, int zero_threshold_for_1bit);
 
+/* Bytes of the handle's device staging buffer: 0 until a packed matrix lay in host memory that the kernels do not write and
+ * read themselves. */
+size_t cntkq_debug_staging_bytes(const cntkq_quantizer* h);
+
 /* Ties caller-owned hipEvent_t objects (either may be NULL) to the NEXT kernel this handle launches: start_event is
  * set when that kernel begins, stop_event when it has finished, by the dispatch itself. Used to time single kernels
  * without putting extra commands into the stream. The stop event also becomes what the matching Wait call waits on,

@@ -131,9 +131,10 @@ int cntkq_stream_wait_event(cntkq_quantizer* h, void* hip_event);
  *   in, res_in, res_out : device, rows x cols fp32; res_out may be the same pointer as res_in (in place),
  *                         no other overlap is allowed.
  *   qbuf                : packed matrix, qbuf_bytes == cntkq_qmatrix_bytes(rows, cols, nbits);
- *                         device memory, or (qbuf_on_host != 0) host memory: pinned host memory is written by the
- *                         kernel itself, for pageable memory the packed data is produced in a device staging buffer
- *                         owned by the handle and copied out.
+ *                         device memory, or (qbuf_on_host != 0) host memory: coherent pinned memory (hipHostMalloc with
+ *                         hipHostMallocDefault, Mapped or Coherent) is written by the kernel itself; for any other
+ *                         (pageable, hipHostMallocNonCoherent, or Portable without Mapped or Coherent) the packed data is
+ *                         produced in a device staging buffer owned by the handle and copied out.
  *   zero_threshold_for_1bit : the reference's zeroThresholdFor1Bit; ignored unless nbits == 1.
  * rows == 0 or cols == 0 is a no-op. */
 int cntkq_quantize_async(cntkq_quantizer* h, const float* in, const float* res_in, size_t rows, size_t cols,
@@ -151,8 +152,8 @@ int cntkq_wait_quantize_done(cntkq_quantizer* h);
 /* MatrixQuantizerImpl::UnquantizeAsync (Source/Math/MatrixQuantizerImpl.h:33, Source/Math/MatrixQuantizerGPU.cu:286-334).
  *   out = (add ? out : 0) + unquantize(qbuf).  qbuf_bytes must equal cntkq_qmatrix_bytes(rows, cols, nbits),
  *   else CNTKQ_LOGIC_ERROR (Source/Math/MatrixQuantizer_kernel.cu:287-289); an empty buffer is a no-op (:290-291).
- *   With qbuf_on_host != 0 the kernel reads pinned host memory where it lies; pageable memory is first copied to the
- *   handle's staging buffer. */
+ *   With qbuf_on_host != 0 the kernel reads coherent pinned memory where it lies; any other host memory is first copied
+ *   to the handle's staging buffer (see cntkq_quantize_async). */
 int cntkq_unquantize_async(cntkq_quantizer* h, const void* qbuf, size_t qbuf_bytes, int qbuf_on_host, float* out,
                            size_t rows, size_t cols, size_t nbits, int add);
 

@@ -1,6 +1,8 @@
-"""Packed matrices in host memory: pinned memory is written and read by the kernels where it lies, pageable memory goes through
+"""Packed matrices in host memory: coherent pinned memory is written and read by the kernels where it lies, any other goes through
 the handle's staging buffer. Either way the bytes are those of a packed matrix in device memory (whose parity with the oracle
 the other files check), and nothing outside the packed matrix is touched."""
+import ctypes
+
 import pytest
 import torch
 
@@ -15,6 +17,25 @@ SHAPES = [(512, 512, 1), (2048, 127, 1), (2048, 128, 1), (2048, 260, 1), (2048, 
           (8160, 40, 1), (8192, 40, 1), (1023, 130, 8), (1024, 130, 8), (1, 1, 1), (7, 5000, 4), (147, 999, 1), (20001, 9, 2),
           (110000, 3, 1), (33, 40, 32)]
 SHAPES_F64 = [(2048, 130, 1), (511, 1025, 1), (8128, 20, 1), (8192, 20, 1), (3, 700, 4), (9001, 17, 8)]
+
+
+# hipHostMalloc's flags, and whether the memory is coherent
+DEFAULT, PORTABLE, MAPPED, WRITE_COMBINED, COHERENT, NON_COHERENT = 0, 1, 2, 4, 0x40000000, 0x80000000
+KINDS = {"default": (DEFAULT, True), "mapped": (MAPPED, True), "portable_coherent": (PORTABLE | COHERENT, True), "portable": (PORTABLE, False),
+         "write_combined": (WRITE_COMBINED, False), "non_coherent": (NON_COHERENT, False), "non_coherent_mapped": (NON_COHERENT | MAPPED, False)}
+
+
+class HostMemory:
+    """A byte tensor over memory of hipHostMalloc."""
+
+    def __init__(self, size, flags):
+        self.hip, self.at = ctypes.CDLL("libamdhip64.so"), ctypes.c_void_p()
+        assert self.hip.hipHostMalloc(ctypes.byref(self.at), ctypes.c_size_t(size), ctypes.c_uint(flags)) == 0
+        self.bytes = torch.frombuffer((ctypes.c_ubyte * size).from_address(self.at.value), dtype=torch.uint8)
+
+    def free(self):
+        torch.cuda.synchronize()
+        assert self.hip.hipHostFree(self.at) == 0
 
 
 def pinned_slice(size, before):
@@ -68,3 +89,47 @@ def check(rows, cols, nbits, dtype, dedicated):
             assert torch.equal(res[k].data, res["device"].data), k
             assert torch.equal(out[k].data, out["device"].data), k
     assert bool((whole[:before] == 0x5A).all()) and bool((whole[before + size:] == 0x5A).all())
+
+
+# one shape per decoder that reads host memory: the LDS-free row-major one (256 QWords of 4 bytes, 128 of 8), the tile decoder, the
+# decoder of the matrix in device memory
+REWRITE = [(torch.float32, (8192, 40, 1)), (torch.float32, (512, 512, 1)), (torch.float32, (2048, 127, 1)), (torch.float32, (300, 64, 8)),
+           (torch.float64, (8192, 20, 1)), (torch.float64, (511, 1025, 1)), (torch.float64, (2000, 40, 1))]
+
+
+@pytest.mark.parametrize("kind", list(KINDS))
+@pytest.mark.parametrize("dtype,shape", REWRITE, ids=["%s_%dx%d_%dbit" % (("f32" if t == torch.float32 else "f64",) + s) for t, s in REWRITE])
+def test_host_rewrites_between_decodes(dtype, shape, kind):
+    """What a transport does: the packed matrix leaves, another worker's arrives in the same buffer and is decoded from there."""
+    rows, cols, nbits = shape
+    flags, coherent = KINDS[kind]
+    size = qcol_bytes(nbits, rows, dtype) * cols
+    memory = HostMemory(size, flags)
+    qz, other = MatrixQuantizerImpl.Create(0, False), MatrixQuantizerImpl.Create(0, False)
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(rows + nbits)
+    here = QuantizedMatrix(rows, cols, nbits, cntk_amd.CPUDEVICE, memory.bytes, dtype=dtype)
+    there = QuantizedMatrix(rows, cols, nbits, 0, dtype=dtype)
+    out, expected = Matrix(rows, cols, dtype=dtype), Matrix(rows, cols, dtype=dtype)
+    for step in range(3):
+        g = [Matrix(rows, cols, 0, torch.randn(rows * cols, generator=gen, device="cuda:0", dtype=dtype)) for _ in range(2)]
+        zero = Matrix(rows, cols, dtype=dtype)
+        left = Matrix(rows, cols, dtype=dtype)
+        qz.QuantizeAsync(g[0], zero, here, left, False)
+        qz.WaitQuantizeAsyncDone()
+        sent = memory.bytes.clone()
+        other.QuantizeAsync(g[0], zero, there, left, False)
+        other.WaitQuantizeAsyncDone()
+        assert torch.equal(sent, there.buffer.cpu()), ("sent", step)
+        for received in (1, 0):  # the other matrix, then the first one again
+            other.QuantizeAsync(g[received], zero, there, left, False)
+            other.UnquantizeAsync(there, expected)
+            other.WaitUnquantizeAsyncDone()
+            memory.bytes.copy_(there.buffer.cpu())
+            qz.UnquantizeAsync(here, out)
+            qz.WaitUnquantizeAsyncDone()
+            assert torch.equal(out.data, expected.data), ("decoded", step, received)
+    # coherent memory is used in place, what the host and the device may see differently is copied
+    staged = cntk_amd.lib().cntkq_debug_staging_bytes(qz._h)
+    assert staged == 0 if coherent else staged >= size
+    memory.free()
