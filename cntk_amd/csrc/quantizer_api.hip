@@ -719,7 +719,7 @@ int cntkq_create(int device_id, int use_dedicated_stream, cntkq_quantizer** out)
             return fail(CNTKQ_RUNTIME_ERROR, "cntkq_create: out of host memory");
         }
     }
-    hipEvent_t* evs[] = {&h->ev_quantize, &h->ev_fetch, &h->ev_assign, &h->ev_unquantize, &h->ev_stripe, &h->ev_main};
+    hipEvent_t* evs[] = {&h->ev_quantize, &h->ev_fetch, &h->ev_assign, &h->ev_unquantize, &h->ev_stripe, &h->ev_main, &h->ev_host_write};
     for (hipEvent_t* e : evs)
     {
         // no blocking-sync flag: waiting spins, as the reference found blocking events to stall for tens of ms
@@ -750,6 +750,7 @@ int cntkq_destroy(cntkq_quantizer* h)
     DeviceGuard guard(h->device);
     if (h->ev_quantize) (void) hipEventSynchronize(h->ev_quantize);
     if (h->ev_fetch) (void) hipEventSynchronize(h->ev_fetch);
+    if (h->ev_host_write) (void) hipEventSynchronize(h->ev_host_write);
     if (h->ev_assign) (void) hipEventSynchronize(h->ev_assign);
     if (h->ev_unquantize) (void) hipEventSynchronize(h->ev_unquantize);
     if (h->ev_stripe) (void) hipEventSynchronize(h->ev_stripe);
@@ -769,7 +770,7 @@ int cntkq_destroy(cntkq_quantizer* h)
     table_destroy(h->quantize_table64);
     table_destroy(h->unquantize_table64);
     table_destroy(h->stripe_table64);
-    hipEvent_t evs[] = {h->ev_quantize, h->ev_fetch, h->ev_assign, h->ev_unquantize, h->ev_stripe, h->ev_main};
+    hipEvent_t evs[] = {h->ev_quantize, h->ev_fetch, h->ev_assign, h->ev_unquantize, h->ev_stripe, h->ev_main, h->ev_host_write};
     for (hipEvent_t e : evs)
         if (e != nullptr)
             (void) hipEventDestroy(e);

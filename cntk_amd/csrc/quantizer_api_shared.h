@@ -178,6 +178,7 @@ struct cntkq_quantizer
     hipEvent_t ev_unquantize = nullptr;
     hipEvent_t ev_stripe = nullptr;
     hipEvent_t ev_main = nullptr;
+    hipEvent_t ev_host_write = nullptr; // set when the last kernel that writes a packed matrix in host memory has finished
     // the event each Wait call waits on: the handle's own, or one attached through the debug hook
     hipEvent_t last_quantize = nullptr;
     hipEvent_t last_unquantize = nullptr;
@@ -186,6 +187,8 @@ struct cntkq_quantizer
     hipEvent_t attach_stop = nullptr;
     bool quantize_included_fetch = false;
     bool fetch_pending = false;   // a device-to-host copy out of the staging buffer may still be running
+    bool host_write_pending = false; // such a kernel may still be running, on host_write_stream
+    hipStream_t host_write_stream = nullptr;
     bool staging_read_pending = false; // a kernel reading the staging buffer may still be running
     char* staging = nullptr;      // device buffer used when the packed matrix lives in host memory that the kernels do not take
     size_t staging_bytes = 0;
@@ -292,6 +295,16 @@ inline bool kernels_take_host_memory(const void* p, size_t bytes)
             return false;
     }
     return true;
+}
+
+// Before a kernel on `s` that writes or reads a packed matrix in host memory: what this handle wrote to host memory on another
+// stream (the caller changed the handle's main stream) comes first, as it does where the copies of the staging buffer take
+// it there and back. The event of the write that follows then covers the earlier one too.
+inline int order_after_host_write(cntkq_quantizer* h, hipStream_t s)
+{
+    if (h->host_write_pending && h->host_write_stream != s)
+        HIP_TRY(hipStreamWaitEvent(s, h->ev_host_write, 0), "hipStreamWaitEvent failed");
+    return CNTKQ_OK;
 }
 
 // Whether work issued on `s` is being recorded into a graph instead of executed.
@@ -521,22 +534,36 @@ int quantize_async_impl(cntkq_quantizer* h, const E* in, const E* res_in, size_t
             HIP_TRY(hipStreamWaitEvent(s, h->ev_fetch, 0), "hipStreamWaitEvent failed");
         qdev = h->staging;
     }
+    const bool in_place = qbuf_on_host && !staged;
+    if (in_place)
+    {
+        const int rc = order_after_host_write(h, s);
+        if (rc != CNTKQ_OK)
+            return rc;
+    }
 
     // serialised mode (Source/Math/MatrixQuantizerGPU.cu:237-240, 118-122, 137-141): the device is idle before the kernel
     // starts, and the host waits for the kernel and for the copy
     const bool force_sync = h->force_sync && !capturing;
     if (force_sync)
         HIP_TRY(hipDeviceSynchronize(), "hipDeviceSynchronize failed");
-    LaunchEvents ev = take_events(h, h->ev_quantize);
+    LaunchEvents ev = take_events(h, in_place ? h->ev_host_write : h->ev_quantize);
     if (capturing)
         ev.stop = nullptr; // recorded, not executed: nothing to wait for
     LaunchTuning tune = h->tune;
-    tune.packed_on_host = qbuf_on_host && !staged;
+    tune.packed_on_host = in_place;
     hipError_t lrc = Elem<E>::quantize(s, ev, in, res_in, res_out, qdev, rows, cols, nbits, zero_threshold_for_1bit != 0, tune);
     if (lrc == hipErrorInvalidValue)
         return fail(CNTKQ_INVALID_ARGUMENT, "quantize: the forced kernel path does not support %zu x %zu at %zu bits", rows, cols, nbits);
     HIP_TRY(lrc, "quantize kernel launch failed");
     h->last_quantize = ev.stop;
+    if (in_place)
+    {
+        h->host_write_pending = true;
+        h->host_write_stream = s;
+        if (ev.stop != h->ev_host_write) // (an event of the debug hook took its place at the dispatch)
+            HIP_TRY(hipEventRecord(h->ev_host_write, s), "hipEventRecord failed");
+    }
     if (force_sync)
         HIP_TRY(hipStreamSynchronize(s), "hipStreamSynchronize failed");
 
@@ -598,6 +625,12 @@ int unquantize_async_impl(cntkq_quantizer* h, const void* qbuf, size_t qbuf_byte
             HIP_TRY(hipStreamSynchronize(h->assign), "hipStreamSynchronize failed");
         HIP_TRY(hipStreamWaitEvent(s, h->ev_assign, 0), "hipStreamWaitEvent failed");
         qdev = h->staging;
+    }
+    else if (reached)
+    {
+        const int rc = order_after_host_write(h, s);
+        if (rc != CNTKQ_OK)
+            return rc;
     }
     LaunchEvents ev = take_events(h, h->ev_unquantize);
     if (stream_capturing(s))

@@ -133,3 +133,50 @@ def test_host_rewrites_between_decodes(dtype, shape, kind):
     staged = cntk_amd.lib().cntkq_debug_staging_bytes(qz._h)
     assert staged == 0 if coherent else staged >= size
     memory.free()
+
+
+@pytest.mark.parametrize("kind", ["default", "non_coherent"])
+def test_order_across_main_streams(kind):
+    """A handle's host-resident packed matrix is decoded after it was written, and written twice in the order of the calls, also where
+    the caller changes the handle's main stream in between without waiting."""
+    rows, cols = 2048, 300
+    size = qcol_bytes(1, rows) * cols
+    memory = HostMemory(size, KINDS[kind][0])
+    qz = MatrixQuantizerImpl.Create(0, False)
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(3)
+    g = [Matrix(rows, cols, 0, torch.randn(rows * cols, generator=gen, device="cuda:0")) for _ in range(2)]
+    zero, left = Matrix(rows, cols), Matrix(rows, cols)
+    here = QuantizedMatrix(rows, cols, 1, cntk_amd.CPUDEVICE, memory.bytes)
+    packed, expected = [], []
+    for m in g:
+        there, e = QuantizedMatrix(rows, cols, 1, 0), Matrix(rows, cols)
+        qz.QuantizeAsync(m, zero, there, left, False)
+        qz.UnquantizeAsync(there, e)
+        packed.append(there)
+        expected.append(e)
+    out = [Matrix(rows, cols), Matrix(rows, cols)]
+    left2 = Matrix(rows, cols)
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for step in range(2):
+        memory.bytes.zero_()
+        with torch.cuda.stream(first):
+            torch.cuda._sleep(20000000)  # the write starts some milliseconds after the calls below were made
+        qz.SetMainStream(first.cuda_stream)
+        qz.QuantizeAsync(g[0], zero, here, left, False)
+        qz.SetMainStream(second.cuda_stream)
+        qz.UnquantizeAsync(here, out[0])
+        qz.WaitUnquantizeAsyncDone()
+        assert torch.equal(out[0].data, expected[0].data)
+        with torch.cuda.stream(first):
+            torch.cuda._sleep(20000000)
+        qz.SetMainStream(first.cuda_stream)
+        qz.QuantizeAsync(g[0], zero, here, left, False)
+        qz.SetMainStream(second.cuda_stream)
+        qz.QuantizeAsync(g[1], zero, here, left2, False)
+        qz.UnquantizeAsync(here, out[1])
+        torch.cuda.synchronize()
+        assert torch.equal(memory.bytes, packed[1].buffer.cpu())
+        assert torch.equal(out[1].data, expected[1].data)
+    memory.free()
