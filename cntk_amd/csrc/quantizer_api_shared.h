@@ -518,8 +518,7 @@ int quantize_async_impl(cntkq_quantizer* h, const E* in, const E* res_in, size_t
     char* qdev = static_cast<char*>(qbuf);
     const bool capturing = stream_capturing(s);
     if (capturing && qbuf_on_host)
-        return fail(CNTKQ_INVALID_ARGUMENT, "cntkq_quantize_async: a host-resident packed matrix needs copies on other streams and cannot "
-                                            "be recorded into a graph");
+        return fail(CNTKQ_INVALID_ARGUMENT, "cntkq_quantize_async: a call with a host-resident packed matrix cannot be recorded into a graph");
     // Coherent pinned host memory is written by the kernel itself while it runs: the transfer needs no stream of its own, no copy after
     // the kernel and none of the events that order the two (512 x 512 at 1 bit, quantize, wait, unquantize, wait: 95 us
     // through the staging buffer, 33 us so; 2048 x 9304: 214 and 150 us).
@@ -606,8 +605,7 @@ int unquantize_async_impl(cntkq_quantizer* h, const void* qbuf, size_t qbuf_byte
     hipStream_t s = work_stream(h);
     const char* qdev = static_cast<const char*>(qbuf);
     if (qbuf_on_host && stream_capturing(s))
-        return fail(CNTKQ_INVALID_ARGUMENT, "cntkq_unquantize_async: a host-resident packed matrix needs copies on other streams and "
-                                            "cannot be recorded into a graph");
+        return fail(CNTKQ_INVALID_ARGUMENT, "cntkq_unquantize_async: a call with a host-resident packed matrix cannot be recorded into a graph");
     const bool reached = qbuf_on_host && kernels_take_host_memory(qbuf, need);
     if (qbuf_on_host && !reached)
     {

@@ -180,3 +180,24 @@ def test_order_across_main_streams(kind):
         assert torch.equal(memory.bytes, packed[1].buffer.cpu())
         assert torch.equal(out[1].data, expected[1].data)
     memory.free()
+
+
+@pytest.mark.parametrize("kind", ["default", "non_coherent"])
+def test_recorded_calls_are_refused(kind):
+    """Calls with a host-resident packed matrix are not recorded into a graph, wherever the memory is written from."""
+    rows, cols = 512, 8
+    memory = HostMemory(qcol_bytes(1, rows) * cols, KINDS[kind][0])
+    qz = MatrixQuantizerImpl.Create(0, False)
+    here = QuantizedMatrix(rows, cols, 1, cntk_amd.CPUDEVICE, memory.bytes)
+    g, res, out = Matrix(rows, cols), Matrix(rows, cols), Matrix(rows, cols)
+    word = torch.zeros(1, device="cuda:0")
+    torch.cuda.synchronize()
+    side, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    qz.SetMainStream(side.cuda_stream)
+    with torch.cuda.graph(graph, stream=side):
+        word.add_(1.0)
+        with pytest.raises(cntk_amd.QuantizerLogicError, match="host-resident packed matrix cannot be recorded"):
+            qz.QuantizeAsync(g, res, here, res, False)
+        with pytest.raises(cntk_amd.QuantizerLogicError, match="host-resident packed matrix cannot be recorded"):
+            qz.UnquantizeAsync(here, out)
+    memory.free()
