@@ -94,6 +94,27 @@ def _check_stripe_reduction(shapes, nbits, zt, k, dtype):
         assert parity.bits_equal(a1[i].to_numpy(), a2[i].to_numpy()), ("aggregate", shape)
 
 
+@pytest.mark.parametrize("nbits,k", [(1, 2), (4, 1), (8, 3)])
+def test_stripes_called_again(nbits, k):
+    """Called again a list is launched from its table, which also knows the stripes with launches of their own (too tall for the register
+    grids; the only member of the general grids), while another list, without a table, comes in between."""
+    qz = MatrixQuantizerImpl.Create(0, False)
+    shapes = [(24580, 2), (9305, 3), (64, 64), (7169, 2), (24555, 1), (14340, 2)]
+    lists = [_stripes(qz, s, nbits, False, k) for s in (shapes, shapes, [(24580, 1), (40, 3)])]
+    sets = [qz.PrepareStripeReduceBatch([(q, s, q[0], a) for q, s, a in zip(*l)]) for l in lists]
+    for _ in range(3):
+        for q, s, a in zip(*lists[0]):
+            qz.StripeReduceAsync(q, 0, s, q[0], False, agg_out=a)
+        qz.StripeReduceBatchAsync(sets[1], 0, False)
+        qz.StripeReduceBatchAsync(sets[2], 0, False)
+        torch.cuda.synchronize()
+        for i, shape in enumerate(shapes):
+            (q1, s1, a1), (q2, s2, a2) = [[part[i] for part in l] for l in lists[:2]]
+            assert np.array_equal(q1[0].to_numpy(), q2[0].to_numpy()), ("packed", shape)
+            assert parity.bits_equal(s1.to_numpy(), s2.to_numpy()), ("stripe residual", shape)
+            assert parity.bits_equal(a1.to_numpy(), a2.to_numpy()), ("aggregate", shape)
+
+
 def test_recorded_stripes_without_a_table():
     """Stripes that each had a launch of their own could always be recorded without an eager call before; they still can."""
     _check_recorded([(9305, 3), (7169, 2), (4099, 2)], 2, 2, eager_first=False)
