@@ -115,6 +115,24 @@ def test_stripes_called_again(nbits, k):
             assert parity.bits_equal(a1.to_numpy(), a2.to_numpy()), ("aggregate", shape)
 
 
+def test_stripes_with_a_forced_path():
+    """A kernel path forced on a handle is that of the stripes that are no members of the general grids, also where the list was called
+    before without it."""
+    qz = MatrixQuantizerImpl.Create(0, False)
+    shapes = [(4099, 3), (5001, 2), (6147, 4)]  # on the tile path another order of additions: other bounds
+    one, many = _stripes(qz, shapes, 4, False, 2), _stripes(qz, shapes, 4, False, 2)
+    batch = qz.PrepareStripeReduceBatch([(q, s, q[0], a) for q, s, a in zip(*many)])
+    for path in (0, 1, 0):
+        qz._set_tuning(quantize_path=path)
+        for q, s, a in zip(*one):
+            qz.StripeReduceAsync(q, 0, s, q[0], False, agg_out=a)
+        qz.StripeReduceBatchAsync(batch, 0, False)
+        torch.cuda.synchronize()
+        for i, shape in enumerate(shapes):
+            assert np.array_equal(one[0][i][0].to_numpy(), many[0][i][0].to_numpy()), ("packed", path, shape)
+            assert parity.bits_equal(one[1][i].to_numpy(), many[1][i].to_numpy()), ("stripe residual", path, shape)
+
+
 def test_recorded_stripes_without_a_table():
     """Stripes that each had a launch of their own could always be recorded without an eager call before; they still can."""
     _check_recorded([(9305, 3), (7169, 2), (4099, 2)], 2, 2, eager_first=False)
