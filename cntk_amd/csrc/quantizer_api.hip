@@ -101,7 +101,7 @@ struct BatchAbi<float>
     static bool quantize_member(const QItem& it, size_t nbits, QEntry& e, size_t& lds, uint64_t& blocks)
     {
         const int path = quantize_auto_path(it.in, it.res_in, it.res_out, it.qbuf, it.rows, nbits);
-        if (path == kPathTile && short_applicable(it.rows))
+        if (path == kPathTile && short_applicable(it.rows, it.cols, qwords_per_col(it.rows, nbits)))
         {
             e.kind = 11;
             e.s = make_short_geom(it.rows, it.cols, qwords_per_col(it.rows, nbits), qcol_bytes(nbits, it.rows), sizeof(float));
@@ -254,7 +254,7 @@ struct BatchAbi<float>
                 lds = stripe_lut_lds_bytes(e.r);
             }
         }
-        else if (short_applicable(it.rows))
+        else if (short_stripe_applicable(it.rows, it.stripe_cols, nbits, qwords_per_col(it.rows, nbits), workers))
         {
             e.kind = 11;
             e.s = make_short_geom(it.rows, it.stripe_cols, qwords_per_col(it.rows, nbits), qcol_bytes(nbits, it.rows), sizeof(float));
@@ -984,6 +984,12 @@ unsigned cntkq_debug_strip_max_strips_f64(cntkq_quantizer* h, size_t nbits, int 
         return 0;
     DeviceGuard guard(h->device);
     return strip_max_strips<double>(nbits, zero_threshold_for_1bit != 0 && nbits == 1);
+}
+
+int cntkq_debug_short_columns(size_t rows, size_t cols, size_t nbits, size_t workers)
+{
+    const size_t nq = qwords_per_col(rows, nbits);
+    return (workers == 0 ? short_applicable(rows, cols, nq) : short_stripe_applicable(rows, cols, nbits, nq, workers)) ? 1 : 0;
 }
 
 size_t cntkq_debug_staging_bytes(const cntkq_quantizer* h)

@@ -182,6 +182,11 @@ struct BatchAbi<double>
 
 extern "C" {
 
+int cntkq_debug_short_columns_f64(size_t rows, size_t cols, size_t nbits)
+{
+    return f64::short_applicable64(rows, cols, f64::qwords_per_col(rows, nbits)) ? 1 : 0;
+}
+
 size_t cntkq_qwords_per_col_f64(size_t rows, size_t nbits)
 {
     return f64::valid_nbits(nbits) ? f64::qwords_per_col(rows, nbits) : 0;

@@ -41,6 +41,10 @@ int cntkq_debug_set_strip_spin_limit(cntkq_quantizer* h, unsigned limit);
 unsigned cntkq_debug_strip_max_strips(cntkq_quantizer* h, size_t nbits, int zero_threshold_for_1bit);
 unsigned cntkq_debug_strip_max_strips_f64(cntkq_quantizer* h, size_t nbits, int zero_threshold_for_1bit);
 
+/* Whether columns of this shape are quantized (workers == 0; _f64) or reduced by one thread each. Need no device. */
+int cntkq_debug_short_columns(size_t rows, size_t cols, size_t nbits, size_t workers);
+int cntkq_debug_short_columns_f64(size_t rows, size_t cols, size_t nbits);
+
 /* Bytes of the handle's device staging buffer: 0 until a packed matrix lay in host memory that the kernels do not write and
  * read themselves. */
 size_t cntkq_debug_staging_bytes(const cntkq_quantizer* h);

@@ -135,9 +135,28 @@ inline TileGeom make_tile_geom(size_t rows, size_t cols, size_t nbits, uint32_t 
 // Columns of at most kShortMaxRows rows: one thread per column, with the tile kernels' sums (same bytes). A thread holds the column
 // in registers; the tile kernel's share of a column grows with the height meanwhile (12 x 1.37 M: 34 us against the tile kernel's
 // 80, 15 x 836000 26 against 50, 28 x 939000 62 with the tile kernel, whose bytes take 53).
-inline bool short_applicable(size_t rows)
+// A column of one QWord is coded out of registers: faster than the tile kernel whatever the number of columns (1 x 64 at 8 bits 2.3
+// against 3.0 us, 16 x 16000 at 1 bit 3.9 against 4.5). With more QWords the thread goes through its column again, value by value
+// out of LDS, and a workgroup lives from that chain's latency until the device is full: tile kernel / this, 16 rows at 4 bits
+// 0.77 at 16000 columns, 0.96 at 64000, 1.25 at 96000; 8 rows at 8 bits 0.88, 1.06, 1.33. The more QWords a column has, the less
+// even a full device hides: at 300000 columns 1.12 to 1.9 up to six QWords, 0.93 to 1.23 at seven and eight, 0.53 at 16.
+constexpr size_t kShortManyCols = 96 * 1024;
+inline bool short_applicable(size_t rows, size_t cols, size_t nq)
 {
-    return rows <= kShortMaxRows;
+    return rows <= kShortMaxRows && (nq == 1 || (cols >= kShortManyCols && nq <= 6));
+}
+
+// The same in the stripe reduction, where the thread also goes through every worker's record, QWord by QWord: up to six QWords 1.1
+// to 1.2 with one worker, but at 1.2 M columns 5 QWords 1.2 with 4 workers and 0.5 with 8, 3 QWords 1.07 with 8 (32-bit codes; two QWords
+// 1.6 or more), above eight workers not tried. Columns of one QWord are faster at any number of workers, except at 2
+// bits on a device that is not full (up to 16000 columns: 0.97 with 16 rows and 5 workers, 0.88 to 0.99 with 32 workers and more).
+inline bool short_stripe_applicable(size_t rows, size_t cols, size_t nbits, size_t nq, size_t workers)
+{
+    if (rows > kShortMaxRows)
+        return false;
+    if (nq == 1)
+        return nbits != 2 || cols >= 32 * 1024 || workers <= (rows <= 12 ? 16u : 4u);
+    return cols >= kShortManyCols && workers <= 8 && nq <= (workers <= 4 ? 5u : 3u);
 }
 
 // A workgroup takes kShortTileBytes of values, or 256 columns where those are more, or fewer columns where the device would
@@ -741,7 +760,7 @@ inline hipError_t launch_quantize(hipStream_t s, LaunchEvents ev, const float* g
     {
         if (rows > kTileMaxRows)
             return hipErrorInvalidValue;
-        if (tune.quantize_path == kPathAuto && short_applicable(rows))
+        if (tune.quantize_path == kPathAuto && short_applicable(rows, cols, qwords_per_col(rows, nbits)))
             return family_short_quantize(nbits, zt, s, ev, g, r_in, r_out, qc, make_short_geom(rows, cols, qwords_per_col(rows, nbits), qcol_bytes(nbits, rows), sizeof(float)));
         const TileGeom t = make_tile_geom(rows, cols, nbits, tune.tile_gs, tune.tile_stage, tune.tile_threads);
         return family_tile_quantize(nbits, zt, s, ev, g, r_in, r_out, qc, t);
@@ -860,7 +879,7 @@ inline hipError_t launch_stripe_reduce(hipStream_t s, LaunchEvents ev, const Str
         char* qo = static_cast<char*>(q_out);
         return family_col_stripe_unrolled(zt, rows == 1024 ? 1 : (rows == 2048 ? 2 : 4), s, ev, src, stripe_res, qo, agg_out, c, qcol);
     }
-    if (tune.quantize_path == kPathAuto && short_applicable(rows))
+    if (tune.quantize_path == kPathAuto && short_stripe_applicable(rows, cols, nbits, qwords_per_col(rows, nbits), src.workers))
         return family_short_stripe(nbits, zt, s, ev, src, stripe_res, static_cast<char*>(q_out), agg_out,
                                    make_short_geom(rows, cols, qwords_per_col(rows, nbits), qcol_bytes(nbits, rows), sizeof(float)));
     // Same tile geometry as launch_quantize would use for a matrix of this height, so that the statistics are summed in

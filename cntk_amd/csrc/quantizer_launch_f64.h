@@ -75,6 +75,14 @@ inline hipError_t dispatch_nbits64(size_t nbits, bool zt, Args... args)
     }
 }
 
+// The rule of the float side's short_applicable with twice the registers a value: one QWord up to 10 rows, with more rows where the
+// device is full (tile kernel / this at 1 to 4 bits: 10 rows 1.0 or more, 16 rows 0.82 to 0.94 up to 16000 columns, 1.2 to 1.3 at 64000); two
+// and three QWords from the same number of columns on (at 600000: 1.0 to 1.9; four 0.89 to 1.1, five 0.92 to 1.0, eight 0.75).
+inline bool short_applicable64(size_t rows, size_t cols, size_t nq)
+{
+    return rows <= kShortMaxRows && (nq == 1 ? rows <= 10 || cols >= 64 * 1024 : cols >= kShortManyCols && nq <= 3);
+}
+
 template <int NBITS, bool ZT>
 struct ShortLauncher
 {
@@ -289,7 +297,7 @@ inline hipError_t launch_quantize(hipStream_t s, LaunchEvents ev, const double* 
     {
         if (rows > kTileMaxRows)
             return hipErrorInvalidValue;
-        if (tune.quantize_path == kPathAuto && short_applicable(rows))
+        if (tune.quantize_path == kPathAuto && short_applicable64(rows, cols, qwords_per_col(rows, nbits)))
             return dispatch_nbits64<ShortLauncher>(nbits, zt, s, ev, g, r_in, r_out, qc,
                                                    make_short_geom(rows, cols, qwords_per_col(rows, nbits), qcol_bytes(nbits, rows), sizeof(double)));
         const TileGeom t = make_tile_geom(rows, cols, nbits, tune.tile_gs);

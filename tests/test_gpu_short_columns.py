@@ -14,6 +14,8 @@ PATH_TILE = 1
 F32, F64 = torch.float32, torch.float64
 # (columns: part of a workgroup, one past a whole one, several columns per thread with a remainder)
 SHAPES = [(r, c) for r in range(1, 18) for c in (1, 255, 257, 1031)] + [(1, 600001), (2, 300007), (3, 270001), (5, 262145), (8, 262143)]
+# columns of several QWords get a thread each from 98304 columns on
+MANY = [(2, 98305), (3, 98304), (4, 98303), (5, 100001), (6, 98307), (7, 98400), (9, 98561), (11, 98304), (13, 98310), (16, 98304)]
 
 
 def _make(rows, cols, dtype, gen, offset):
@@ -34,7 +36,7 @@ def test_quantize_unquantize(dtype, nbits, zt):
     tile._set_tuning(quantize_path=PATH_TILE)
     gen = torch.Generator(device="cuda:0")
     gen.manual_seed(datagen.case_seed(nbits))
-    for n, (rows, cols) in enumerate(SHAPES):
+    for n, (rows, cols) in enumerate(SHAPES + MANY):
         g, r = _make(rows, cols, dtype, gen, n % 4)
         kw = dict(dtype=dtype)
         G = Matrix(rows, cols, 0, g, **kw)
@@ -61,7 +63,7 @@ def test_stripe_reduction(nbits, zt, k):
     gen = torch.Generator(device="cuda:0")
     gen.manual_seed(datagen.case_seed(70 + nbits))
     owner = k // 2
-    shapes = [(r, c) for r in (1, 2, 3, 4, 7, 8, 9, 15, 16, 17) for c in (5, 257, 1031)]
+    shapes = [(r, c) for r in (1, 2, 3, 4, 7, 8, 9, 15, 16, 17) for c in (5, 257, 1031)] + [(2, 98305), (5, 98304), (9, 98303), (12, 98311)]
     runs = [[], [], []]
     for n, (rows, cols) in enumerate(shapes):
         packed = []

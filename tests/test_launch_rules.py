@@ -1,0 +1,50 @@
+"""Which kernel a call takes, on both sides of the lines that the rules draw. The rules are host code: no device is needed."""
+import pytest
+
+import cntk_amd
+
+
+def short(rows, cols, nbits, workers=0, double=0):
+    L = cntk_amd.lib()
+    return bool(L.cntkq_debug_short_columns_f64(rows, cols, nbits) if double else L.cntkq_debug_short_columns(rows, cols, nbits, workers))
+
+
+@pytest.mark.parametrize("nbits", [1, 2, 4, 8, 16, 32])
+def test_short_columns_of_one_qword(nbits):
+    """One thread per column whatever their number, as far as a column is one QWord."""
+    last = min(16, 32 // nbits)
+    for rows in range(1, last + 1):
+        for cols in (1, 300, 16000, 10 ** 6):
+            assert short(rows, cols, nbits)
+            for workers in (1, 4):
+                assert short(rows, cols, nbits, workers)
+    assert not short(17, 10 ** 6, nbits) and not short(17, 10 ** 6, nbits, 1)
+
+
+@pytest.mark.parametrize("rows,nbits,qwords", [(9, 4, 2), (16, 4, 2), (5, 8, 2), (16, 8, 4), (3, 16, 2), (12, 16, 6), (2, 32, 2), (6, 32, 6)])
+def test_short_columns_of_several_qwords(rows, nbits, qwords):
+    """... and with more QWords only where the columns fill the device (16 x 16000 at 8 bits: 5.2 us, the tile kernel 3.4)."""
+    for cols in (1, 300, 16000, 64000, 98303):
+        assert not short(rows, cols, nbits)
+        for workers in (1, 2, 4, 8):
+            assert not short(rows, cols, nbits, workers)
+    assert short(rows, 98304, nbits)
+    for workers in (1, 2, 4, 8, 9):
+        assert short(rows, 98304, nbits, workers) == (workers <= 8 and qwords <= (5 if workers <= 4 else 3))
+
+
+@pytest.mark.parametrize("rows,nbits", [(13, 16), (16, 16), (7, 32), (8, 32), (16, 32)])
+def test_short_columns_of_many_qwords(rows, nbits):
+    """The tile kernels keep them (16 x 300000 at 32 bits and 8 workers: nine times faster)."""
+    assert not short(rows, 10 ** 6, nbits) and not short(rows, 10 ** 6, nbits, 1) and not short(rows, 10 ** 6, nbits, 8)
+
+
+def test_short_columns_at_two_bits_and_many_workers():
+    assert short(12, 16000, 2, 16) and not short(12, 16000, 2, 17) and short(16, 16000, 2, 4) and not short(16, 16000, 2, 5)
+    assert short(16, 32768, 2, 64) and short(16, 16000, 1, 64) and short(8, 16000, 4, 64)
+
+
+def test_short_columns_of_doubles():
+    assert short(10, 5, 1, double=1) and not short(11, 65535, 1, double=1) and short(11, 65536, 1, double=1) and not short(17, 10 ** 6, 1, double=1)
+    assert not short(9, 98303, 8, double=1) and short(9, 98304, 8, double=1) and short(12, 98304, 16, double=1)
+    assert not short(13, 10 ** 6, 16, double=1) and not short(4, 10 ** 6, 64, double=1)
