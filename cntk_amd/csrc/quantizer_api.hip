@@ -986,6 +986,14 @@ unsigned cntkq_debug_strip_max_strips_f64(cntkq_quantizer* h, size_t nbits, int 
     return strip_max_strips<double>(nbits, zero_threshold_for_1bit != 0 && nbits == 1);
 }
 
+int cntkq_debug_decoder(size_t rows, size_t cols, size_t nbits, int packed_on_host)
+{
+    LaunchTuning tune;
+    tune.packed_on_host = packed_on_host != 0;
+    float* const out = reinterpret_cast<float*>(static_cast<uintptr_t>(256)); // (only its alignment is looked at)
+    return (int) plan_unquantize(out, out, rows, cols, nbits, tune).kind;
+}
+
 int cntkq_debug_short_columns(size_t rows, size_t cols, size_t nbits, size_t workers)
 {
     const size_t nq = qwords_per_col(rows, nbits);

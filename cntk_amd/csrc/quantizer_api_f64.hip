@@ -182,6 +182,14 @@ struct BatchAbi<double>
 
 extern "C" {
 
+int cntkq_debug_decoder_f64(size_t rows, size_t cols, size_t nbits, int packed_on_host)
+{
+    LaunchTuning tune;
+    tune.packed_on_host = packed_on_host != 0;
+    double* const out = reinterpret_cast<double*>(static_cast<uintptr_t>(256)); // (only its alignment is looked at)
+    return (int) f64::plan_unquantize(out, rows, cols, nbits, tune).kind;
+}
+
 int cntkq_debug_short_columns_f64(size_t rows, size_t cols, size_t nbits)
 {
     return f64::short_applicable64(rows, cols, f64::qwords_per_col(rows, nbits)) ? 1 : 0;

@@ -45,6 +45,11 @@ unsigned cntkq_debug_strip_max_strips_f64(cntkq_quantizer* h, size_t nbits, int 
 int cntkq_debug_short_columns(size_t rows, size_t cols, size_t nbits, size_t workers);
 int cntkq_debug_short_columns_f64(size_t rows, size_t cols, size_t nbits);
 
+/* The decoder (UnqKind, quantizer_kernels_batch.h) of an unquantize call on aligned matrices, the packed one in device memory or in
+ * host memory that the kernels read themselves. Need no device. */
+int cntkq_debug_decoder(size_t rows, size_t cols, size_t nbits, int packed_on_host);
+int cntkq_debug_decoder_f64(size_t rows, size_t cols, size_t nbits, int packed_on_host);
+
 /* Bytes of the handle's device staging buffer: 0 until a packed matrix lay in host memory that the kernels do not write and
  * read themselves. */
 size_t cntkq_debug_staging_bytes(const cntkq_quantizer* h);

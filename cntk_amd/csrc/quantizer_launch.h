@@ -986,6 +986,9 @@ inline UnquantizePlan plan_unquantize(const void* q, const float* out, size_t ro
     const bool host_auto = tune.packed_on_host && mode == 0 && slots_free;
     const bool host_direct = host_auto && direct_can && nq >= 256;
     const bool host_tile = host_auto && !host_direct && tile_can && (rows < kUnqRowsMinRows || cols >= 4 * 256);
+    // Columns in between, too few for the tiles: the row-major decoder with the packed column in LDS, which asks once too (up to 300
+    // QWords within 5 % of the best: 6000 x 1000 at 1 bit 72 -> 33 us, 8160 x 1023 119 -> 40, 1800 x 1023 at 4 bits 46 -> 36).
+    const bool host_rows = host_auto && !host_direct && !host_tile && !direct_auto && rows_can;
     // The LDS-free decoder for short columns, wherever it can run below 10000 rows: in a launch of its
     // own it measured 4 to 24 % faster than the tile, row-major and QWord-major decoders it replaces (512 x 100000: 38.3 ->
     // 33.7 us, 576 x 16384 at 2 bits 9.1 -> 7.0 us, 64 x 400000 at 8 bits 22.9 -> 19.4 us, 1536 x 12288 13.4 -> 12.1 us,
@@ -993,7 +996,7 @@ inline UnquantizePlan plan_unquantize(const void* q, const float* out, size_t ro
     // even at 512 x 40000 and 2304 x 4096 at 4 bits). As a member of a gradient-set launch only a large matrix (4 M elements)
     // gains (the LSTM set's decode with its 512 x 100000 and 1024 x 4096 members: 80.6 -> 69.4 us); ResNet-50's 161 members
     // and the 2048 x 1163 stripes of the all-reduce measured 5 to 7 % slower with it and keep their decoders.
-    const bool flat_auto = mode == 0 && !host_direct && !host_tile && !direct_auto && rows < 10000 && // (9304 x 2048: 14.4 -> 13.7 us; even from 10000 rows on)
+    const bool flat_auto = mode == 0 && !host_direct && !host_tile && !host_rows && !direct_auto && rows < 10000 && // (9304 x 2048: 14.4 -> 13.7 us; even from 10000 rows on)
                            (!tune.unq_member || (uint64_t) rows * cols >= ((uint64_t) 1 << 22));
     if ((mode == 6 || flat_auto) && slots_free && out16 && make_unq_flat_geom(p.flat, rows, cols, nq, qcol_bytes(nbits, rows), 4))
     {
@@ -1008,6 +1011,8 @@ inline UnquantizePlan plan_unquantize(const void* q, const float* out, size_t ro
         direct = true;
     else if (host_tile)
         tile = true;
+    else if (host_rows)
+        rowmajor = true;
     else if (mode == 0 && direct_auto)
         direct = true;
     else if (mode == 1)

@@ -536,8 +536,11 @@ inline UnquantizePlan64 plan_unquantize(const double* out, size_t rows, size_t c
     // (a packed matrix in host memory: the rule of the float side, by the bytes of a QWord)
     const bool host_auto = tune.packed_on_host && mode == 0 && tune.unq_slots == 0;
     const bool host_direct = host_auto && direct_can && nq >= 128;
-    const bool host_tile = host_auto && !host_direct && tile_can && (rows < kUnqRowsMinRows64 || cols >= 4 * 256);
-    const bool flat_auto = mode == 0 && !host_direct && !host_tile && !direct_auto && rows <= 2048 && nq % 2 == 0 &&
+    // (tiles up to the float side's height: 1500 x 1023 at 4 bits 48 us with the LDS-free decoder, 29 with tiles and with the packed
+    // column in LDS, 700 x 1023 at 2 bits 22, 18 and 23)
+    const bool host_tile = host_auto && !host_direct && tile_can && (rows < kUnqRowsMinRows || cols >= 4 * 256);
+    const bool host_rows = host_auto && !host_direct && !host_tile && !direct_auto && rows_can;
+    const bool flat_auto = mode == 0 && !host_direct && !host_tile && !host_rows && !direct_auto && rows <= 2048 && nq % 2 == 0 &&
                            (!tune.unq_member || (uint64_t) rows * cols >= ((uint64_t) 1 << 22));
     if ((mode == 6 || flat_auto) && tune.unq_slots == 0 && out16 && make_unq_flat_geom(p.flat, rows, cols, nq, qcol_bytes(nbits, rows), 2))
     {
@@ -559,7 +562,7 @@ inline UnquantizePlan64 plan_unquantize(const double* out, size_t rows, size_t c
     }
     else if ((mode == 2 && tile_can) || host_tile)
         use_tile = true;
-    else if (mode == 4 && rows_can)
+    else if ((mode == 4 && rows_can) || host_rows)
         use_rows = true;
     else if (mode == 0 && tune.unq_slots == 0 && !vec_ideal)
     {
