@@ -923,6 +923,7 @@ inline bool make_unq_flat_geom(UnqFlatGeom& t, size_t rows, size_t cols, size_t 
 constexpr size_t kUnqRowsMaxLds = 48 * 1024;
 constexpr uint32_t kUnqRowsChunk = 2048;
 constexpr size_t kUnqTileMaxRows = 16384; // 4 columns of that height: 65536 elements, small enough for the magic divisions
+constexpr size_t kUnqHostWholeBytes = 512 * 1024; // values of a column whose QWords cross the bus one thread each
 constexpr size_t kUnqTileElems = 4096;    // values per workgroup the tile decoder aims for
 constexpr size_t kUnqRowsMinRows = 1664;  // from this height on a column per workgroup (row-major decoder) beats several columns per
                                           // workgroup (tile decoder): 1152 x 8192 7.5 us against 9.8 us, 1792 x 5266 8.5 us against 7.6 us
@@ -984,11 +985,16 @@ inline UnquantizePlan plan_unquantize(const void* q, const float* out, size_t ro
     // memory: 2048 x 9304 at 1 bit 97 -> 60 us (2.46 MB, 48 us on the bus), 9304 x 2048 245 -> 55 us, 1000 x 20000
     // 106 -> 63 us, 1152 x 10378 at 8 bits 322 -> 247 us (12 MB).
     const bool host_auto = tune.packed_on_host && mode == 0 && slots_free;
-    const bool host_direct = host_auto && direct_can && nq >= 256;
-    const bool host_tile = host_auto && !host_direct && tile_can && (rows < kUnqRowsMinRows || cols >= 4 * 256);
+    // Columns of 512 KB of values and more: their chunks of the row-major decoder, several per QWord, no longer meet in one die's L2, and a line
+    // crosses the bus up to once per bit position (600000 x 6 at 1 / 4 / 8 bits 79 / 258 / 291 us, where the copy to the staging
+    // buffer took 52 / 81 / 112). A thread of the QWord-major decoder that takes all of its QWord's values asks once: 29 / 52 /
+    // 87 us; below, where the chunks do meet, it is up to 20 % slower (50000 x 300 at 1 bit 66 and 56 us).
+    const bool host_whole = host_auto && rows * 4 >= kUnqHostWholeBytes && (uint64_t) nq * cols <= 0xFFFFFFFFull;
+    const bool host_direct = host_auto && !host_whole && direct_can && nq >= 256;
+    const bool host_tile = host_auto && !host_whole && !host_direct && tile_can && (rows < kUnqRowsMinRows || cols >= 4 * 256);
     // Columns in between, too few for the tiles: the row-major decoder with the packed column in LDS, which asks once too (up to 300
     // QWords within 5 % of the best: 6000 x 1000 at 1 bit 72 -> 33 us, 8160 x 1023 119 -> 40, 1800 x 1023 at 4 bits 46 -> 36).
-    const bool host_rows = host_auto && !host_direct && !host_tile && !direct_auto && rows_can;
+    const bool host_rows = host_auto && !host_whole && !host_direct && !host_tile && !direct_auto && rows_can;
     // The LDS-free decoder for short columns, wherever it can run below 10000 rows: in a launch of its
     // own it measured 4 to 24 % faster than the tile, row-major and QWord-major decoders it replaces (512 x 100000: 38.3 ->
     // 33.7 us, 576 x 16384 at 2 bits 9.1 -> 7.0 us, 64 x 400000 at 8 bits 22.9 -> 19.4 us, 1536 x 12288 13.4 -> 12.1 us,
@@ -1007,6 +1013,8 @@ inline UnquantizePlan plan_unquantize(const void* q, const float* out, size_t ro
     }
     if (mode == 5 && direct_can)
         direct = true;
+    else if (host_whole)
+        seg_allowed = false;
     else if (host_direct)
         direct = true;
     else if (host_tile)
@@ -1128,7 +1136,7 @@ inline UnquantizePlan plan_unquantize(const void* q, const float* out, size_t ro
     t.groups = (uint32_t) ((nq + wv - 1) / wv);
     uint32_t slots = tune.unq_slots;
     if (slots == 0)
-        slots = vpw < 2 ? (uint32_t) vpw : 2;
+        slots = vpw < 2 || host_whole ? (uint32_t) vpw : 2;
     if (slots > vpw)
         slots = (uint32_t) vpw;
     t.slots = slots;

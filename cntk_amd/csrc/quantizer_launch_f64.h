@@ -535,11 +535,13 @@ inline UnquantizePlan64 plan_unquantize(const double* out, size_t rows, size_t c
     // bits were 11 % slower with it, 576 x 16384 at 1 bit 10 % faster)
     // (a packed matrix in host memory: the rule of the float side, by the bytes of a QWord)
     const bool host_auto = tune.packed_on_host && mode == 0 && tune.unq_slots == 0;
-    const bool host_direct = host_auto && direct_can && nq >= 128;
+    // (600000 x 6 at 1 / 8 bits: 81 / 477 us row-major, 57 / 117 through the staging buffer, 35 / 85 so)
+    const bool host_whole = host_auto && rows * 8 >= kUnqHostWholeBytes && (uint64_t) nq * cols <= 0xFFFFFFFFull;
+    const bool host_direct = host_auto && !host_whole && direct_can && nq >= 128;
     // (tiles up to the float side's height: 1500 x 1023 at 4 bits 48 us with the LDS-free decoder, 29 with tiles and with the packed
     // column in LDS, 700 x 1023 at 2 bits 22, 18 and 23)
-    const bool host_tile = host_auto && !host_direct && tile_can && (rows < kUnqRowsMinRows || cols >= 4 * 256);
-    const bool host_rows = host_auto && !host_direct && !host_tile && !direct_auto && rows_can;
+    const bool host_tile = host_auto && !host_whole && !host_direct && tile_can && (rows < kUnqRowsMinRows || cols >= 4 * 256);
+    const bool host_rows = host_auto && !host_whole && !host_direct && !host_tile && !direct_auto && rows_can;
     const bool flat_auto = mode == 0 && !host_direct && !host_tile && !host_rows && !direct_auto && rows <= 2048 && nq % 2 == 0 &&
                            (!tune.unq_member || (uint64_t) rows * cols >= ((uint64_t) 1 << 22));
     if ((mode == 6 || flat_auto) && tune.unq_slots == 0 && out16 && make_unq_flat_geom(p.flat, rows, cols, nq, qcol_bytes(nbits, rows), 2))
@@ -550,7 +552,7 @@ inline UnquantizePlan64 plan_unquantize(const double* out, size_t rows, size_t c
         return p;
     }
     bool use_rows = false, use_tile = false;
-    if ((mode == 5 && direct_can) || host_direct || (mode == 0 && !host_tile && direct_auto))
+    if ((mode == 5 && direct_can) || host_direct || (mode == 0 && !host_whole && !host_tile && direct_auto))
     {
         if (make_unq_direct_geom(p.rowg, rows, cols, nq, qcol_bytes(nbits, rows), 2))
         {
@@ -564,7 +566,7 @@ inline UnquantizePlan64 plan_unquantize(const double* out, size_t rows, size_t c
         use_tile = true;
     else if ((mode == 4 && rows_can) || host_rows)
         use_rows = true;
-    else if (mode == 0 && tune.unq_slots == 0 && !vec_ideal)
+    else if (mode == 0 && tune.unq_slots == 0 && !vec_ideal && !host_whole)
     {
         if (rows_can && rows >= kUnqRowsMinRows64)
             use_rows = true;
@@ -621,7 +623,7 @@ inline UnquantizePlan64 plan_unquantize(const double* out, size_t rows, size_t c
             return p;
         }
     }
-    const bool vec = mode != 1 && (nq % 2 == 0) && (rows % 2 == 0) && out16;
+    const bool vec = mode != 1 && !host_whole && (nq % 2 == 0) && (rows % 2 == 0) && out16;
     const uint32_t wv = vec ? 2 : 1;
     UnqGeom& t = p.qw;
     t.rows = (uint32_t) rows;
@@ -630,7 +632,7 @@ inline UnquantizePlan64 plan_unquantize(const double* out, size_t rows, size_t c
     t.groups = (uint32_t) ((nq + wv - 1) / wv);
     uint32_t slots = tune.unq_slots;
     if (slots == 0)
-        slots = vpw < 4 ? (uint32_t) vpw : 4;
+        slots = vpw < 4 || host_whole ? (uint32_t) vpw : 4;
     if (slots > vpw)
         slots = (uint32_t) vpw;
     t.slots = slots;

@@ -15,8 +15,8 @@ pytestmark = pytest.mark.gpu
 # 260), tile decoder against row-major one (1023 / 1024 columns from 1664 rows on), short columns, one column, strips
 SHAPES = [(512, 512, 1), (2048, 127, 1), (2048, 128, 1), (2048, 260, 1), (2048, 1025, 1), (2049, 129, 2), (1664, 1023, 1),
           (8160, 40, 1), (8192, 40, 1), (1023, 130, 8), (1024, 130, 8), (1, 1, 1), (7, 5000, 4), (147, 999, 1), (20001, 9, 2),
-          (110000, 3, 1), (33, 40, 32)]
-SHAPES_F64 = [(2048, 130, 1), (511, 1025, 1), (8128, 20, 1), (8192, 20, 1), (3, 700, 4), (9001, 17, 8)]
+          (110000, 3, 1), (33, 40, 32), (131071, 3, 4), (131072, 2, 1), (200003, 3, 8), (131075, 2, 32), (6000, 70, 1), (1800, 33, 4)]
+SHAPES_F64 = [(2048, 130, 1), (511, 1025, 1), (8128, 20, 1), (8192, 20, 1), (3, 700, 4), (9001, 17, 8), (65537, 3, 1), (100003, 2, 8), (65536, 2, 64), (1500, 40, 4), (3000, 50, 2)]
 
 
 # hipHostMalloc's flags, and whether the memory is coherent

@@ -61,14 +61,16 @@ def decoder(rows, cols, nbits, host=0, double=0):
 
 @pytest.mark.parametrize("rows,cols,nbits,kind", [
     (1663, 40, 1, TILE), (1664, 1024, 1, TILE), (1664, 1023, 1, ROWS), (6000, 1000, 1, ROWS), (8160, 1023, 1, ROWS), (8160, 1024, 1, TILE),
-    (8161, 1023, 1, DIRECT), (3072, 100, 1, ROWS), (2048, 100, 1, DIRECT), (1800, 1023, 4, ROWS), (2304, 1023, 4, DIRECT), (1, 40, 1, TILE)])
+    (8161, 1023, 1, DIRECT), (3072, 100, 1, ROWS), (2048, 100, 1, DIRECT), (1800, 1023, 4, ROWS), (2304, 1023, 4, DIRECT), (1, 40, 1, TILE),
+    (131071, 9, 8, DIRECT), (131072, 9, 8, SCALAR), (600000, 6, 1, SCALAR), (131072, 5000, 1, SCALAR)])
 def test_decoder_out_of_host_memory(rows, cols, nbits, kind):
-    """Every line crosses the bus once (6000 x 1000 at 1 bit took 72 us with the decoder of device memory, 33 with the column in LDS)."""
+    """Every line crosses the bus once (6000 x 1000 at 1 bit took 72 us with the decoder of device memory, 33 with the column in LDS; 600000 x 6 at 8 bits 291 us
+    row-major, 87 with a thread per QWord)."""
     assert decoder(rows, cols, nbits, host=1) == kind
 
 
 @pytest.mark.parametrize("rows,cols,nbits,kind", [
     (1500, 1023, 4, TILE), (1663, 40, 1, TILE), (1666, 1023, 4, ROWS), (1666, 1024, 4, TILE), (3000, 600, 2, ROWS), (8160, 500, 1, DIRECT),
-    (7000, 500, 1, ROWS)])
+    (7000, 500, 1, ROWS), (65535, 9, 8, DIRECT), (65536, 9, 8, SCALAR), (600000, 6, 1, SCALAR)])
 def test_decoder_of_doubles_out_of_host_memory(rows, cols, nbits, kind):
     assert decoder(rows, cols, nbits, host=1, double=1) == kind
