@@ -947,6 +947,15 @@ inline bool make_unq_direct_geom(UnqRowGeom& t, size_t rows, size_t cols, size_t
     return true;
 }
 
+// Matrices of one row in device memory: every thread of the QWord-major decoder stores one value or two and most of a QWord is padding,
+// but the tile decoder (its LDS within an eighth of a compute unit, see below) has two barriers and an empty device until columns are
+// many. QWord-major / tile, us: 1 bit 2.7 / 3.7 at 32000 columns, 5.4 / 3.7 at 128000; 2 bits 7.2 / 7.3 at 300000; 4 bits 6.7 / 8.5 at
+// 600000, 11.7 / 9.3 at 1.2 M; 8 bits 44 / 46 at 10 M, 109 / 88 at 20 M; 16 and 32 bits 66 / 88 and 65 / 83 at 20 M.
+inline bool one_row_tiles(size_t cols, size_t nbits)
+{
+    return nbits <= 8 && cols >= (nbits == 1 ? 96000u : nbits == 2 ? 400000u : nbits == 4 ? 1000000u : 12000000u);
+}
+
 inline UnquantizePlan plan_unquantize(const void* q, const float* out, size_t rows, size_t cols, size_t nbits,
                                       const LaunchTuning& tune)
 {
@@ -1039,7 +1048,7 @@ inline UnquantizePlan plan_unquantize(const void* q, const float* out, size_t ro
         vec = true;
     else if (rows_can && rows >= kUnqRowsMinRows)
         rowmajor = true; // a column fills a workgroup
-    else if (tile_can)
+    else if (tile_can && (rows > 1 || one_row_tiles(cols, nbits)))
         tile = true;
     else if (rows_can)
         rowmajor = true;

@@ -504,6 +504,14 @@ struct UnquantizePlan64
     bool ok = false;
 };
 
+// The rule of the float side's one_row_tiles (QWord-major / tile, us: 1 bit 2.8 / 2.9 at 32000 columns, 3.8 / 3.1 at 64000; 2 bits 4.8 /
+// 4.7 at 128000; 4 bits 4.8 / 5.6 at 300000, 7.7 / 6.3 at 600000; 8 bits 27 / 31 at 5 M, 66 / 59 at 10 M; 16 and 32 bits 110 / 115 at 20 M,
+// 64 bits 55 / 57 at 10 M).
+inline bool one_row_tiles64(size_t cols, size_t nbits)
+{
+    return nbits <= 8 && cols >= (nbits == 1 ? 48000u : nbits == 2 ? 128000u : nbits == 4 ? 500000u : 8000000u);
+}
+
 inline UnquantizePlan64 plan_unquantize(const double* out, size_t rows, size_t cols, size_t nbits, const LaunchTuning& tune)
 {
     UnquantizePlan64 p;
@@ -570,7 +578,7 @@ inline UnquantizePlan64 plan_unquantize(const double* out, size_t rows, size_t c
     {
         if (rows_can && rows >= kUnqRowsMinRows64)
             use_rows = true;
-        else if (tile_can)
+        else if (tile_can && (rows > 1 || one_row_tiles64(cols, nbits)))
             use_tile = true;
         else if (rows_can)
             use_rows = true;
