@@ -217,9 +217,16 @@ __device__ __forceinline__ void stripe_reduce_batch_body(const StripeBatchEntry*
 }
 
 // The stripes of a single worker: columns of up to six pieces per thread as quantize_reg_body has them (kinds 12 / 13: up to 3 / 6
-// pieces; r), the rest as above.
+// pieces; r), the rest as above. At 1 bit (a level picked by a bit) six pieces fit 64 registers; a code's decoding takes two more, and
+// a wavefront less is cheaper than 20 bytes of scratch (eight wavefronts / seven, us: stripes of 2049 to 6144 rows at 8 bits 32.6 / 31.3,
+// ResNet-50 at 2 bits 55.9 / 53.8, at 8 bits 58.9 / 58.4; up to 3072 rows, where the scratch is not touched, at 8 bits 18.7 / 19.0).
+constexpr int stripe_one_batch_waves(int nbits)
+{
+    return nbits == 1 || nbits == 32 ? 8 : 7;
+}
+
 template <int NBITS, bool ZT>
-__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(8, 8))) CNTKQ_SGPRS_FOR_8_WAVES void stripe_one_batch_kernel(const StripeBatchEntry* __restrict__ entries,
+__global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(stripe_one_batch_waves(NBITS), stripe_one_batch_waves(NBITS)))) CNTKQ_SGPRS_FOR_8_WAVES void stripe_one_batch_kernel(const StripeBatchEntry* __restrict__ entries,
                                                                                                 const uint32_t* __restrict__ begins, uint32_t count)
 {
     extern __shared__ f32x4 smem_v4[];
@@ -301,11 +308,12 @@ stripe_reduce_reg_batch_kernel(const StripeBatchEntry* __restrict__ entries, con
         stripe_reduce_reg_member<NBITS, ZT, T, P[2]>(en, c, column, smem_v4);
 }
 
-// ... of a single worker
+// ... of a single worker (WIDE: fifteen pieces take seven registers more than four wavefronts per SIMD leave; three without scratch
+// memory against four with it: stripes of 8200 to 14336 rows at 1 / 8 bits 17.6 / 19.1 -> 17.0 / 17.2 us)
 template <int T, bool WIDE>
 constexpr int stripe_one_reg_batch_waves()
 {
-    return T == 1024 ? 8 : (WIDE ? 4 : 6);
+    return T == 1024 ? 8 : (WIDE ? 3 : 6);
 }
 
 template <int NBITS, bool ZT, int T, bool WIDE>

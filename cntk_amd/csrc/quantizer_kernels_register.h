@@ -602,7 +602,7 @@ __device__ __forceinline__ void stripe_one_reg_body(const char* q_in, float* str
             return unquantize_value<NBITS>(uf, lo, (word >> (k * PS::SHIFT)) & PS::CODEMASK);
     };
     float* ag = agg_out != nullptr ? agg_out + base : nullptr;
-    // (pieces whose QWords are in flight together: three or four measured the same and spill)
+    // (pieces whose QWords are in flight together: three or four measured the same and take more registers)
     constexpr int B = 2;
     const float inv_nq = small_divisor(c.nq); // (element numbers are far below the 2^20 that small_div takes)
 #pragma unroll

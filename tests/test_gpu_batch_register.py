@@ -94,6 +94,29 @@ def _check_stripe_reduction(shapes, nbits, zt, k, dtype):
         assert parity.bits_equal(a1[i].to_numpy(), a2[i].to_numpy()), ("aggregate", shape)
 
 
+# a single worker's stripes: tiles and short columns, whole pieces up to 3 / 6 per thread on both sides of each line (with and without a line
+# shift), the register grids, slices that start anywhere within 16 bytes
+SINGLE = [(16, 300), (300, 31), (512, 65), (1024, 40), (1028, 9), (2048, 33), (2052, 8), (3044, 9), (3068, 5), (3072, 9), (3076, 7), (4608, 11),
+          (6116, 4), (6140, 3), (6144, 6), (6148, 70), (2049, 4), (2051, 6), (7166, 3), (9305, 2), (14336, 40), (16384, 2)]
+
+
+@pytest.mark.parametrize("nbits,zt", [(1, False), (1, True), (2, False), (4, False), (8, False), (16, False), (32, False)])
+def test_single_worker_stripes(nbits, zt):
+    qz = MatrixQuantizerImpl.Create(0, False)
+    shapes = [s for s in SINGLE if nbits < 32 or s[0] <= 14336]  # (32-bit codes: no stripes above)
+    one, many = _stripes(qz, shapes, nbits, zt, 1), _stripes(qz, shapes, nbits, zt, 1)
+    batch = qz.PrepareStripeReduceBatch([(q, s, q[0], a) for q, s, a in zip(*many)])
+    for step in range(3):
+        for q, s, a in zip(*one):
+            qz.StripeReduceAsync(q, 0, s, q[0], zt, agg_out=a)
+        qz.StripeReduceBatchAsync(batch, 0, zt)
+        torch.cuda.synchronize()
+        for i, shape in enumerate(shapes):
+            assert np.array_equal(one[0][i][0].to_numpy(), many[0][i][0].to_numpy()), ("packed", shape, step)
+            assert parity.bits_equal(one[1][i].to_numpy(), many[1][i].to_numpy()), ("stripe residual", shape, step)
+            assert parity.bits_equal(one[2][i].to_numpy(), many[2][i].to_numpy()), ("aggregate", shape, step)
+
+
 @pytest.mark.parametrize("nbits,k", [(1, 2), (4, 1), (8, 3)])
 def test_stripes_called_again(nbits, k):
     """Called again a list is launched from its table, which also knows the stripes with launches of their own (too tall for the register
