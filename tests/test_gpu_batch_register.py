@@ -38,6 +38,13 @@ def test_quantize(shapes, nbits, zt):
     _check_quantize(shapes, nbits, zt, torch.float32)
 
 
+@pytest.mark.parametrize("nbits", [1, 8])
+def test_quantize_of_few_tall_columns_alone(nbits):
+    """A large set made of nothing but the few tall columns that would be staged in memory: there is nothing else to hide them, so they
+    share a register grid (64 x 14336 x 32 at 1 bit: 108 us staged, 65 us so)."""
+    _check_quantize([(14336, 32)] * 55 + [(13312, 31)] * 4, nbits, False, torch.float32)
+
+
 @pytest.mark.parametrize("nbits,zt", [(1, False), (1, True), (4, False), (32, False)])
 def test_quantize_doubles(nbits, zt):
     _check_quantize(DOUBLE, nbits, zt, torch.float64)
