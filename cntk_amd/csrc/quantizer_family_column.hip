@@ -65,12 +65,20 @@ struct StripeColLauncher
     }
 };
 
+template <bool ZT, int PER, bool RUNS>
+inline void launch_quantize_col_dealt(hipStream_t s, LaunchEvents ev, const float* g, const float* r_in, float* r_out, char* q, uint32_t cols,
+                                      uint64_t qcol)
+{
+    hipExtLaunchKernelGGL((quantize_col_kernel<ZT, PER, RUNS>), dim3(cols), dim3(kColThreads), col_lds_bytes<PER>(), s, ev.start, ev.stop, 0, g,
+                          r_in, r_out, q, qcol);
+}
+
 template <bool ZT, int PER>
 inline void launch_quantize_col(hipStream_t s, LaunchEvents ev, const float* g, const float* r_in, float* r_out, char* q, uint32_t cols,
                                 uint64_t qcol, bool runs)
 {
-    hipExtLaunchKernelGGL((quantize_col_kernel<ZT, PER>), dim3(cols), dim3(kColThreads), col_lds_bytes<PER>(), s, ev.start, ev.stop, 0, g,
-                          r_in, r_out, q, qcol, runs ? 1u : 0u);
+    runs ? launch_quantize_col_dealt<ZT, PER, true>(s, ev, g, r_in, r_out, q, cols, qcol)
+         : launch_quantize_col_dealt<ZT, PER, false>(s, ev, g, r_in, r_out, q, cols, qcol);
 }
 
 template <bool ZT, int PER>

@@ -9,6 +9,13 @@ template <int NBITS, bool ZT, int T, int PER>
 inline hipError_t launch_reg_one(hipStream_t s, LaunchEvents ev, const float* g, const float* r_in, float* r_out, char* q, uint32_t cols,
                                  const RegGeom& c)
 {
+    if constexpr (T == 256 && PER <= kRegRunsPer)
+        if (c.runs != 0)
+        {
+            hipExtLaunchKernelGGL((quantize_reg_kernel<NBITS, ZT, T, PER, false, true>), dim3(cols), dim3(T), reg_lds_bytes(c), s, ev.start, ev.stop, 0, g, r_in,
+                                  r_out, q, c);
+            return hipGetLastError();
+        }
     hipExtLaunchKernelGGL((quantize_reg_kernel<NBITS, ZT, T, PER>), dim3(cols), dim3(T), reg_lds_bytes(c), s, ev.start, ev.stop, 0, g, r_in,
                           r_out, q, c);
     return hipGetLastError();

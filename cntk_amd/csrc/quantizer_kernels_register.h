@@ -14,6 +14,12 @@ namespace cntkq {
 // number of resident workgroups no longer falls with the column height. Statistics are summed in the piece order of
 // the LDS kernels above, so with T = 256 the bytes are theirs.
 
+// Up to this many pieces per thread, on 256 threads, the register kernels have a variant that deals columns in runs for packed matrices in
+// host memory (c.runs; the choice at run time in one kernel cost every small matrix in device memory 0.1 us). With taller columns a
+// record is several lines and there is nothing in it: 2049 x 9304 at 1 bit 86 -> 74 us, 1152 x 10378 68 -> 62, at 8 bits 249 -> 244,
+// 3000 x 3000 at 2 bits 68 -> 67; 4608 x 2000 at 4 bits, 6000 x 1000 and 9304 x 2048 at 1 bit the same either way.
+constexpr int kRegRunsPer = 3;
+
 struct RegGeom
 {
     uint32_t rows;   // multiple of 4, at most 4 * T * PER
@@ -283,12 +289,13 @@ __device__ __forceinline__ void quantize_reg_body(const float* __restrict__ g, c
     reg_stats_pack<NBITS, ZT, T, PER>(a, edge, has_edge, edge_at, head, pieces, shift, c, red, red_u, words, r_out + base, qc);
 }
 
-template <int NBITS, bool ZT, int T, int PER, bool EDGE = false>
+// RUNS: columns are dealt by column_of_workgroup, where packed records are short (see kRegRunsPer)
+template <int NBITS, bool ZT, int T, int PER, bool EDGE = false, bool RUNS = false>
 __global__ __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(reg_waves<T, PER>(), reg_waves<T, PER>()))) void quantize_reg_kernel(
     const float* __restrict__ g, const float* r_in, float* r_out, char* __restrict__ q, RegGeom c)
 {
     extern __shared__ f32x4 smem_v4[];
-    quantize_reg_body<NBITS, ZT, T, PER, EDGE>(g, r_in, r_out, q, c, c.runs != 0 ? column_of_workgroup(blockIdx.x, gridDim.x) : blockIdx.x, smem_v4);
+    quantize_reg_body<NBITS, ZT, T, PER, EDGE>(g, r_in, r_out, q, c, RUNS ? column_of_workgroup(blockIdx.x, gridDim.x) : blockIdx.x, smem_v4);
 }
 
 // Stripe reduction for tall columns (above the LDS kernels' 14336 rows), in the register kernel's shape: 1024 threads per
