@@ -203,9 +203,9 @@ struct BatchAbi<float>
         DeviceGuard guard(h->device);
         return cntkq::stripe_takes_strips(work_stream(h), rows, cols, nbits, zt, h->tune);
     }
-    // taller stripes run 1024 threads per column, or on strips: a launch of their own
-    // (so do stripes that the table-driven register kernel takes with more than six pieces per thread: the shared launch is
-    // compiled for what its largest member needs)
+    // Whether a stripe can be a member of the general grids. Taller stripes (1024 threads per column, edge elements) and those that the
+    // table-driven register kernel takes with more than six pieces per thread cannot: the grid is compiled for what its largest
+    // member needs. They are members of the register grids (stripe_register_member), or have a launch of their own (strips).
     static bool stripe_is_member(const SItem& it, size_t workers, size_t nbits)
     {
         if (stripe_uses_reg(it.rows, it.stripe_res, nbits))
@@ -408,9 +408,10 @@ __global__ __launch_bounds__(256) void table_store_kernel(TableChunk chunk, uint
 
 // ---- the gradient-set quantize that allocates nothing -----------------------------------------------------------------
 //
-// Same planning, same kernels and hence the same bytes as quantize_batch_impl<float>; what differs is where the argument
-// table lives (the fixed device array `scratch`, reached through the per-device pointer) and how it gets there (as kernel
-// arguments of table_store_kernel). Nothing on this path calls an allocator: no hipMalloc / hipHostMalloc / hipFree, no
+// The bytes of quantize_batch_impl<float>, with its general grids (small / large LDS need) and their members' kernels; there are no
+// register grids here and LDS classes are not merged, so columns in registers on 1024 threads or with edge elements have a launch per
+// matrix and few tall columns stay staged in memory. What differs besides is where the argument table lives (the fixed device array
+// `scratch`, reached through the per-device pointer) and how it gets there (as kernel arguments of table_store_kernel). Nothing on this path calls an allocator: no hipMalloc / hipHostMalloc / hipFree, no
 // host heap (the plan is built in the handle's NoAllocState), no copy that would need staging memory.
 int quantize_batch_noalloc_impl(cntkq_quantizer* h, const cntkq_quantize_item* items, size_t count, size_t nbits, int zero_threshold_for_1bit)
 {

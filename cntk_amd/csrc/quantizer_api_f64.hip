@@ -54,8 +54,8 @@ struct BatchAbi<double>
     static BatchTable& unquantize_table(cntkq_quantizer* h) { return h->unquantize_table64; }
     static BatchTable& stripe_table(cntkq_quantizer* h) { return h->stripe_table64; }
 
-    // members are runs of column tiles; the register and tall kernels' matrices get launches of their own, except small
-    // matrices of the element-wise register kernel, which stay members and run the tile body (the same bytes)
+    // members of the general grid are runs of column tiles, small matrices of the element-wise register kernel among them, which run the
+    // tile body (the same bytes); columns on 1024 threads are members of the register grid below, the rest gets launches of its own
     static bool quantize_member(const QItem& it, size_t nbits, QEntry& e, size_t& lds, uint64_t& blocks)
     {
         const int path = f64::quantize_auto_path(it.in, it.res_in, it.res_out, it.rows, nbits);
@@ -134,7 +134,8 @@ struct BatchAbi<double>
         DeviceGuard guard(h->device);
         return f64::stripe_takes_strips(work_stream(h), rows, cols, nbits, zt, h->tune);
     }
-    // stripes of the register kernel's heights run 1024 threads per column, taller ones on strips: a launch of their own
+    // stripes of the register kernel's heights are members of the register grid (stripe_register_member), taller ones run on strips: a
+    // launch of their own
     static bool stripe_is_member(const SItem& it, size_t, size_t nbits)
     {
         return it.rows <= f64::stripe_reduce_max_rows(nbits) && !f64::stripe_uses_reg(it.rows, nbits);

@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 # (rows, columns, bits): what decides the kernels -- 255 / 256 QWords per column, columns in runs of 16 x 8 (127 / 128 / 129 /
 # 260), tile decoder against row-major one (1023 / 1024 columns from 1664 rows on), short columns, one column, strips
 SHAPES = [(512, 512, 1), (2048, 127, 1), (2048, 128, 1), (2048, 260, 1), (2048, 1025, 1), (2049, 129, 2), (1664, 1023, 1),
-          (8160, 40, 1), (8192, 40, 1), (1023, 130, 8), (1024, 130, 8), (1, 1, 1), (7, 5000, 4), (147, 999, 1), (20001, 9, 2),
+          (8160, 40, 1), (8192, 40, 1), (1023, 130, 8), (1024, 130, 8), (1, 1, 1), (7, 5000, 4), (16, 300, 1), (16, 98305, 4), (3, 98304, 16), (147, 999, 1), (20001, 9, 2),
           (110000, 3, 1), (33, 40, 32), (131071, 3, 4), (131072, 2, 1), (200003, 3, 8), (131075, 2, 32), (6000, 70, 1), (1800, 33, 4)]
 SHAPES_F64 = [(2048, 130, 1), (511, 1025, 1), (8128, 20, 1), (8192, 20, 1), (3, 700, 4), (9001, 17, 8), (65537, 3, 1), (100003, 2, 8), (65536, 2, 64), (1500, 40, 4), (3000, 50, 2)]
 
@@ -50,12 +50,18 @@ def test_float(shape, dedicated):
     check(*shape, torch.float32, dedicated)
 
 
+@pytest.mark.parametrize("shape", SHAPES, ids=["%dx%d_%dbit" % s for s in SHAPES])
+def test_float_at_four_bytes(shape):
+    """The packed matrix at the alignment of a value and no better, as a transport's message may have it."""
+    check(*shape, torch.float32, False, before=4 * 27)
+
+
 @pytest.mark.parametrize("shape", SHAPES_F64, ids=["%dx%d_%dbit" % s for s in SHAPES_F64])
 def test_double(shape):
     check(*shape, torch.float64, False)
 
 
-def check(rows, cols, nbits, dtype, dedicated):
+def check(rows, cols, nbits, dtype, dedicated, before=8 * 13):
     qz = MatrixQuantizerImpl.Create(0, dedicated)
     gen = torch.Generator(device="cuda:0")
     gen.manual_seed(rows * 131 + cols)
@@ -63,7 +69,6 @@ def check(rows, cols, nbits, dtype, dedicated):
     n = rows * cols
     g = torch.randn(n, generator=gen, device="cuda:0", dtype=dtype)
     G = Matrix(rows, cols, 0, g)
-    before = 8 * 13
     pinned, whole = pinned_slice(size, before)
     pageable = torch.zeros(size, dtype=torch.uint8)
     places = {"device": QuantizedMatrix(rows, cols, nbits, 0, dtype=dtype),

@@ -6,7 +6,7 @@ import torch
 
 import datagen
 import parity
-from cntk_amd import Matrix, MatrixQuantizerImpl, QuantizedMatrix
+from cntk_amd import Matrix, MatrixQuantizerImpl, QuantizedMatrix, qcol_bytes
 
 pytestmark = pytest.mark.gpu
 
@@ -86,3 +86,49 @@ def test_stripe_reduction(nbits, zt, k):
             assert np.array_equal(runs[0][i][2].to_numpy(), run[i][2].to_numpy()), ("packed", shape)
             assert parity.bits_equal(runs[0][i][1].to_numpy(), run[i][1].to_numpy()), ("stripe residual", shape)
             assert parity.bits_equal(runs[0][i][3].to_numpy(), run[i][3].to_numpy()), ("aggregate", shape)
+
+
+def _same(a, b):
+    """Equal, or both not a number."""
+    return torch.equal(torch.where(a.isnan(), torch.zeros_like(a), a), torch.where(b.isnan(), torch.zeros_like(b), b)) and torch.equal(a.isnan(), b.isnan())
+
+
+@pytest.mark.parametrize("dtype,nbits,zt", [(F32, 1, False), (F32, 1, True), (F32, 2, False), (F32, 4, False), (F32, 8, False), (F32, 32, False),
+                                            (F64, 1, False), (F64, 8, False), (F64, 64, False)])
+def test_special_values_and_offsets(dtype, nbits, zt):
+    """NaN, infinities, zeros of both signs and tiny values, one kind per column; gradient and residuals each at an offset of their
+    own within 16 bytes; the packed matrix at the alignment of a value. What the tile kernels give."""
+    plain, tile = MatrixQuantizerImpl.Create(0, False), MatrixQuantizerImpl.Create(0, False)
+    tile._set_tuning(quantize_path=PATH_TILE)
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(datagen.case_seed(900 + nbits))
+    tiny = torch.finfo(dtype).tiny
+    kinds = [float("nan"), float("inf"), -float("inf"), 0.0, -0.0, tiny, tiny / 4, torch.finfo(dtype).max]
+    word, size = (torch.int64, 8) if dtype == F64 else (torch.int32, 4)
+    for n, (rows, cols) in enumerate([(r, 300) for r in range(1, 17)] + [(3, 98400), (5, 98305), (12, 98304)]):
+        def at(offset, fill=None):
+            v = torch.empty(rows * cols + 4, dtype=dtype, device="cuda:0")[offset:offset + rows * cols]
+            return v.normal_(generator=gen) if fill is None else v.copy_(fill)
+
+        g, r = at(n % 4), at((n + 1) % 4)
+        for k, x in enumerate(kinds):
+            g[(20 + k) * rows:(21 + k) * rows] = x  # whole columns ...
+            r[(20 + k) * rows:(21 + k) * rows] = 0.0
+            g[(40 + k) * rows + k % rows] = x       # ... and one value of a column
+            r[(60 + k) * rows + k % rows] = x
+        runs = []
+        for qz in (plain, tile):
+            out = at((n + 2) % 4, r)
+            buffer = torch.empty(qcol_bytes(nbits, rows, dtype) * cols + 8, dtype=torch.uint8, device="cuda:0")[size % 8:]
+            q = QuantizedMatrix(rows, cols, nbits, 0, buffer[:qcol_bytes(nbits, rows, dtype) * cols], dtype=dtype)
+            qz.QuantizeAsync(Matrix(rows, cols, 0, g), Matrix(rows, cols, 0, r), q, Matrix(rows, cols, 0, out), zt)
+            runs.append((q, out))
+        torch.cuda.synchronize()
+        (q1, o1), (q2, o2) = runs
+        v1, v2 = [q.buffer.clone().view(dtype).view(cols, -1) for q in (q1, q2)]
+        assert _same(v1[:, :2], v2[:, :2]), ("bounds", rows, cols)
+        if nbits != size * 8:
+            assert torch.equal(v1.contiguous().view(word)[:, 2:], v2.contiguous().view(word)[:, 2:]), ("words", rows, cols)
+        else:  # the codes are the values themselves
+            assert _same(v1[:, 2:], v2[:, 2:]), ("values", rows, cols)
+        assert _same(o1, o2), ("residual", rows, cols)
