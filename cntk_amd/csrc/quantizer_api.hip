@@ -285,8 +285,12 @@ struct BatchAbi<float>
                 line_shift = false;
             threads = it.rows > kTileMaxRows ? 1024u : reg_edge_threads(it.rows);
         }
+        // Whole pieces, more than six per thread, at 2 bits and more: with several workers the general grid's column kernel, which decodes
+        // them out of LDS side by side and leaves room for more workgroups, is the faster one (general / register grid: 9304 x 14 at 8
+        // bits 24 / 27 us with 4 workers, 25 / 35 with 8; 14336 x 14 28 / 36 and 29 / 54; with 2 workers 9304 x 3000 at 4 bits
+        // 68 / 77, 14336 x 400 26 / 30). A single worker's stripes are (9304 x 14 at 8 bits 1.35 times as fast, 14336 x 3000 1.3).
         else if (!stripe_auto_col(it.rows, it.stripe_res) || stripe_lookup_per(it.rows, line_shift) <= 6 ||
-                 (nbits == 1 ? !stripe_looks_up(it.rows, nbits, workers) : workers > 2 && it.stripe_cols > 64))
+                 (nbits == 1 ? !stripe_looks_up(it.rows, nbits, workers) : workers > 1))
             return kBatchOwnLaunch; // (a member of the general grids)
         const RegGeom r = make_reg_geom(it.rows, nbits, threads, line_shift);
         e.kind = register_kind((r.pieces + (r.line_shift ? 7u : 0u) + threads - 1) / threads, threads);
@@ -985,6 +989,24 @@ unsigned cntkq_debug_strip_max_strips_f64(cntkq_quantizer* h, size_t nbits, int 
         return 0;
     DeviceGuard guard(h->device);
     return strip_max_strips<double>(nbits, zero_threshold_for_1bit != 0 && nbits == 1);
+}
+
+int cntkq_debug_stripe_shares_register_grid(size_t rows, size_t cols, size_t nbits, size_t workers)
+{
+    cntkq_stripe_reduce_item it;
+    std::memset(&it, 0, sizeof it);
+    it.rows = rows;
+    it.stripe_cols = cols;
+    it.stripe_res = reinterpret_cast<float*>(static_cast<uintptr_t>(256)); // (only its alignment is looked at)
+    StripeBatchEntry e;
+    size_t lds = 0;
+    uint64_t blocks = 0;
+    return BatchAbi<float>::stripe_register_member(it, workers, nbits, e, lds, blocks) != kBatchOwnLaunch ? 1 : 0;
+}
+
+size_t cntkq_debug_staged_max_rows(size_t nbits)
+{
+    return staged_max_rows(nbits);
 }
 
 int cntkq_debug_decoder(size_t rows, size_t cols, size_t nbits, int packed_on_host)

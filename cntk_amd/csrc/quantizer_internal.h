@@ -50,6 +50,11 @@ int cntkq_debug_short_columns_f64(size_t rows, size_t cols, size_t nbits);
 int cntkq_debug_decoder(size_t rows, size_t cols, size_t nbits, int packed_on_host);
 int cntkq_debug_decoder_f64(size_t rows, size_t cols, size_t nbits, int packed_on_host);
 
+/* Whether an aligned stripe of a set is a member of the register grids, and the height up to which few tall columns of a set stay
+ * staged in memory rather than have a register grid launched for them. Need no device. */
+int cntkq_debug_stripe_shares_register_grid(size_t rows, size_t cols, size_t nbits, size_t workers);
+size_t cntkq_debug_staged_max_rows(size_t nbits);
+
 /* Bytes of the handle's device staging buffer: 0 until a packed matrix lay in host memory that the kernels do not write and
  * read themselves. */
 size_t cntkq_debug_staging_bytes(const cntkq_quantizer* h);

@@ -89,3 +89,26 @@ def test_decoder_of_one_row(double, nbits, cols):
 def test_decoder_of_one_row_of_wide_codes():
     for nbits in (16, 32):
         assert decoder(1, 2 * 10 ** 7, nbits) == SCALAR and decoder(1, 2 * 10 ** 7, nbits, double=1) == SCALAR
+
+
+def test_stripes_in_register_grids():
+    """Whole pieces, more than six per thread: a single worker's, and at 1 bit up to eight workers' (9304 x 14 at 8 bits and 8 workers took
+    25 us in the general grid, 35 in a register grid); odd heights and 1024 threads whatever the workers."""
+    def shares(*a):
+        return bool(cntk_amd.lib().cntkq_debug_stripe_shares_register_grid(*a))
+
+    for rows in (6176, 9304, 14336):
+        for cols in (1, 64, 1000):
+            for nbits in (2, 4, 8, 16):
+                assert shares(rows, cols, nbits, 1)
+                assert not any(shares(rows, cols, nbits, k) for k in (2, 3, 4, 8))
+            assert shares(rows, cols, 1, 1) and shares(rows, cols, 1, 8) and not shares(rows, cols, 1, 9)
+    for nbits in (2, 8):
+        assert shares(9305, 3, nbits, 4) and shares(20000, 3, nbits, 4) and shares(4099, 3, nbits, 8)
+        assert not shares(4096, 3, nbits, 1) and not shares(2048, 3, nbits, 4)
+
+
+def test_heights_of_few_tall_columns():
+    """Staged in memory beside 8 M elements: 8192 rows 22.9 us, 26.1 with a register grid of their own; 14336 rows 33.0 and 27.6."""
+    L = cntk_amd.lib()
+    assert [L.cntkq_debug_staged_max_rows(b) for b in (1, 2, 4, 8, 16)] == [8192, 8192, 8192, 10240, 10240]
