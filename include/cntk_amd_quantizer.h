@@ -195,8 +195,9 @@ int cntkq_quantize_batch_async(cntkq_quantizer* h, const cntkq_quantize_item* it
 int cntkq_unquantize_batch_async(cntkq_quantizer* h, const cntkq_unquantize_item* items, size_t count, size_t nbits, int add);
 
 /* cntkq_quantize_batch_async for callers that cannot allocate. It has no counterpart in the reference; it is for code
- * under HIP graph capture, tight serving loops and harnesses that forbid hipMalloc. Same arguments, same kernels and the
- * same bytes as cntkq_quantize_batch_async (one exception below), but the call touches no allocator, device or host: the argument table that
+ * under HIP graph capture, tight serving loops and harnesses that forbid hipMalloc. Same arguments and the same bytes as
+ * cntkq_quantize_batch_async (one exception below; matrices whose columns are kept in registers with edge elements or on 1024
+ * threads share a grid there and have a launch each here), but the call touches no allocator, device or host: the argument table that
  * the batched kernels read (the only memory of that call beyond its inputs and outputs) lives in a fixed array in the
  * library's device image -- 32 KB, held by every GPU the library runs on until the process ends -- and reaches it as
  * kernel arguments of a small store kernel, not through a copy.
