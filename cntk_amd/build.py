@@ -23,7 +23,7 @@ HIPCC_FLAGS = [
 
 # The library's source files share no device code and are compiled side by side: the C ABI (float matrices and everything
 # independent of the element type), one file per kernel family of the float instantiation, and the double instantiation.
-SOURCES = ["quantizer_api.hip", "quantizer_family_tile.hip", "quantizer_family_column.hip", "quantizer_family_register_256.hip",
+SOURCES = ["quantizer_api.hip", "quantizer_family_tile.hip", "quantizer_family_lanes.hip", "quantizer_family_lanes_stripe.hip", "quantizer_family_column.hip", "quantizer_family_register_256.hip",
            "quantizer_family_register_1024.hip", "quantizer_family_register_edge.hip", "quantizer_family_strip.hip",
            "quantizer_family_stripe_register_256.hip", "quantizer_family_stripe_register_1024.hip", "quantizer_family_unquantize.hip",
            "quantizer_family_batch_quantize.hip", "quantizer_family_batch_stripe.hip", "quantizer_family_batch_register.hip",

@@ -111,8 +111,17 @@ struct BatchAbi<float>
         }
         if (path == kPathTile)
         {
+            const TileGeom t = make_tile_geom(it.rows, it.cols, nbits, 0, -1, 0);
+            if (lanes_applicable<float>(it.rows, nbits, t.gs))
+            {
+                e.kind = 14;
+                e.l = make_lanes_geom<float>(it.rows, it.cols, nbits, t.gs);
+                lds = lanes_lds_bytes<float>(e.l, 0);
+                blocks = lanes_blocks(e.l);
+                return true;
+            }
             e.kind = 0;
-            e.t = make_tile_geom(it.rows, it.cols, nbits, 0, -1, 0);
+            e.t = t;
             lds = tile_lds_bytes(e.t, 0);
             blocks = (e.t.cols + e.t.cols_per_tile - 1) / e.t.cols_per_tile;
             return true;
@@ -265,6 +274,14 @@ struct BatchAbi<float>
         {
             e.kind = 0;
             e.t = make_tile_geom(it.rows, it.stripe_cols, nbits, 0, -1, 0);
+            if (lanes_stripe_member<float>(it.rows, it.stripe_cols, nbits, e.t.gs, workers))
+            {
+                e.kind = 14;
+                e.l = make_lanes_geom<float>(it.rows, it.stripe_cols, nbits, e.t.gs);
+                lds = lanes_lds_bytes<float>(e.l, workers);
+                blocks = lanes_blocks(e.l);
+                return true;
+            }
             lds = tile_lds_bytes(e.t, (uint32_t) workers);
             blocks = (e.t.cols + e.t.cols_per_tile - 1) / e.t.cols_per_tile;
         }

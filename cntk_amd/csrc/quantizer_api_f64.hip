@@ -66,6 +66,13 @@ struct BatchAbi<double>
         if (lds > f64::kMaxLdsBytes)
             return false;
         blocks = (e.t.cols + e.t.cols_per_tile - 1) / e.t.cols_per_tile;
+        if (path == kPathTile && lanes_applicable<double>(it.rows, nbits, e.t.gs))
+        {
+            e.kind = 14;
+            e.l = make_lanes_geom<double>(it.rows, it.cols, nbits, e.t.gs);
+            lds = lanes_lds_bytes<double>(e.l, 0);
+            blocks = lanes_blocks(e.l);
+        }
         return true;
     }
     // Fills the geometry of a member of the register grid, with the slots dealt as launch_quantize deals them; kBatchOwnLaunch: none.
@@ -150,7 +157,16 @@ struct BatchAbi<double>
         e.t = f64::make_tile_geom(it.rows, it.stripe_cols, nbits, 0); // the plain call's geometry: same bytes
         lds = f64::tile_lds_bytes(e.t, (uint32_t) workers);
         blocks = (e.t.cols + e.t.cols_per_tile - 1) / e.t.cols_per_tile;
-        return lds <= f64::kMaxLdsBytes;
+        if (lds > f64::kMaxLdsBytes)
+            return false;
+        if (lanes_stripe_member<double>(it.rows, it.stripe_cols, nbits, e.t.gs, workers))
+        {
+            e.kind = 14;
+            e.l = make_lanes_geom<double>(it.rows, it.stripe_cols, nbits, e.t.gs);
+            lds = lanes_lds_bytes<double>(e.l, workers);
+            blocks = lanes_blocks(e.l);
+        }
+        return true;
     }
     // ... with the slots dealt as launch_stripe_reduce deals them
     static int stripe_register_member(const SItem& it, size_t, size_t nbits, SEntry& e, size_t& lds, uint64_t& blocks)

@@ -3,6 +3,7 @@
 
 #include "quantizer_kernels_column.h"
 #include "quantizer_kernels_short.h"
+#include "quantizer_kernels_lanes.h"
 #include "quantizer_kernels_register.h"
 #include "quantizer_kernels_unquantize.h"
 
@@ -32,6 +33,15 @@ __device__ __forceinline__ uint32_t batch_find(const uint32_t* __restrict__ begi
     return first + (uint32_t) __popcll(__ballot(v <= b)) - 1u;
 }
 
+// The value of x, the same for the whole wavefront, but unknown to the compiler: what a body loads through it is loaded there. Recognised as
+// the same for several bodies, an entry's fields are all loaded before the first branch, and kernels of many bodies have more of them
+// than scalar registers, which every workgroup then pays for.
+__device__ __forceinline__ uint32_t opaque_scalar(uint32_t x)
+{
+    asm volatile("" : "+s"(x));
+    return x;
+}
+
 // Many matrices in one launch: the workgroups of all matrices form one grid; `begins` (count + 1 entries, ascending)
 // gives the first workgroup of every matrix. A matrix is a run of column tiles (quantize_tile_body) or of single columns
 // (quantize_colg_body). Removes the per-launch floor (several microseconds) that dominates gradient sets made of many
@@ -46,7 +56,7 @@ struct QuantizeBatchEntry
     // 5: columns staged in the residual's memory instead of LDS (c), 6 / 7: columns in registers, up to 3 / 6 pieces per
     // thread (r; below 32 bits); 8 / 9 / 10: members of the register grids (quantize_reg_batch_kernel), up to 4 / 8 / 15 pieces
     // for each of 256 threads, up to 3 / 4 / 6 for each of 1024 (r);
-    // 11: columns of at most 16 rows, one thread each (s)
+    // 11: columns of at most 16 rows, one thread each (s); 14: short columns, a few lanes each (l)
     uint32_t kind;
     uint32_t pad;
     union // the geometry of the entry's kind
@@ -55,6 +65,7 @@ struct QuantizeBatchEntry
         ColGeom c;
         RegGeom r;
         ShortGeom s;
+        LanesGeom l;
     };
     uint32_t reserved[6]; // (keeps the entry at the size the no-allocation call's fixed array is laid out for)
 };
@@ -76,6 +87,15 @@ __global__ __launch_bounds__(kTileThreads) CNTKQ_SGPRS_FOR_8_WAVES void quantize
     {
         const ShortGeom t = entries[e].s;
         quantize_short_body<NBITS, ZT>(entries[e].g, entries[e].r_in, entries[e].r_out, entries[e].q, t, index, reinterpret_cast<float*>(smem_v4));
+    }
+    else if (NBITS < 32 && entries[e].kind == 14)
+    {
+        if constexpr (NBITS < 32)
+        {
+            const QuantizeBatchEntry& en = entries[opaque_scalar(e)];
+            const LanesGeom t = en.l;
+            quantize_lanes_any<NBITS, ZT, float>(en.g, en.r_in, en.r_out, en.q, t, index, reinterpret_cast<char*>(smem_v4));
+        }
     }
     else if (entries[e].kind == 5)
     {
@@ -156,13 +176,15 @@ struct StripeBatchEntry
     // 0: tiles (t), 1: columns (c), 2 / 3: 1-bit columns of 1024 / 2048 rows (the unrolled body; c.qcol),
     // 4 / 5: 1-bit columns of up to eight workers, sums looked up, up to 3 / 6 pieces per thread (r);
     // 8 / 9 / 10: members of the register grids, pieces as QuantizeBatchEntry has them (r, group);
-    // 11: columns of at most 16 rows (s); 12 / 13: columns of a single worker, up to 3 / 6 pieces per thread (r)
+    // 11: columns of at most 16 rows (s); 12 / 13: columns of a single worker, up to 3 / 6 pieces per thread (r);
+    // 14: short columns of a single worker, a few lanes each (l)
     uint32_t kind;
     uint32_t group; // workers whose packed columns are in LDS together
     TileGeom t;
     ColGeom c;
     RegGeom r;
     ShortGeom s;
+    LanesGeom l;
 };
 
 // LOOKUP: the variant that also runs members of kinds 4 and 5 (76 registers instead of 44: a launch without such members
@@ -242,6 +264,15 @@ __global__ __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(st
     {
         const ShortGeom t = en.s;
         stripe_reduce_short_body<NBITS, ZT>(en.src, en.stripe_res, en.q_out, en.agg_out, t, index, reinterpret_cast<float*>(smem_v4));
+    }
+    else if (NBITS < 32 && en.kind == 14)
+    {
+        if constexpr (NBITS < 32)
+        {
+            const StripeBatchEntry& le = entries[opaque_scalar(e)];
+            const LanesGeom t = le.l;
+            stripe_lanes_any<NBITS, ZT, float>(le.src, le.stripe_res, le.q_out, le.agg_out, t, index, reinterpret_cast<char*>(smem_v4));
+        }
     }
     else if constexpr (NBITS == 32)
     {

@@ -859,12 +859,15 @@ struct QuantizeBatchEntry64
     const double* r_in;
     double* r_out;
     char* q;
-    uint32_t kind; // 8 / 9: members of the register grid, up to 4 / 6 pieces for each of 1024 threads (r); otherwise column tiles (t)
+    // 8 / 9: members of the register grid, up to 4 / 6 pieces for each of 1024 threads (r); 14: short columns, a few lanes each (l);
+    // otherwise column tiles (t)
+    uint32_t kind;
     uint32_t pad;
     union
     {
         TileGeom t;
         RegGeom r;
+        LanesGeom l;
     };
 };
 
@@ -874,6 +877,16 @@ __global__ __launch_bounds__(kThreads) void quantize_batch_kernel64(const Quanti
 {
     extern __shared__ f64x2 smem_f64[];
     const uint32_t e = batch_find(begins, count, blockIdx.x);
+    if (NBITS < 64 && entries[e].kind == 14)
+    {
+        if constexpr (NBITS < 64)
+        {
+            const QuantizeBatchEntry64& en = entries[opaque_scalar(e)];
+            const LanesGeom t = en.l;
+            quantize_lanes_any<NBITS, ZT, double>(en.g, en.r_in, en.r_out, en.q, t, blockIdx.x - begins[e], reinterpret_cast<char*>(smem_f64));
+        }
+        return;
+    }
     const TileGeom t = entries[e].t; // by value: read once, then held in registers whatever the kernel stores
     quantize_tile_body<NBITS, ZT>(entries[e].g, entries[e].r_in, entries[e].r_out, entries[e].q, t, blockIdx.x - begins[e],
                                   reinterpret_cast<double*>(smem_f64));
@@ -891,6 +904,7 @@ struct StripeBatchEntry64
     {
         TileGeom t;
         RegGeom r;
+        LanesGeom l;
     };
 };
 
@@ -901,6 +915,16 @@ __global__ __launch_bounds__(kThreads) CNTKQ_SGPRS_FOR_8_WAVES void stripe_reduc
     extern __shared__ f64x2 smem_f64[];
     const uint32_t e = batch_find(begins, count, blockIdx.x);
     const StripeBatchEntry64& en = entries[e]; // the table is read-only while the kernel runs
+    if (NBITS < 64 && en.kind == 14)
+    {
+        if constexpr (NBITS < 64)
+        {
+            const StripeBatchEntry64& le = entries[opaque_scalar(e)];
+            const LanesGeom t = le.l;
+            stripe_lanes_any<NBITS, ZT, double>(le.src, le.stripe_res, le.q_out, le.agg_out, t, blockIdx.x - begins[e], reinterpret_cast<char*>(smem_f64));
+        }
+        return;
+    }
     const TileGeom t = en.t;
     stripe_reduce_tile_body<NBITS, ZT>(en.src, en.stripe_res, en.q_out, en.agg_out, t, blockIdx.x - begins[e],
                                        reinterpret_cast<double*>(smem_f64));

@@ -178,6 +178,75 @@ inline uint32_t short_blocks(const ShortGeom& t)
     return (t.cols - 1) / t.cpt + 1;
 }
 
+// Columns that a few lanes of one wavefront hold, as many as the tile kernels give a column threads (lanes: what make_tile_geom says); the same
+// bytes. Quantize: at every height and size. Tile kernel / this, 36 heights of 17 to 1279 rows: 1.2 to 1.6 at 100000 elements, 1.0 to 1.5
+// at 1 M, 0.98 to 1.2 at 10 M (1.8 at 32 rows); doubles 1.2 to 1.4, 1.06 to 1.4, 0.95 to 1.4.
+template <typename E>
+inline bool lanes_applicable(size_t rows, size_t nbits, uint32_t lanes)
+{
+    return rows > kShortMaxRows && nbits < 8 * sizeof(E) && lanes <= 64 && (rows + lanes - 1) / lanes <= (sizeof(E) == 4 ? kLanesMaxChain : 8u);
+}
+
+// ... in the stripe reduction, where the decoding is the same work for the tile kernels' threads, and a tile's larger share of a compute
+// unit's LDS does not matter once its loads are under way. One worker: 1.04 to 1.6 at 100000 elements, 0.94 to 2.2 above that, but below 32
+// rows at 1 M 0.84 to 1.0. Eight workers: 1.0 to 1.3 at 100000, 0.94 to 1.3 at 1 M, 0.85 to 1.2 at 5 M; below 32 rows 0.94 to 1.1, 0.75 to 1.0
+// and 0.8 to 1.1. Doubles with one worker 1.1 to 1.6, 1.05 to 1.5, 0.9 to 1.8; with eight 0.97 to 1.4, 0.95 to 1.5, 0.73 to 1.8, below 24 rows at
+// 500000 0.81 to 1.3.
+template <typename E>
+inline bool lanes_stripe_applicable(size_t rows, size_t cols, size_t nbits, uint32_t lanes, size_t workers)
+{
+    if (!lanes_applicable<E>(rows, nbits, lanes))
+        return false;
+    constexpr bool F = sizeof(E) == 4;
+    const size_t n = rows * cols;
+    if (workers <= 2)
+        return !F || rows >= 32 || n <= 256 * 1024;
+    return n <= (F ? (rows >= 32 ? 1024 * 1024 : 128 * 1024) : (rows >= 24 ? 512 * 1024 : 64 * 1024));
+}
+
+// ... as members of a set's launch, among which a stripe's size says little about how full the device is: a single worker's (ResNet-50's at 1
+// bit with one worker 50.9 -> 49.2 us, at 4 bits with eight 92 -> 96)
+template <typename E>
+inline bool lanes_stripe_member(size_t rows, size_t cols, size_t nbits, uint32_t lanes, size_t workers)
+{
+    return workers == 1 && lanes_stripe_applicable<E>(rows, cols, nbits, lanes, workers);
+}
+
+template <typename E>
+inline LanesGeom make_lanes_geom(size_t rows, size_t cols, size_t nbits, uint32_t lanes)
+{
+    LanesGeom t;
+    t.rows = (uint32_t) rows;
+    t.cols = (uint32_t) cols;
+    const size_t vpw = 8 * sizeof(E) / nbits;
+    t.nq = (uint32_t) ((rows + vpw - 1) / vpw);
+    t.lanes = lanes;
+    t.lanes_log2 = 3;
+    while ((1u << t.lanes_log2) < lanes)
+        t.lanes_log2++;
+    const uint32_t chain = (t.rows + lanes - 1) / lanes;
+    t.chain = chain <= 4 ? 4 : (chain <= 8 ? 8 : (chain <= 16 ? 16 : 20));
+    t.step_k = lanes / t.nq;
+    t.step_w = lanes % t.nq;
+    const uint32_t columns = 64 / lanes;
+    t.run_elems = (columns * t.rows + 3 + 3) & ~3u; // (as many elements before the run as put it at its phase within 16 bytes)
+    t.rec_words = (columns * (t.nq + 2) + 3) & ~3u;
+    t.qcol = (uint64_t) (2 + t.nq) * sizeof(E);
+    return t;
+}
+
+inline uint32_t lanes_blocks(const LanesGeom& t)
+{
+    const uint32_t c = kLanesWaves * (64 / t.lanes);
+    return (t.cols - 1) / c + 1;
+}
+
+// (a call that sets the tile kernels' geometry by hand is about the tile kernels)
+inline bool tile_geometry_forced(const LaunchTuning& tune)
+{
+    return tune.quantize_path != kPathAuto || tune.tile_gs != 0 || tune.tile_stage >= 0 || tune.tile_threads != 0;
+}
+
 template <template <int, bool> class Launcher, typename... Args>
 inline hipError_t dispatch_nbits(size_t nbits, bool zt, Args... args)
 {
@@ -206,6 +275,14 @@ hipError_t family_short_quantize(size_t nbits, bool zt, hipStream_t s, LaunchEve
                                  ShortGeom t);
 hipError_t family_short_stripe(size_t nbits, bool zt, hipStream_t s, LaunchEvents ev, const StripeSources& src, float* stripe_res, char* q_out,
                                float* agg_out, ShortGeom t);
+hipError_t family_lanes_quantize(size_t nbits, bool zt, hipStream_t s, LaunchEvents ev, const float* g, const float* r_in, float* r_out, char* q,
+                                 const LanesGeom& t);
+hipError_t family_lanes_quantize(size_t nbits, bool zt, hipStream_t s, LaunchEvents ev, const double* g, const double* r_in, double* r_out, char* q,
+                                 const LanesGeom& t);
+hipError_t family_lanes_stripe(size_t nbits, bool zt, hipStream_t s, LaunchEvents ev, const StripeSources& src, float* stripe_res, char* q_out,
+                               float* agg_out, const LanesGeom& t);
+hipError_t family_lanes_stripe(size_t nbits, bool zt, hipStream_t s, LaunchEvents ev, const StripeSources& src, double* stripe_res, char* q_out,
+                               double* agg_out, const LanesGeom& t);
 hipError_t family_tall_quantize(size_t nbits, bool zt, hipStream_t s, LaunchEvents ev, const float* g, const float* r_in, float* r_out, char* q,
                                 uint32_t rows, uint32_t cols, uint32_t nq, uint64_t qcol);
 hipError_t family_col_quantize(size_t nbits, bool zt, hipStream_t s, LaunchEvents ev, const float* g, const float* r_in, float* r_out, char* q,
@@ -763,6 +840,8 @@ inline hipError_t launch_quantize(hipStream_t s, LaunchEvents ev, const float* g
         if (tune.quantize_path == kPathAuto && short_applicable(rows, cols, qwords_per_col(rows, nbits)))
             return family_short_quantize(nbits, zt, s, ev, g, r_in, r_out, qc, make_short_geom(rows, cols, qwords_per_col(rows, nbits), qcol_bytes(nbits, rows), sizeof(float)));
         const TileGeom t = make_tile_geom(rows, cols, nbits, tune.tile_gs, tune.tile_stage, tune.tile_threads);
+        if (!tile_geometry_forced(tune) && lanes_applicable<float>(rows, nbits, t.gs))
+            return family_lanes_quantize(nbits, zt, s, ev, g, r_in, r_out, qc, make_lanes_geom<float>(rows, cols, nbits, t.gs));
         return family_tile_quantize(nbits, zt, s, ev, g, r_in, r_out, qc, t);
     }
     return family_tall_quantize(nbits, zt, s, ev, g, r_in, r_out, qc, (uint32_t) rows, (uint32_t) cols,
@@ -885,6 +964,8 @@ inline hipError_t launch_stripe_reduce(hipStream_t s, LaunchEvents ev, const Str
     // Same tile geometry as launch_quantize would use for a matrix of this height, so that the statistics are summed in
     // the same order and the fused call gives the bytes of the reference's unquantize ... quantize call sequence.
     const TileGeom t = make_tile_geom(rows, cols, nbits, tune.tile_gs, tune.tile_stage, tune.tile_threads);
+    if (!tile_geometry_forced(tune) && lanes_stripe_applicable<float>(rows, cols, nbits, t.gs, src.workers))
+        return family_lanes_stripe(nbits, zt, s, ev, src, stripe_res, static_cast<char*>(q_out), agg_out, make_lanes_geom<float>(rows, cols, nbits, t.gs));
     return family_tile_stripe(nbits, zt, s, ev, src, stripe_res, static_cast<char*>(q_out), agg_out, t);
 }
 
