@@ -8,18 +8,23 @@
 // from registers; the parts of a QWord meet in LDS. The kernels are written once over the element type. Gradient and
 // residual are read once whatever the height, which columns above 102400 rows -- more than any workgroup's registers
 // hold -- could otherwise only have by reading their inputs two or three times. A strip needs 2 to 8 KB of LDS and, at
-// 1 to 4 bits, some 100 registers (its 32 values, their addresses, the masks of the ragged last strip), so two
-// workgroups share a CU; it is the exchange described next, not memory, that bounds the kernel (4.0 to 5.0 TB/s), and
-// below 102400 rows the kernels with one workgroup per column are faster. (Strips of 256 threads, five to a CU, were 7
+// 1 to 4 bits, some 100 registers (its 32 values and as many of the residual on their way), so two workgroups share a
+// CU; memory and the exchange described next bound the kernel together (200000 x 256: 138 us at 1 bit, 125 at 2, 135 at
+// 8; without the exchange 125, 122 and 119), and below 102400 rows the kernels with one workgroup per column are faster.
+// (Three workgroups to a CU, 80 registers: 8 to 14 % slower wherever the last strip is ragged, level elsewhere. Strips of 256 threads, five to a CU, were 7
 // to 25 % slower, strips of 1024 threads about as fast as these at a few shapes and slower at most: the fewer
 // workgroups a column's sums must cross, the better, until too few bytes are in flight.)
 //
 // The column statistics span the strips of a column. Every workgroup publishes its partial sums in a scratch buffer,
 // one 8-byte record per 32 bits of a sum (a double takes two): the bits and the tag of the launch, written by one
 // atomic store, so that whoever reads the tag of this launch has the bits with it and no second word needs ordering
-// against the first. Then the first wavefront of every workgroup of the column polls the S records (a lane per record,
+// against the first. Then the first wavefront of every workgroup of the column polls the S records (a lane per strip,
 // with pauses) until all carry the tag, and adds them up, lanes meeting by butterfly -- one fixed order, the same bytes
-// in every workgroup. One exchange for the sum of squares (more than 1 bit) or the split sums (1 bit against 0), two
+// in every workgroup. Reads of one address take their turns, and the records that S workgroups poll are S times as
+// much in demand as anything else: the publishing stores had to queue behind the polls of those that were waiting for
+// them. So a record is written into several copies, one for every four strips (at most 16 copies), and a workgroup polls
+// its own (200000 x 256 at 8 bits, 25 strips: 152 us with one copy, 139 / 137 / 135 / 137 with one for every 8 / 4 / 2 / 1
+// strips; 262144 x 200: 157, 142 / 135 / 135 / 136). One exchange for the sum of squares (more than 1 bit) or the split sums (1 bit against 0), two
 // for 1 bit against the mean (mean, then split sums). The tag is a launch count kept in the scratch buffer itself:
 // every workgroup reads it when it starts, and the last workgroup to finish (a second counter tells) raises it, so that
 // replays of a recorded graph see fresh tags like any other launch. The strips of a column take workgroup indices 8
@@ -87,9 +92,9 @@ struct StripShape
     static constexpr uint32_t RUNS = kStripThreads / CHUNKS;      // runs of PER QWords per strip
     // QWords per strip: float 512, 1024, 2048, 2048, 2048 at 1, 2, 4, 8, 16 bits; double 128, 256, 512, 1024, 1024, 1024 at 1 ... 32 bits
     static constexpr uint32_t WORDS = PER * RUNS;
-    // wavefronts per SIMD the kernels are compiled for (the registers that leaves them: 128 at 4, 64 at 8): two workgroups of
-    // eight wavefronts are what a compute unit holds where a thread has eight bit positions, and with fewer registers the
-    // ragged last strip spills, and every strip of its column waits for it
+    // wavefronts per SIMD the kernels are compiled for (the registers that leaves them: 128 at 4, 64 at 8): where a thread
+    // has eight bit positions, two workgroups of eight wavefronts whose loads of gradient and residual are all in flight at
+    // once are faster than three that fetch the residual two pieces at a time
     static constexpr uint32_t WAVES = SLOTS == 8 ? 4 : 8;
 };
 
@@ -115,7 +120,7 @@ struct StripGeom
     uint32_t spread;     // non-zero: a column's strips take consecutive workgroup indices, i.e. all dies (columns of more strips than one die holds)
     uint32_t whole_positions; // rows / nq: bit positions at which every QWord of a column has an element
     uint32_t last_words;      // rows % nq: QWords with an element at bit position whole_positions (none beyond it)
-    uint32_t pad;
+    uint32_t copy_shift;      // a column's records are kept once for every 2^copy_shift of its strips
     uint64_t qcol;
 };
 
@@ -183,57 +188,76 @@ __device__ __forceinline__ void strip_publish_value(uint64_t* rec, uint32_t stri
         strip_publish(rec + h * strips, w[h], tag);
 }
 
-// Waits for one record to carry the tag and returns its 32 bits. `bad`: its workgroup abandoned it, or it was not there
-// after the bounded wait.
-__device__ __forceinline__ uint32_t strip_poll(const uint64_t* rec, uint32_t tag, const StripGeom& c, bool& bad)
+// A column's records: [copy][record][strip]. A strip writes its own into every copy and reads those of one copy, which it
+// shares with 2^copy_shift - 1 neighbours.
+__host__ __device__ inline uint32_t strip_copies(uint32_t strips, uint32_t copy_shift)
 {
-    uint32_t polls = 0;
-    uint64_t x;
-    for (;;)
+    return ((strips - 1) >> copy_shift) + 1;
+}
+template <typename E>
+__device__ __forceinline__ uint64_t* strip_column_records(const StripScratch& scratch, uint32_t column, const StripGeom& c)
+{
+    return scratch.records + (size_t) column * strip_copies(c.strips, c.copy_shift) * strip_records<E>() * c.strips;
+}
+
+template <typename T>
+__device__ __forceinline__ T strip_value(const uint32_t* w)
+{
+    T value;
+    __builtin_memcpy(&value, w, sizeof(T));
+    return value;
+}
+
+// Waits for N records, `stride` apart, to carry the tag and returns their 32 bits each. False: their workgroup abandoned
+// them, or they were not there after the bounded wait. (All N are asked for in every poll: one round trip, not N.)
+template <uint32_t N>
+__device__ __forceinline__ bool strip_poll(const uint64_t* rec, uint32_t stride, uint32_t tag, const StripGeom& c, uint32_t* w)
+{
+    for (uint32_t polls = 0;; ++polls)
     {
-        x = __hip_atomic_load(rec, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const uint32_t got = (uint32_t) (x >> 32);
-        if (got == tag)
-            break;
-        if (got == (tag | kStripAbandoned) || polls >= c.spin_limit)
+        uint64_t x[N];
+#pragma unroll
+        for (uint32_t n = 0; n < N; ++n)
+            x[n] = __hip_atomic_load(rec + n * stride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        bool there = true, abandoned = false;
+#pragma unroll
+        for (uint32_t n = 0; n < N; ++n)
         {
-            bad = true;
-            break;
+            const uint32_t got = (uint32_t) (x[n] >> 32);
+            there = there && got == tag;
+            abandoned = abandoned || got == (tag | kStripAbandoned);
+            w[n] = (uint32_t) x[n];
         }
-        ++polls;
+        if (there)
+            return true;
+        if (abandoned || polls >= c.spin_limit)
+            return false;
         for (uint32_t z = 0; z < c.poll_pause; ++z)
             __builtin_amdgcn_s_sleep(1);
     }
-    return (uint32_t) x;
 }
 
-// One wavefront collects the S values of a sum: lane l polls the records of strips l, l + 64, ... until they carry the tag,
-// adds their values in ascending order, and the lanes meet by butterfly. Every lane returns the same bits.
-// Polls are loads at device scope, and a thousand resident workgroups polling as fast as they can took half of the L2's
-// request rate from the loads and stores that the records wait for: a lane pauses poll_pause x 64 cycles between two polls
-// (200000 x 256 at 1 bit over 1 / 16 / 64 / 128 / 256: 214 / 208 / 200 / 198 / 208 us), and first_pause x 64 cycles
-// before the first one of an exchange, which with many strips per column practically never finds the record there
-// (with strips of 256 threads: 262144 x 200, 32 strips: 174 -> 154 us with 64; 24576 x 2048, 3 strips: 116 -> 132 us; with
-// strips of 512 threads: 204800 x 256, 13 strips: 140 -> 135 us; 102401 x 512, 7 strips: 173 -> 175 us: from 8 strips on).
-template <typename T>
-__device__ __forceinline__ T strip_collect(const uint64_t* recs, uint32_t strips, uint32_t tag, const StripGeom& c, uint32_t first_pause, bool& gave_up)
+// One wavefront collects the S values of N / H sums: lane l polls the records of strips l, l + 64, ... until they carry the
+// tag and hands their words to `add` in ascending order; the caller's lanes then meet by butterfly. False in every lane if
+// a record of any lane did not come.
+// Polls are loads at device scope and stand in the way of the stores that they wait for: a lane pauses poll_pause x 64
+// cycles between two polls (over 8 / 16 / 32 / 64: 200000 x 256 at 1 bit 140 / 139 / 138 / 144 us, at 8 bits 142 / 140 /
+// 136 / 135), and the wavefront poll_first x 64 cycles before the first one, which with many strips per column practically
+// never finds the records there. All sums of an exchange are asked for together: at 1 bit the split sums cost one round
+// trip instead of three (1000003 x 24: 79 -> 75 us).
+template <uint32_t N, typename Add>
+__device__ __forceinline__ bool strip_collect(const uint64_t* recs, uint32_t strips, uint32_t tag, const StripGeom& c, Add add)
 {
-    T t = 0;
-    bool bad = false;
-    for (uint32_t s = threadIdx.x & 63u; s < strips; s += 64)
+    for (uint32_t z = 0; z < c.poll_first; ++z)
+        __builtin_amdgcn_s_sleep(1);
+    bool there = true;
+    for (uint32_t s = threadIdx.x & 63u; s < strips && there; s += 64)
     {
-        for (uint32_t z = 0; z < first_pause; ++z)
-            __builtin_amdgcn_s_sleep(1);
-        uint32_t w[sizeof(T) / 4];
-#pragma unroll
-        for (uint32_t h = 0; h < sizeof(T) / 4; ++h)
-            w[h] = bad ? 0u : strip_poll(recs + h * strips + s, tag, c, bad);
-        T val;
-        __builtin_memcpy(&val, w, sizeof(T));
-        t += val;
+        uint32_t w[N];
+        there = strip_poll<N>(recs + s, strips, tag, c, w);
+        add(w);
     }
-    gave_up = gave_up || __ballot(bad) != 0ull; // the same in every lane of the wavefront
-    return wave_sum(t);
+    return __ballot(!there) == 0ull; // the same in every lane of the wavefront
 }
 
 // The workgroup abandons its strip: every record of it says so (whichever exchange a neighbour is in, it meets the mark),
@@ -241,8 +265,8 @@ __device__ __forceinline__ T strip_collect(const uint64_t* recs, uint32_t strips
 __device__ __forceinline__ void strip_abandon(uint64_t* recs, uint32_t records_each, uint32_t strip, uint32_t tag, const StripGeom& c,
                                               const StripScratch& scratch)
 {
-    for (uint32_t f = 0; f < records_each; ++f)
-        strip_publish(recs + f * c.strips + strip, 0u, tag | kStripAbandoned);
+    for (uint32_t f = 0; f < records_each * strip_copies(c.strips, c.copy_shift); ++f)
+        strip_publish(recs + (size_t) f * c.strips + strip, 0u, tag | kStripAbandoned);
     __hip_atomic_store(scratch.error, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     if (strip == 0)
         __hip_atomic_fetch_add(&scratch.header->abandoned, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -300,15 +324,18 @@ __device__ __forceinline__ E strip_exchange_stat(E stat, uint32_t column, uint32
     if (PASS == 0 && c.strips == 1)
         return stat;
     constexpr uint32_t H = sizeof(E) / 4; // records per sum
-    uint64_t* recs = scratch.records + (size_t) column * strip_records<E>() * c.strips; // [record][strip]
-    if (threadIdx.x == 0 && PASS <= kStripPassStat)
-        strip_publish_value(recs + strip, c.strips, stat, tag);
+    uint64_t* recs = strip_column_records<E>(scratch, column, c);
+    const uint32_t copies = strip_copies(c.strips, c.copy_shift), copy_records = strip_records<E>() * c.strips;
+    if (threadIdx.x < copies && PASS <= kStripPassStat)
+        strip_publish_value(recs + threadIdx.x * copy_records + strip, c.strips, stat, tag);
     if constexpr (PASS == kStripPassStat)
         return stat;
+    const uint64_t* mine = recs + (strip >> c.copy_shift) * copy_records;
     if (threadIdx.x < 64)
     {
-        bool gave_up = false;
-        const E t = strip_collect<E>(recs, c.strips, tag, c, c.poll_first, gave_up);
+        E t = 0;
+        const bool gave_up = !strip_collect<H>(mine, c.strips, tag, c, [&](const uint32_t* w) { t += strip_value<E>(w); });
+        t = wave_sum(t);
         if (threadIdx.x == 0)
         {
             red[0] = t;
@@ -332,21 +359,30 @@ __device__ __forceinline__ void strip_exchange_split(E& s0, E& s1, uint32_t& n0,
     if (PASS == 0 && c.strips == 1)
         return;
     constexpr uint32_t H = sizeof(E) / 4;
-    uint64_t* recs = scratch.records + (size_t) column * strip_records<E>() * c.strips;
-    if (threadIdx.x == 0 && PASS != kStripPassPack)
+    uint64_t* recs = strip_column_records<E>(scratch, column, c);
+    const uint32_t copies = strip_copies(c.strips, c.copy_shift), copy_records = strip_records<E>() * c.strips;
+    if (threadIdx.x < copies && PASS != kStripPassPack)
     {
-        strip_publish_value(recs + 1 * H * c.strips + strip, c.strips, s0, tag);
-        strip_publish_value(recs + 2 * H * c.strips + strip, c.strips, s1, tag);
-        strip_publish_value(recs + 3 * H * c.strips + strip, c.strips, n0, tag);
+        uint64_t* at = recs + threadIdx.x * copy_records + strip;
+        strip_publish_value(at + 1 * H * c.strips, c.strips, s0, tag);
+        strip_publish_value(at + 2 * H * c.strips, c.strips, s1, tag);
+        strip_publish_value(at + 3 * H * c.strips, c.strips, n0, tag);
     }
     if constexpr (PASS == kStripPassSplit)
         return;
+    const uint64_t* mine = recs + (strip >> c.copy_shift) * copy_records;
     if (threadIdx.x < 64)
     {
-        bool gave_up = false;
-        const E t0 = strip_collect<E>(recs + 1 * H * c.strips, c.strips, tag, c, c.poll_first, gave_up);
-        const E t1 = strip_collect<E>(recs + 2 * H * c.strips, c.strips, tag, c, 0u, gave_up);
-        const uint32_t tn = strip_collect<uint32_t>(recs + 3 * H * c.strips, c.strips, tag, c, 0u, gave_up);
+        E t0 = 0, t1 = 0;
+        uint32_t tn = 0;
+        const bool gave_up = !strip_collect<2 * H + 1>(mine + 1 * H * c.strips, c.strips, tag, c, [&](const uint32_t* w) {
+            t0 += strip_value<E>(w);
+            t1 += strip_value<E>(w + H);
+            tn += w[2 * H];
+        });
+        t0 = wave_sum(t0);
+        t1 = wave_sum(t1);
+        tn = wave_sum(tn);
         if (threadIdx.x == 0)
         {
             red[0] = t0;
@@ -470,6 +506,7 @@ __device__ __forceinline__ void strip_stats_pack(StripVec<E>* v, uint32_t valid,
                     s0 += below ? x : (E) 0;
                     s1 += below ? (E) 0 : x;
                     n0 += below ? 1u : 0u;
+                    asm volatile("" : "+v"(s0), "+v"(s1), "+v"(n0));
                 }
             if constexpr (!FULL)
                 n0 -= (E) 0 < mean ? (uint32_t) __popc(~valid) : 0u; // the zeros that stand in for elements that do not exist
@@ -491,7 +528,10 @@ __device__ __forceinline__ void strip_stats_pack(StripVec<E>* v, uint32_t valid,
 #pragma unroll
     for (uint32_t kk = 0; kk < SS::SLOTS; ++kk)
     {
+        constexpr uint32_t ALL = (1u << PER) - 1u;
+        const uint32_t ok = FULL ? ALL : (opaque(valid) >> (PER * kk)) & ALL;
         typename SE::V r;
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (uint32_t e = 0; e < PER; ++e)
         {
@@ -504,12 +544,10 @@ __device__ __forceinline__ void strip_stats_pack(StripVec<E>* v, uint32_t valid,
                 back = unquantize_value<NBITS, E>(vq, code);
             r[e] = x - back;
             if constexpr (!FULL)
-                code &= (Q) 0 - (Q) ((valid >> (PER * kk + e)) & 1u);
+                code &= (Q) 0 - (Q) ((ok >> e) & 1u);
             word[e] |= code << ((k0 + kk) * PS::SHIFT);
         }
         E* dst = res + (size_t) kk * c.nq + w;
-        constexpr uint32_t ALL = (1u << PER) - 1u;
-        const uint32_t ok = FULL ? ALL : (valid >> (PER * kk)) & ALL;
         if (ok == ALL)
             __builtin_nontemporal_store(r, reinterpret_cast<typename SE::VU*>(dst));
         else if (ok != 0u)
@@ -633,12 +671,30 @@ __device__ __forceinline__ uint32_t strip_valid_mask(const StripGeom& c, uint32_
     return valid;
 }
 
+// A piece loaded `over` values early (its own place runs over the column's end): its values to the front, and what does
+// not exist to zero.
+template <typename E>
+__device__ __forceinline__ void strip_clear(StripVec<E>& x, uint32_t over, uint32_t ok)
+{
+    constexpr uint32_t PER = StripElem<E>::PER;
+#pragma unroll
+    for (uint32_t by = PER / 2; by >= 1; by /= 2)
+#pragma unroll
+        for (uint32_t e = 0; e < PER; ++e)
+            x[e] = (over & by) ? (e + by < PER ? x[e + by] : (E) 0) : x[e];
+#pragma unroll
+    for (uint32_t e = 0; e < PER; ++e)
+        x[e] = ((ok >> e) & 1u) ? x[e] : (E) 0;
+}
+
 // N pieces of a column, the PER consecutive values from element i0 + n * stride on each (16 bytes at the alignment of an
 // element), all requested before any is used. FULL: all values exist. Otherwise bit PER * n + e of `valid` says whether
 // value e of piece n does, and the others read as zero. Every lane loads 16 bytes from inside its column whatever it
-// holds (its own piece where that ends inside the column, the column's first elements otherwise), so that no branch
-// stands between the loads; what does not exist is then cleared, and the few values of a piece that runs over the
-// column's end (fewer than PER per column) are fetched one by one.
+// holds: its own piece, or the column's last PER elements where that would run over the end, so that no branch stands
+// between the loads. Values that came early are then moved to their place and what does not exist is cleared, a piece at a
+// time from opaque copies of the index and the mask (kept for all pieces at once, the predicates took more registers
+// than the values: every strip of a column waits for its ragged one; 102401 x 64 at 1 bit 27.7 -> 26.1 us, 600000 x 40
+// 86 -> 77).
 template <bool FULL, uint32_t N, typename E>
 __device__ __forceinline__ void strip_load_pieces(const E* col, uint32_t i0, uint32_t stride, uint32_t rows, uint32_t valid, StripVec<E>* out)
 {
@@ -652,24 +708,20 @@ __device__ __forceinline__ void strip_load_pieces(const E* col, uint32_t i0, uin
     }
     else
     {
-        uint32_t over = 0; // pieces with values that run over the column's end
         if (rows >= PER)
         {
 #pragma unroll
             for (uint32_t n = 0; n < N; ++n)
             {
                 const uint32_t i = i0 + n * stride;
-                out[n] = __builtin_nontemporal_load(reinterpret_cast<const typename SE::VU*>(col + (i + PER <= rows ? i : 0u)));
+                out[n] = __builtin_nontemporal_load(reinterpret_cast<const typename SE::VU*>(col + (i < rows - PER ? i : rows - PER)));
             }
 #pragma unroll
             for (uint32_t n = 0; n < N; ++n)
             {
-                const uint32_t i = i0 + n * stride, ok = (valid >> (PER * n)) & ALL;
-                const bool inside = i + PER <= rows;
-                over |= (!inside && ok != 0u) ? (1u << n) : 0u;
-#pragma unroll
-                for (uint32_t e = 0; e < PER; ++e)
-                    out[n][e] = (inside && ((ok >> e) & 1u)) ? out[n][e] : (E) 0;
+                const uint32_t i = opaque(i0) + n * stride;
+                const uint32_t over = i < rows - PER ? 0u : i - (rows - PER);
+                strip_clear<E>(out[n], over, opaque(valid) >> (PER * n));
             }
         }
         else
@@ -677,31 +729,18 @@ __device__ __forceinline__ void strip_load_pieces(const E* col, uint32_t i0, uin
 #pragma unroll
             for (uint32_t n = 0; n < N; ++n)
             {
+                const uint32_t i = i0 + n * stride;
 #pragma unroll
                 for (uint32_t e = 0; e < PER; ++e)
-                    out[n][e] = 0;
-                over |= ((valid >> (PER * n)) & ALL) != 0u ? (1u << n) : 0u;
-            }
-        }
-        if (over != 0u)
-        {
-#pragma unroll
-            for (uint32_t n = 0; n < N; ++n)
-            {
-                const uint32_t i = i0 + n * stride, ok = (valid >> (PER * n)) & ALL;
-                if ((over >> n) & 1u)
-                {
-#pragma unroll
-                    for (uint32_t e = 0; e < PER; ++e)
-                        if ((ok >> e) & 1u)
-                            out[n][e] = col[i + e];
-                }
+                    out[n][e] = col[i + e < rows ? i + e : 0u];
+                strip_clear<E>(out[n], 0u, opaque(valid) >> (PER * n));
             }
         }
     }
 }
 
-// The gradient goes straight into the registers that will hold the sums, the residual joins it four loads at a time. Every
+// The gradient goes straight into the registers that will hold the sums; the residual's loads are in flight with it (four
+// at a time: 200000 x 256 at 1 bit 151 -> 147 us). Every
 // value of the strip is in registers before anything is stored, so r_out may be r_in.
 template <int NBITS, bool ZT, bool FULL, typename E, int PASS>
 __device__ __forceinline__ void quantize_strip_body(const E* g_col, const E* r_col, E* res_col, char* qc, uint32_t column, uint32_t strip,
@@ -715,10 +754,11 @@ __device__ __forceinline__ void quantize_strip_body(const E* g_col, const E* r_c
     const uint32_t i0 = k0 * c.nq + w;
     StripVec<E> v[SS::SLOTS];
     strip_load_pieces<FULL, SS::SLOTS, E>(g_col, i0, c.nq, c.rows, valid, v);
-    constexpr uint32_t BATCH = SS::SLOTS < 4 ? SS::SLOTS : 4;
+    constexpr uint32_t BATCH = SS::SLOTS;
 #pragma unroll
     for (uint32_t k1 = 0; k1 < SS::SLOTS; k1 += BATCH)
     {
+        __builtin_amdgcn_sched_barrier(0);
         StripVec<E> b[BATCH];
         strip_load_pieces<FULL, BATCH, E>(r_col, i0 + k1 * c.nq, c.nq, c.rows, valid >> (PER * k1), b);
 #pragma unroll
@@ -858,10 +898,11 @@ __device__ __forceinline__ void stripe_reduce_strip_body(const StripeSources& sr
             }
         }
     }
-    constexpr uint32_t BATCH = SS::SLOTS < 4 ? SS::SLOTS : 4;
+    constexpr uint32_t BATCH = SS::SLOTS;
 #pragma unroll
     for (uint32_t k1 = 0; k1 < SS::SLOTS; k1 += BATCH)
     {
+        __builtin_amdgcn_sched_barrier(0);
         StripVec<E> b[BATCH];
         strip_load_pieces<FULL, BATCH, E>(res_col, i0 + k1 * c.nq, c.nq, c.rows, valid >> (PER * k1), b);
 #pragma unroll

@@ -29,8 +29,12 @@ enum QuantizePath
 
 constexpr uint32_t kTileMaxRows = 14336; // 56 KB of LDS for a one-column tile
 constexpr size_t kTileMaxFloats = 5120;   // ... and 20 KB for a tile of several columns
-constexpr uint32_t kStripPollPause = 64;           // strip kernel: 64-cycle pauses between two polls of a partial sum
-constexpr uint32_t kStripFirstPauseMinStrips = 8; // ... strips per column from which a pause of 2 x strips precedes the first poll
+constexpr uint32_t kStripPollPause = 32;           // strip kernel: 64-cycle pauses between two polls of a partial sum
+// ... strips per column from which a pause of 3 x strips, at most kStripFirstPauseMax, precedes the first poll. No pause, 1,
+// 2, 3, 4 x strips: 200000 x 256 at 8 bits (25 strips) 144, 139, 138, 135, 132 us; 524288 x 64 at 1 bit (32) 93, 90, 92, 95,
+// 98; 1000003 x 24 at 1 bit (62) 75, 76, 82, 90, 99: more strips wait for each other less long, so the pause stops growing.
+constexpr uint32_t kStripFirstPauseMinStrips = 8;
+constexpr uint32_t kStripFirstPauseMax = 80;
 constexpr uint32_t kStripeWideItems = 768;   // work items per column from which the stripe reduction may use more than 256 threads
 constexpr uint32_t kStripeWideMaxCols = 256; // ... 1024 threads up to this many columns
 constexpr uint32_t kColMinRows = 1024;   // shorter columns are better served several to a workgroup (tile kernels)
@@ -59,7 +63,7 @@ struct StripScratchOwner
 struct LaunchTuning
 {
     StripScratchOwner* strip = nullptr; // null: the strip kernels are not available to this launch
-    uint32_t strip_spin_limit = 1u << 17; // polls of a partial sum (two microseconds or so each) before a lane gives up
+    uint32_t strip_spin_limit = 1u << 18; // polls of a partial sum (two microseconds or so each) before a lane gives up
     bool strip_may_allocate = true; // false: the strip kernels only where the scratch buffer as it stands holds the launch
     bool strip_never_waits = false; // true: tall columns take the strips in passes, whose workgroups never wait for one another
     int quantize_path = kPathAuto;
@@ -512,12 +516,12 @@ inline StripGeom make_strip_geom(size_t rows, size_t cols, size_t nbits, uint32_
     c.strips = (c.nq + strip_words<E>(nbits) - 1) / strip_words<E>(nbits);
     c.spin_limit = spin_limit;
     c.poll_pause = kStripPollPause;
-    c.poll_first = c.strips >= kStripFirstPauseMinStrips ? 2u * std::min(c.strips, kStripMaxPerColumn) : 0u;
+    c.poll_first = c.strips >= kStripFirstPauseMinStrips ? std::min(3u * c.strips, kStripFirstPauseMax) : 0u;
     c.inv_strips = 1.0 / (double) c.strips;
     c.spread = c.strips > per_die ? 1u : 0u;
     c.whole_positions = (uint32_t) (rows / c.nq);
     c.last_words = (uint32_t) (rows % c.nq);
-    c.pad = 0;
+    c.copy_shift = 31; // one copy
     c.qcol = (uint64_t) (2 + c.nq) * sizeof(E); // the header's two bounds, then the QWords
     return c;
 }
@@ -584,6 +588,15 @@ inline hipError_t strip_scratch_for(StripScratchOwner& o, hipStream_t s, size_t 
     out.groups = reinterpret_cast<uint32_t*>(o.dev + sizeof(StripHeader));
     out.records = reinterpret_cast<uint64_t*>(o.dev + sizeof(StripHeader) + o.groups_bytes);
     return hipSuccess;
+}
+
+// A copy of a column's records for every four strips, and at most 16 of them: 1 KB of records per strip of 16 KB and more.
+inline uint32_t strip_copy_shift(uint32_t strips)
+{
+    uint32_t shift = 2;
+    while (strip_copies(strips, shift) > 16)
+        ++shift;
+    return shift;
 }
 
 // whether this launch finds its scratch buffer without allocating, or may allocate (the caller permits it and the stream
@@ -686,11 +699,16 @@ inline hipError_t launch_on_strips(hipStream_t s, size_t rows, size_t cols, size
         return hipErrorInvalidValue;
     StripScratchOwner& o = *tune.strip;
     StripScratch scratch;
-    hipError_t rc = strip_scratch_for(o, s, cols, c.strips, strip_records<E>(), scratch);
-    if (rc != hipSuccess)
-        return rc;
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     const bool capturing = hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+    // (the copies of the records only where the buffer has or may get the room: without them it takes what it always took)
+    const uint32_t copy_shift = strip_copy_shift(c.strips);
+    if (!passes && (strip_scratch_fits(o, cols, c.strips, strip_records<E>() * strip_copies(c.strips, copy_shift)) ||
+                    (tune.strip_may_allocate && !capturing)))
+        c.copy_shift = copy_shift;
+    hipError_t rc = strip_scratch_for(o, s, cols, c.strips, strip_records<E>() * strip_copies(c.strips, c.copy_shift), scratch);
+    if (rc != hipSuccess)
+        return rc;
     if (capturing)
         o.captured = true;
     if (!capturing)

@@ -1,0 +1,78 @@
+"""Tall columns in strips: ragged ends at every remainder, every number of copies of the strips' partial sums, and a launch whose scratch
+buffer has no room for copies. The strips in passes (nothing waits, one copy) add the same sums in the same order and are the oracle.
+Needs an MI355X."""
+import pytest
+import torch
+
+import datagen
+from cntk_amd import Matrix, MatrixQuantizerImpl, QuantizedMatrix
+
+pytestmark = pytest.mark.gpu
+
+PATH_STRIP, PATH_STRIP_PASSES = 6, 7
+F32, F64 = torch.float32, torch.float64
+WORDS = {F32: {1: 512, 2: 1024, 4: 2048, 8: 2048, 16: 2048}, F64: {1: 128, 4: 512, 32: 1024}}  # QWords per strip
+
+
+def _quantize(qz, g, r, rows, cols, nbits, dtype, zt):
+    G, R = Matrix(rows, cols, 0, g, dtype=dtype), Matrix(rows, cols, 0, r.clone(), dtype=dtype)
+    Q = QuantizedMatrix(rows, cols, nbits, 0, dtype=dtype)
+    Q.buffer.fill_(0xA5)
+    qz.QuantizeAsync(G, R, Q, R, zt)
+    qz.WaitQuantizeAsyncDone()
+    torch.cuda.synchronize()
+    return Q.buffer, R.data.view(torch.uint8)
+
+
+# strips per column: fewer than share a copy, the edges of 1, 2 and 3 copies, the edges of the pause before the first look (8, 27),
+# more than a wavefront has lanes, and more than 16 copies of four take (65); ends: whole strips, one QWord more, a piece
+# that runs over the column's end by one to three elements, a last bit position that is nearly or almost empty
+@pytest.mark.parametrize("dtype,nbits,zt", [(F32, 1, False), (F32, 1, True), (F32, 2, False), (F32, 4, False), (F32, 8, False), (F32, 16, False),
+                                            (F64, 1, False), (F64, 4, False), (F64, 32, False)])
+def test_strips_against_passes(dtype, nbits, zt):
+    qz = MatrixQuantizerImpl.Create(0, False)
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(datagen.case_seed(97, nbits))
+    words, per = WORDS[dtype][nbits], (32 if dtype == F32 else 64) // nbits
+    for strips in (2, 4, 5, 8, 9, 27, 28, 64, 65, 70):
+        if strips > qz._strip_max_strips(nbits, zt, dtype):
+            continue
+        for extra in (0, 1, 2, 3, 5, per, words * per - 1, words * per // 2 + 1):
+            rows = (strips - 1) * words * per + (extra if extra else words * per)
+            cols = 3 if strips < 28 else 1
+            print(dtype, nbits, zt, "strips", strips, "rows", rows, "cols", cols, flush=True)
+            g = (torch.randn(rows * cols + 3, generator=gen, device="cuda:0") * 0.01).to(dtype)[extra & 1:][:rows * cols]
+            r = (torch.randn(rows * cols, generator=gen, device="cuda:0") * 0.002).to(dtype)
+            if cols > 1:
+                g[rows // 3] = float("inf")
+                g[rows + 7] = float("nan")
+            outs = []
+            for path in (PATH_STRIP, PATH_STRIP_PASSES):
+                qz._set_tuning(quantize_path=path)
+                outs.append(_quantize(qz, g, r, rows, cols, nbits, dtype, zt))
+            assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1]), (strips, rows)
+
+
+@pytest.mark.parametrize("dtype,rows", [(F32, 102401), (F64, 51201)])
+def test_recorded_launch_without_room_for_copies(dtype, rows):
+    """7 strips x 4000 (2000) columns: the starting buffer of 1 MB holds one copy of the records and not two, and a stream
+    under capture cannot wait for a larger one."""
+    cols = 4000 if dtype == F32 else 2000
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(rows)
+    g = torch.randn(rows * cols, generator=gen, device="cuda:0").to(dtype)
+    r = torch.zeros(rows * cols, dtype=dtype, device="cuda:0")
+    want = _quantize(MatrixQuantizerImpl.Create(0, False), g, r, rows, cols, 1, dtype, False)  # an eager launch takes the room
+    qz = MatrixQuantizerImpl.Create(0, False)
+    G, R, Q = Matrix(rows, cols, 0, g, dtype=dtype), Matrix(rows, cols, 0, r.clone(), dtype=dtype), QuantizedMatrix(rows, cols, 1, 0, dtype=dtype)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+        qz.SetMainStream(torch.cuda.current_stream().cuda_stream)
+        qz.QuantizeAsync(G, R, Q, R, False)
+    for _ in range(3):
+        R.data.zero_()
+        Q.buffer.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(Q.buffer, want[0]) and torch.equal(R.data.view(torch.uint8), want[1])
