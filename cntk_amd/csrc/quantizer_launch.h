@@ -707,6 +707,12 @@ inline hipError_t launch_on_strips(hipStream_t s, size_t rows, size_t cols, size
                     (tune.strip_may_allocate && !capturing)))
         c.copy_shift = copy_shift;
     hipError_t rc = strip_scratch_for(o, s, cols, c.strips, strip_records<E>() * strip_copies(c.strips, c.copy_shift), scratch);
+    if (rc == hipErrorOutOfMemory && c.copy_shift != 31)
+    {
+        (void) hipGetLastError();
+        c.copy_shift = 31;
+        rc = strip_scratch_for(o, s, cols, c.strips, strip_records<E>(), scratch);
+    }
     if (rc != hipSuccess)
         return rc;
     if (capturing)
