@@ -261,12 +261,16 @@ __device__ __forceinline__ bool strip_collect(const uint64_t* recs, uint32_t str
 }
 
 // The workgroup abandons its strip: every record of it says so (whichever exchange a neighbour is in, it meets the mark),
-// the host learns of it through the error word, and strip 0 counts the column.
-__device__ __forceinline__ void strip_abandon(uint64_t* recs, uint32_t records_each, uint32_t strip, uint32_t tag, const StripGeom& c,
-                                              const StripScratch& scratch)
+// the host learns of it through the error word, and strip 0 counts the column. Called by the first wavefront as one: the
+// thread that wrote a copy of the records marks it, so its two stores to one address keep their order.
+template <typename E>
+__device__ __forceinline__ void strip_abandon(uint64_t* recs, uint32_t strip, uint32_t tag, const StripGeom& c, const StripScratch& scratch)
 {
-    for (uint32_t f = 0; f < records_each * strip_copies(c.strips, c.copy_shift); ++f)
-        strip_publish(recs + (size_t) f * c.strips + strip, 0u, tag | kStripAbandoned);
+    if (threadIdx.x < strip_copies(c.strips, c.copy_shift))
+        for (uint32_t f = 0; f < strip_records<E>(); ++f)
+            strip_publish(recs + (threadIdx.x * strip_records<E>() + f) * c.strips + strip, 0u, tag | kStripAbandoned);
+    if (threadIdx.x != 0)
+        return;
     __hip_atomic_store(scratch.error, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     if (strip == 0)
         __hip_atomic_fetch_add(&scratch.header->abandoned, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -340,9 +344,9 @@ __device__ __forceinline__ E strip_exchange_stat(E stat, uint32_t column, uint32
         {
             red[0] = t;
             red_u[3] = gave_up ? 1u : 0u;
-            if (gave_up)
-                strip_abandon(recs, H * 4, strip, tag, c, scratch);
         }
+        if (gave_up)
+            strip_abandon<E>(recs, strip, tag, c, scratch);
     }
     __syncthreads();
     const E total = red[0];
@@ -389,9 +393,9 @@ __device__ __forceinline__ void strip_exchange_split(E& s0, E& s1, uint32_t& n0,
             red[1] = t1;
             red_u[2] = tn;
             red_u[3] = gave_up ? 1u : 0u;
-            if (gave_up)
-                strip_abandon(recs, H * 4, strip, tag, c, scratch);
         }
+        if (gave_up)
+            strip_abandon<E>(recs, strip, tag, c, scratch);
     }
     __syncthreads();
     s0 = red[0];
