@@ -97,8 +97,9 @@ struct BatchAbi<float>
         return family_batch_reg_quantize(nbits, zt && nbits == 1, s, ev, de, db, members, blocks, lds, threads, wide);
     }
 
-    // Fills the geometry of a member of the quantize grid; false: the matrix gets a launch of its own.
-    static bool quantize_member(const QItem& it, size_t nbits, QEntry& e, size_t& lds, uint64_t& blocks)
+    // Fills the geometry of a member of the quantize grid; false: the matrix gets a launch of its own. any_lds: the grid is resident as a whole
+    // whatever LDS its members take.
+    static bool quantize_member(const QItem& it, size_t nbits, QEntry& e, size_t& lds, uint64_t& blocks, bool any_lds)
     {
         const int path = quantize_auto_path(it.in, it.res_in, it.res_out, it.qbuf, it.rows, nbits);
         if (path == kPathTile && short_applicable(it.rows, it.cols, qwords_per_col(it.rows, nbits)))
@@ -112,7 +113,7 @@ struct BatchAbi<float>
         if (path == kPathTile)
         {
             const TileGeom t = make_tile_geom(it.rows, it.cols, nbits, 0, -1, 0);
-            if (lanes_applicable<float>(it.rows, nbits, t.gs))
+            if (lanes_member<float>(it.rows, it.cols, nbits, t.gs, tile_lds_bytes(t, 0), any_lds))
             {
                 e.kind = 14;
                 e.l = make_lanes_geom<float>(it.rows, it.cols, nbits, t.gs);
@@ -228,7 +229,7 @@ struct BatchAbi<float>
         return cntkq_stripe_reduce_async(h, it.stripes, workers, owner, it.rows, it.stripe_cols, nbits, it.stripe_res, it.q_out, it.agg_out, zt);
     }
     // the kernel family the plain call would take, so that both give the same bytes; false: does not fit the kernel
-    static bool stripe_member(const SItem& it, size_t workers, size_t nbits, SEntry& e, size_t& lds, uint64_t& blocks)
+    static bool stripe_member(const SItem& it, size_t workers, size_t nbits, SEntry& e, size_t& lds, uint64_t& blocks, bool any_lds)
     {
         if (stripe_auto_col(it.rows, it.stripe_res))
         {
@@ -274,16 +275,15 @@ struct BatchAbi<float>
         {
             e.kind = 0;
             e.t = make_tile_geom(it.rows, it.stripe_cols, nbits, 0, -1, 0);
-            if (lanes_stripe_member<float>(it.rows, it.stripe_cols, nbits, e.t.gs, workers))
+            lds = tile_lds_bytes(e.t, (uint32_t) workers);
+            blocks = (e.t.cols + e.t.cols_per_tile - 1) / e.t.cols_per_tile;
+            if (lanes_stripe_member<float>(it.rows, it.stripe_cols, nbits, e.t.gs, workers, lds, any_lds))
             {
                 e.kind = 14;
                 e.l = make_lanes_geom<float>(it.rows, it.stripe_cols, nbits, e.t.gs);
                 lds = lanes_lds_bytes<float>(e.l, workers);
                 blocks = lanes_blocks(e.l);
-                return true;
             }
-            lds = tile_lds_bytes(e.t, (uint32_t) workers);
-            blocks = (e.t.cols + e.t.cols_per_tile - 1) / e.t.cols_per_tile;
         }
         return true;
     }
@@ -431,7 +431,7 @@ __global__ __launch_bounds__(256) void table_store_kernel(TableChunk chunk, uint
 //
 // The bytes of quantize_batch_impl<float>, with its general grids (small / large LDS need) and their members' kernels; there are no
 // register grids here and LDS classes are not merged, so columns in registers on 1024 threads or with edge elements have a launch per
-// matrix and few tall columns stay staged in memory. What differs besides is where the argument table lives (the fixed device array
+// matrix, few tall columns stay staged in memory and short ones are on lanes only where that needs no more LDS than tiles. What differs besides is where the argument table lives (the fixed device array
 // `scratch`, reached through the per-device pointer) and how it gets there (as kernel arguments of table_store_kernel). Nothing on this path calls an allocator: no hipMalloc / hipHostMalloc / hipFree, no
 // host heap (the plan is built in the handle's NoAllocState), no copy that would need staging memory.
 int quantize_batch_noalloc_impl(cntkq_quantizer* h, const cntkq_quantize_item* items, size_t count, size_t nbits, int zero_threshold_for_1bit)
@@ -495,7 +495,7 @@ int quantize_batch_noalloc_impl(cntkq_quantizer* h, const cntkq_quantize_item* i
             std::memset(&e, 0, sizeof e);
             size_t lds = 0;
             uint64_t blocks = 0;
-            if (A::quantize_member(it, nbits, e, lds, blocks))
+            if (A::quantize_member(it, nbits, e, lds, blocks, false))
                 members[lds <= kBatchSmallLds ? 0 : 1]++;
         }
         const bool single = members[0] + members[1] == 1; // a grid of its own is nothing to share: plain launch
@@ -525,7 +525,7 @@ int quantize_batch_noalloc_impl(cntkq_quantizer* h, const cntkq_quantize_item* i
                 std::memset(&en, 0, sizeof en);
                 size_t lds = 0;
                 uint64_t blocks = 0;
-                if (!A::quantize_member(it, nbits, en, lds, blocks) || (lds <= kBatchSmallLds ? 0 : 1) != cls)
+                if (!A::quantize_member(it, nbits, en, lds, blocks, false) || (lds <= kBatchSmallLds ? 0 : 1) != cls)
                     continue;
                 en.g = it.in;
                 en.r_in = it.res_in;
@@ -552,7 +552,7 @@ int quantize_batch_noalloc_impl(cntkq_quantizer* h, const cntkq_quantize_item* i
             Entry en;
             size_t lds = 0;
             uint64_t blocks = 0;
-            if (single || !A::quantize_member(it, nbits, en, lds, blocks))
+            if (single || !A::quantize_member(it, nbits, en, lds, blocks, false))
                 st.own[st.own_count++] = i;
         }
         st.entries_bytes = entries_bytes;
@@ -1019,6 +1019,13 @@ int cntkq_debug_stripe_shares_register_grid(size_t rows, size_t cols, size_t nbi
     size_t lds = 0;
     uint64_t blocks = 0;
     return BatchAbi<float>::stripe_register_member(it, workers, nbits, e, lds, blocks) != kBatchOwnLaunch ? 1 : 0;
+}
+
+// The kind of member (QuantizeBatchEntry, StripeBatchEntry) that a matrix or stripe of whole aligned pieces is in the general grids, and its LDS;
+// -1: none of them. workers 0: quantized.
+int cntkq_debug_set_member(size_t rows, size_t cols, size_t nbits, size_t workers, size_t* lds)
+{
+    return debug_set_member<float>(rows, cols, nbits, workers, lds);
 }
 
 size_t cntkq_debug_staged_max_rows(size_t nbits)

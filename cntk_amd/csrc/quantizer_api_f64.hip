@@ -56,7 +56,7 @@ struct BatchAbi<double>
 
     // members of the general grid are runs of column tiles, small matrices of the element-wise register kernel among them, which run the
     // tile body (the same bytes); columns on 1024 threads are members of the register grid below, the rest gets launches of its own
-    static bool quantize_member(const QItem& it, size_t nbits, QEntry& e, size_t& lds, uint64_t& blocks)
+    static bool quantize_member(const QItem& it, size_t nbits, QEntry& e, size_t& lds, uint64_t& blocks, bool any_lds)
     {
         const int path = f64::quantize_auto_path(it.in, it.res_in, it.res_out, it.rows, nbits);
         if (path != kPathTile && !(path == kPathRegScalar && it.rows * it.cols < kOwnLaunchElements))
@@ -66,7 +66,7 @@ struct BatchAbi<double>
         if (lds > f64::kMaxLdsBytes)
             return false;
         blocks = (e.t.cols + e.t.cols_per_tile - 1) / e.t.cols_per_tile;
-        if (path == kPathTile && lanes_applicable<double>(it.rows, nbits, e.t.gs))
+        if (path == kPathTile && lanes_member<double>(it.rows, it.cols, nbits, e.t.gs, lds, any_lds))
         {
             e.kind = 14;
             e.l = make_lanes_geom<double>(it.rows, it.cols, nbits, e.t.gs);
@@ -152,14 +152,14 @@ struct BatchAbi<double>
         return cntkq_stripe_reduce_async_f64(h, it.stripes, workers, owner, it.rows, it.stripe_cols, nbits, it.stripe_res, it.q_out, it.agg_out,
                                              zt);
     }
-    static bool stripe_member(const SItem& it, size_t workers, size_t nbits, SEntry& e, size_t& lds, uint64_t& blocks)
+    static bool stripe_member(const SItem& it, size_t workers, size_t nbits, SEntry& e, size_t& lds, uint64_t& blocks, bool any_lds)
     {
         e.t = f64::make_tile_geom(it.rows, it.stripe_cols, nbits, 0); // the plain call's geometry: same bytes
         lds = f64::tile_lds_bytes(e.t, (uint32_t) workers);
         blocks = (e.t.cols + e.t.cols_per_tile - 1) / e.t.cols_per_tile;
         if (lds > f64::kMaxLdsBytes)
             return false;
-        if (lanes_stripe_member<double>(it.rows, it.stripe_cols, nbits, e.t.gs, workers))
+        if (lanes_stripe_member<double>(it.rows, it.stripe_cols, nbits, e.t.gs, workers, lds, any_lds))
         {
             e.kind = 14;
             e.l = make_lanes_geom<double>(it.rows, it.stripe_cols, nbits, e.t.gs);
@@ -210,6 +210,11 @@ int cntkq_debug_decoder_f64(size_t rows, size_t cols, size_t nbits, int packed_o
 int cntkq_debug_short_columns_f64(size_t rows, size_t cols, size_t nbits)
 {
     return f64::short_applicable64(rows, cols, f64::qwords_per_col(rows, nbits)) ? 1 : 0;
+}
+
+int cntkq_debug_set_member_f64(size_t rows, size_t cols, size_t nbits, size_t workers, size_t* lds)
+{
+    return debug_set_member<double>(rows, cols, nbits, workers, lds);
 }
 
 size_t cntkq_qwords_per_col_f64(size_t rows, size_t nbits)

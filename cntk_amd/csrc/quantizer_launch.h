@@ -208,12 +208,10 @@ inline bool lanes_stripe_applicable(size_t rows, size_t cols, size_t nbits, uint
     return n <= (F ? (rows >= 32 ? 1024 * 1024 : 128 * 1024) : (rows >= 24 ? 512 * 1024 : 64 * 1024));
 }
 
-// ... as members of a set's launch, among which a stripe's size says little about how full the device is: a single worker's (ResNet-50's at 1
-// bit with one worker 50.9 -> 49.2 us, at 4 bits with eight 92 -> 96)
-template <typename E>
-inline bool lanes_stripe_member(size_t rows, size_t cols, size_t nbits, uint32_t lanes, size_t workers)
+// Workgroups of 256 threads that a compute unit's LDS lets in: it is given out in blocks of 1280 bytes, 128 of them.
+inline uint32_t lds_workgroups(size_t lds)
 {
-    return workers == 1 && lanes_stripe_applicable<E>(rows, cols, nbits, lanes, workers);
+    return std::min<uint32_t>(8u, 128u / (uint32_t) std::max<size_t>(1, (lds + 1279) / 1280));
 }
 
 template <typename E>
@@ -237,6 +235,27 @@ inline LanesGeom make_lanes_geom(size_t rows, size_t cols, size_t nbits, uint32_
     t.rec_words = (columns * (t.nq + 2) + 3) & ~3u;
     t.qcol = (uint64_t) (2 + t.nq) * sizeof(E);
     return t;
+}
+
+// Short columns of a set to be quantized: all workgroups of a grid are given the LDS of its largest member, and members above 20 KB may
+// cost a launch of their own. The records in LDS, which the tile kernels need at 1 and 2 bits only, take many heights across that
+// line (147 rows at 4 bits 19.1 -> 21.6 KB, 512 at 8 bits 16.7 -> 20.6, 147 at 16 bits 19.1 -> 28.6). There the member is a tile, unless all
+// of the grid is resident at once anyway (any_lds). Lanes everywhere / by this rule, us: ResNet-50 at 4, 8, 16 bits 57.0 / 57.0, 60.6 / 59.1, 71.6 / 63.3,
+// without allocation 63.2 / 56.4, 63.7 / 57.3, 70.3 / 62.0; the stripes of one worker 53.1 / 53.6, 60.9 / 58.7, 75.8 / 66.1.
+template <typename E>
+inline bool lanes_member(size_t rows, size_t cols, size_t nbits, uint32_t lanes, size_t tile_lds, bool any_lds)
+{
+    return lanes_applicable<E>(rows, nbits, lanes) &&
+           (any_lds || lds_workgroups(lanes_lds_bytes<E>(make_lanes_geom<E>(rows, cols, nbits, lanes), 0)) >= lds_workgroups(tile_lds));
+}
+
+// ... of a set's stripes, among which a stripe's size says little about how full the device is: a single worker's (ResNet-50's at 1
+// bit with one worker 50.9 -> 49.2 us, at 4 bits with eight 92 -> 96)
+template <typename E>
+inline bool lanes_stripe_member(size_t rows, size_t cols, size_t nbits, uint32_t lanes, size_t workers, size_t tile_lds, bool any_lds)
+{
+    return workers == 1 && lanes_stripe_applicable<E>(rows, cols, nbits, lanes, workers) &&
+           (any_lds || lds_workgroups(lanes_lds_bytes<E>(make_lanes_geom<E>(rows, cols, nbits, lanes), workers)) >= lds_workgroups(tile_lds));
 }
 
 inline uint32_t lanes_blocks(const LanesGeom& t)

@@ -99,17 +99,20 @@ def test_stripe_reduce(dtype, nbits, zt, workers):
                 assert np.array_equal(_bytes(x), _bytes(y)), (what, rows, cols)
 
 
-@pytest.mark.parametrize("dtype,nbits,zt", [(F32, 1, True), (F32, 4, False), (F64, 2, False)])
-def test_members_of_a_set(dtype, nbits, zt):
-    """Quantized and reduced (one worker) in one call each: the bytes of the tile kernels, also where the owner's result replaces its stripe."""
+@pytest.mark.parametrize("full", [False, True])
+@pytest.mark.parametrize("dtype,nbits,zt", [(F32, 1, True), (F32, 4, False), (F32, 16, False), (F64, 2, False), (F64, 16, False)])
+def test_members_of_a_set(dtype, nbits, zt, full):
+    """Quantized and reduced (one worker) in one call each: the bytes of the tile kernels, also where the owner's result replaces its stripe. A
+    set that is resident as a whole has all of these members on lanes, one that fills the device (full) those whose LDS is no more than
+    their tiles'."""
     plain, tile = MatrixQuantizerImpl.Create(0, False), MatrixQuantizerImpl.Create(0, False)
     tile._set_tuning(quantize_path=PATH_TILE)
     gen = torch.Generator(device="cuda:0")
     gen.manual_seed(datagen.case_seed(nbits) + 1)
     kw = dict(dtype=dtype)
     items, want, stripes = [], [], []
-    for n, rows in enumerate(ROWS[dtype]):
-        cols = COLS[n % len(COLS)]
+    for n, rows in enumerate(ROWS[dtype] + [128] * full):
+        cols = COLS[n % len(COLS)] if n < len(ROWS[dtype]) else 80000
         g, r = _make(rows, cols, dtype, gen, 0)
         G = Matrix(rows, cols, 0, g, **kw)
         both = []

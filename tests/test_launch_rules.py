@@ -1,4 +1,6 @@
 """Which kernel a call takes, on both sides of the lines that the rules draw. The rules are host code: no device is needed."""
+import ctypes
+
 import pytest
 
 import cntk_amd
@@ -112,3 +114,47 @@ def test_heights_of_few_tall_columns():
     """Staged in memory beside 8 M elements: 8192 rows 22.9 us, 26.1 with a register grid of their own; 14336 rows 33.0 and 27.6."""
     L = cntk_amd.lib()
     assert [L.cntkq_debug_staged_max_rows(b) for b in (1, 2, 4, 8, 16)] == [8192, 8192, 8192, 10240, 10240]
+
+
+TILES, LANES = 0, 14
+SMALL_LDS = 20480  # eight workgroups in a compute unit; a set's members above it may get a launch of their own
+
+
+def member(rows, nbits, workers=0, double=0, cols=100):
+    """(kind, bytes of LDS) of a member of a set's general grid."""
+    L = cntk_amd.lib()
+    lds = ctypes.c_size_t()
+    kind = (L.cntkq_debug_set_member_f64 if double else L.cntkq_debug_set_member)(rows, cols, nbits, workers, ctypes.byref(lds))
+    return kind, lds.value
+
+
+def tile_lds(rows, nbits, workers, double):
+    """A column tile: at most 5120 floats or 2048 doubles, a few lanes' scratch, QWords where several threads share one, the workers' levels."""
+    threads, most, word = (256, 2048, 64) if double else (256, 5120, 32)
+    lanes = 8
+    while lanes < threads and (rows > lanes * 32 or threads // lanes * rows > most):
+        lanes *= 2
+    columns, qwords = threads // lanes, -(-rows * nbits // word)
+    values = (columns * rows + 1) & ~1 if double else (columns * rows + 7) & ~3
+    words = columns * qwords if nbits <= (4 if double else 2) else 0
+    return ((74 if double else 76) + values + words + 2 * workers * columns) * (8 if double else 4)
+
+
+@pytest.mark.parametrize("double,workers", [(0, 0), (0, 1), (1, 0), (1, 1)])
+def test_short_members_of_a_set_stay_in_their_grid(double, workers):
+    """A short column is on lanes only where a compute unit holds as many of its workgroups as of the tiles that the member was before: 147 rows at 4 bits
+    need 19.1 KB as tiles and 21.6 on lanes, and everything else of the grid would be given those too."""
+    for nbits in (1, 2, 4, 8, 16, 32):
+        for rows in range(17, 513 if double else 1024):
+            kind, lds = member(rows, nbits, workers, double)
+            tiles = tile_lds(rows, nbits, workers, double)
+            assert kind in (TILES, LANES)
+            assert kind == LANES or lds == tiles, (rows, nbits)
+            assert 163840 // lds >= min(8, 163840 // tiles) and (lds <= SMALL_LDS or tiles > SMALL_LDS), (rows, nbits, lds, tiles)
+
+
+def test_short_members_on_lanes():
+    """ResNet-50's heights (64, 128, 147, 256, 512, 576) and an odd one."""
+    lanes = {rows: [b for b in (1, 2, 4, 8, 16) if member(rows, b)[0] == LANES] for rows in (33, 64, 128, 147, 256, 512, 576)}
+    assert lanes == {33: [1, 2, 4, 8, 16], 64: [1, 2, 4, 8, 16], 128: [1, 2, 4], 147: [1, 2], 256: [1, 2, 4], 512: [1, 2, 4], 576: [1, 2]}
+    assert [b for b in (1, 2, 4, 8, 16) if member(147, b, 1)[0] == LANES] == [1, 2] and member(147, 1, 2)[0] == TILES
