@@ -149,10 +149,12 @@ struct BatchAbi<float>
                 e.kind = it.rows == 1024 ? 2 : (it.rows == 2048 ? 3 : 4);
                 lds = it.rows == 1024 ? col_lds_bytes<1>() : (it.rows == 2048 ? col_lds_bytes<2>() : col_lds_bytes<4>());
             }
-            else if (path == kPathReg && e.kind == 1)
+            else if (path == kPathReg && (e.kind == 1 || e.kind == 5))
             {
                 // what the plain call runs for this matrix, where a thread holds at most 6 pieces (6144 rows): the column in
-                // registers, with the slots dealt as the plain call deals them (same bytes as the LDS body either way)
+                // registers, with the slots dealt as the plain call deals them (same bytes as the LDS bodies). Few columns of those heights
+                // were staged in memory: three passes over it, the tail of the grid since the short members next to them ask for all
+                // their values at once (20 columns of 5856 rows beside 15 M elements: 51.1 us with tiles, 53.3 with lanes, 50.7 so).
                 const RegGeom r = make_reg_geom(it.rows, nbits, kTileThreads, line_shift);
                 const uint32_t per = (r.pieces + (r.line_shift ? 7u : 0u) + kTileThreads - 1) / kTileThreads;
                 if (per <= 6)

@@ -38,6 +38,12 @@ def test_quantize(shapes, nbits, zt):
     _check_quantize(shapes, nbits, zt, torch.float32)
 
 
+@pytest.mark.parametrize("nbits,zt", [(1, False), (1, True), (4, False), (16, False)])
+def test_quantize_of_few_columns_of_six_pieces(nbits, zt):
+    """At most 32 columns of 5124 to 6144 rows (6140: not on lines, so one piece more per thread) are in registers, the next height is staged in memory."""
+    _check_quantize([(5124, 1), (5632, 32), (6112, 7), (6140, 5), (6144, 20), (6176, 32)] + SMALL, nbits, zt, torch.float32)
+
+
 @pytest.mark.parametrize("nbits", [1, 8])
 def test_quantize_of_few_tall_columns_alone(nbits):
     """A large set made of nothing but the few tall columns that would be staged in memory: there is nothing else to hide them, so they

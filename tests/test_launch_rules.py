@@ -116,7 +116,7 @@ def test_heights_of_few_tall_columns():
     assert [L.cntkq_debug_staged_max_rows(b) for b in (1, 2, 4, 8, 16)] == [8192, 8192, 8192, 10240, 10240]
 
 
-TILES, LANES = 0, 14
+TILES, COLUMNS, STAGED, REGISTERS_6, LANES = 0, 1, 5, 7, 14
 SMALL_LDS = 20480  # eight workgroups in a compute unit; a set's members above it may get a launch of their own
 
 
@@ -158,3 +158,12 @@ def test_short_members_on_lanes():
     lanes = {rows: [b for b in (1, 2, 4, 8, 16) if member(rows, b)[0] == LANES] for rows in (33, 64, 128, 147, 256, 512, 576)}
     assert lanes == {33: [1, 2, 4, 8, 16], 64: [1, 2, 4, 8, 16], 128: [1, 2, 4], 147: [1, 2], 256: [1, 2, 4], 512: [1, 2, 4], 576: [1, 2]}
     assert [b for b in (1, 2, 4, 8, 16) if member(147, b, 1)[0] == LANES] == [1, 2] and member(147, 1, 2)[0] == TILES
+
+
+@pytest.mark.parametrize("nbits", [1, 2, 4, 8, 16])
+def test_few_columns_of_a_set_that_registers_hold(nbits):
+    """Up to six pieces for each of 256 threads: in registers however few there are; above, at most 32 columns are staged in memory."""
+    for cols in (1, 32, 33, 400):
+        assert member(5632, nbits, cols=cols)[0] == member(6144, nbits, cols=cols)[0] == REGISTERS_6
+        assert member(6144, nbits, cols=cols)[1] <= SMALL_LDS
+    assert member(6176, nbits, cols=32)[0] == STAGED
