@@ -1030,6 +1030,14 @@ int cntkq_debug_set_member(size_t rows, size_t cols, size_t nbits, size_t worker
     return debug_set_member<float>(rows, cols, nbits, workers, lds);
 }
 
+// Whether a plain call that the tile kernels could take runs on lanes (workers 0: quantize)
+int cntkq_debug_lanes(size_t rows, size_t cols, size_t nbits, size_t workers)
+{
+    const TileGeom t = make_tile_geom(rows, cols, nbits, 0, -1, 0);
+    return (workers == 0 ? lanes_applicable<float>(rows, cols, nbits, t.gs)
+                         : lanes_stripe_applicable<float>(rows, cols, nbits, t.gs, workers, tile_lds_bytes(t, (uint32_t) workers))) ? 1 : 0;
+}
+
 size_t cntkq_debug_staged_max_rows(size_t nbits)
 {
     return staged_max_rows(nbits);

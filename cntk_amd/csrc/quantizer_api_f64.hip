@@ -212,6 +212,13 @@ int cntkq_debug_short_columns_f64(size_t rows, size_t cols, size_t nbits)
     return f64::short_applicable64(rows, cols, f64::qwords_per_col(rows, nbits)) ? 1 : 0;
 }
 
+int cntkq_debug_lanes_f64(size_t rows, size_t cols, size_t nbits, size_t workers)
+{
+    const f64::TileGeom t = f64::make_tile_geom(rows, cols, nbits, 0);
+    return (workers == 0 ? lanes_applicable<double>(rows, cols, nbits, t.gs)
+                         : lanes_stripe_applicable<double>(rows, cols, nbits, t.gs, workers, f64::tile_lds_bytes(t, (uint32_t) workers))) ? 1 : 0;
+}
+
 int cntkq_debug_set_member_f64(size_t rows, size_t cols, size_t nbits, size_t workers, size_t* lds)
 {
     return debug_set_member<double>(rows, cols, nbits, workers, lds);

@@ -183,29 +183,21 @@ inline uint32_t short_blocks(const ShortGeom& t)
 }
 
 // Columns that a few lanes of one wavefront hold, as many as the tile kernels give a column threads (lanes: what make_tile_geom says); the same
-// bytes. Quantize: at every height and size. Tile kernel / this, 36 heights of 17 to 1279 rows: 1.2 to 1.6 at 100000 elements, 1.0 to 1.5
-// at 1 M, 0.98 to 1.2 at 10 M (1.8 at 32 rows); doubles 1.2 to 1.4, 1.06 to 1.4, 0.95 to 1.4.
+// bytes.
 template <typename E>
-inline bool lanes_applicable(size_t rows, size_t nbits, uint32_t lanes)
+inline bool lanes_hold(size_t rows, size_t nbits, uint32_t lanes)
 {
     return rows > kShortMaxRows && nbits < 8 * sizeof(E) && lanes <= 64 && (rows + lanes - 1) / lanes <= (sizeof(E) == 4 ? kLanesMaxChain : 8u);
 }
 
-// ... in the stripe reduction, where the decoding is the same work for the tile kernels' threads, and a tile's larger share of a compute
-// unit's LDS does not matter once its loads are under way. One worker: 1.04 to 1.6 at 100000 elements, 0.94 to 2.2 above that, but below 32
-// rows at 1 M 0.84 to 1.0. Eight workers: 1.0 to 1.3 at 100000, 0.94 to 1.3 at 1 M, 0.85 to 1.2 at 5 M; below 32 rows 0.94 to 1.1, 0.75 to 1.0
-// and 0.8 to 1.1. Doubles with one worker 1.1 to 1.6, 1.05 to 1.5, 0.9 to 1.8; with eight 0.97 to 1.4, 0.95 to 1.5, 0.73 to 1.8, below 24 rows at
-// 500000 0.81 to 1.3.
+// Quantize. Tile kernel / this at 1, 2, 4, 8, 16 bits, 24 heights of 17 to 1279 rows: 1.1 to 1.6 at 100000 elements, 0.98 to 1.55 at 1 M, 0.97 to
+// 1.8 at 10 M (below 0.99 at five of 360 points). Doubles at 1, 4, 16, 32 bits, 17 to 512 rows: 1.08 to 1.45 at 50000, 1.02 to 1.35 at 500000,
+// 0.98 to 1.4 at 5 M, except that columns below 32 rows at 8 bits and more, whose records are a third of them and more, take 0.92 to 1.01 from
+// 2 M elements on: the tile kernels keep those.
 template <typename E>
-inline bool lanes_stripe_applicable(size_t rows, size_t cols, size_t nbits, uint32_t lanes, size_t workers)
+inline bool lanes_applicable(size_t rows, size_t cols, size_t nbits, uint32_t lanes)
 {
-    if (!lanes_applicable<E>(rows, nbits, lanes))
-        return false;
-    constexpr bool F = sizeof(E) == 4;
-    const size_t n = rows * cols;
-    if (workers <= 2)
-        return !F || rows >= 32 || n <= 256 * 1024;
-    return n <= (F ? (rows >= 32 ? 1024 * 1024 : 128 * 1024) : (rows >= 24 ? 512 * 1024 : 64 * 1024));
+    return lanes_hold<E>(rows, nbits, lanes) && (sizeof(E) == 4 || rows >= 32 || nbits < 8 || rows * cols <= 1024 * 1024);
 }
 
 // Workgroups of 256 threads that a compute unit's LDS lets in: it is given out in blocks of 1280 bytes, 128 of them.
@@ -237,6 +229,40 @@ inline LanesGeom make_lanes_geom(size_t rows, size_t cols, size_t nbits, uint32_
     return t;
 }
 
+// In the stripe reduction the decoding is the same work for the tile kernels' threads, eight bit positions of a QWord each, and lanes without
+// one of their own wait for it: the more workers and bits, the less there is to gain, and what is lost grows with the number of workers
+// (float / double columns, 100 K to 1 M elements: 0.74 to 1.1 with 16 workers at 4 to 16 bits, 0.64 to 1.0 with 64 at 1 and 2; 0.65 to 1.0 with 32). Tile
+// kernel / this wherever the rule says yes (3800 points: 1 to 16 workers, 1 to 32 bits, 17 to 1279 rows, 20000 to 8 M elements): 0.975 to 2.2, 1.15 in the median.
+// Beyond it, float: below 32 rows 0.84 to 1.0 at 1 M elements; from 1 M on with one and two workers 0.82 to 1.2 where a compute unit holds fewer
+// workgroups than tiles for the records' LDS, and with two 0.95 to 1.05 at 4 bits and more where a lane holds few of the elements it
+// could (65, 161, 321, 641 rows); with eight at 8 bits 0.89 to 1.0 below 64 rows. Doubles: 0.92 to 1.2 with eight at 8 bits, 0.90 to 1.1 at 16 and 32.
+template <typename E>
+inline bool lanes_stripe_applicable(size_t rows, size_t cols, size_t nbits, uint32_t lanes, size_t workers, size_t tile_lds)
+{
+    if (!lanes_hold<E>(rows, nbits, lanes))
+        return false;
+    const size_t n = rows * cols, K = 1024;
+    if (sizeof(E) == 8)
+    {
+        if (workers <= 2)
+            return true;
+        if (workers <= 4)
+            return n <= (rows >= 24 ? 512 * K : 64 * K);
+        return n <= (rows >= 32 ? 512 * K : 64 * K) && workers <= (nbits <= 4 ? 8u : (nbits == 8 ? 6u : 4u));
+    }
+    if (workers <= 2)
+    {
+        if (n <= 256 * K || (n <= K * K && rows >= 32))
+            return true;
+        const LanesGeom t = make_lanes_geom<E>(rows, cols, nbits, lanes);
+        return rows >= 32 && lds_workgroups(lanes_lds_bytes<E>(t, workers)) >= lds_workgroups(tile_lds) &&
+               (workers == 1 || nbits <= 2 || 3 * rows >= 2 * (size_t) lanes * t.chain);
+    }
+    if (rows >= 64)
+        return n <= K * K && workers <= (nbits == 1 ? 16u : (nbits == 2 ? 12u : (nbits == 4 ? 8u : 6u)));
+    return n <= (rows >= 32 ? 512 * K : 128 * K) && workers <= (nbits <= 4 ? 8u : 5u);
+}
+
 // Short columns of a set to be quantized: all workgroups of a grid are given the LDS of its largest member, and members above 20 KB may
 // cost a launch of their own. The records in LDS, which the tile kernels need at 1 and 2 bits only, take many heights across that
 // line (147 rows at 4 bits 19.1 -> 21.6 KB, 512 at 8 bits 16.7 -> 20.6, 147 at 16 bits 19.1 -> 28.6). There the member is a tile, unless all
@@ -245,7 +271,7 @@ inline LanesGeom make_lanes_geom(size_t rows, size_t cols, size_t nbits, uint32_
 template <typename E>
 inline bool lanes_member(size_t rows, size_t cols, size_t nbits, uint32_t lanes, size_t tile_lds, bool any_lds)
 {
-    return lanes_applicable<E>(rows, nbits, lanes) &&
+    return lanes_applicable<E>(rows, cols, nbits, lanes) &&
            (any_lds || lds_workgroups(lanes_lds_bytes<E>(make_lanes_geom<E>(rows, cols, nbits, lanes), 0)) >= lds_workgroups(tile_lds));
 }
 
@@ -254,7 +280,7 @@ inline bool lanes_member(size_t rows, size_t cols, size_t nbits, uint32_t lanes,
 template <typename E>
 inline bool lanes_stripe_member(size_t rows, size_t cols, size_t nbits, uint32_t lanes, size_t workers, size_t tile_lds, bool any_lds)
 {
-    return workers == 1 && lanes_stripe_applicable<E>(rows, cols, nbits, lanes, workers) &&
+    return workers == 1 && lanes_stripe_applicable<E>(rows, cols, nbits, lanes, workers, tile_lds) &&
            (any_lds || lds_workgroups(lanes_lds_bytes<E>(make_lanes_geom<E>(rows, cols, nbits, lanes), workers)) >= lds_workgroups(tile_lds));
 }
 
@@ -883,7 +909,7 @@ inline hipError_t launch_quantize(hipStream_t s, LaunchEvents ev, const float* g
         if (tune.quantize_path == kPathAuto && short_applicable(rows, cols, qwords_per_col(rows, nbits)))
             return family_short_quantize(nbits, zt, s, ev, g, r_in, r_out, qc, make_short_geom(rows, cols, qwords_per_col(rows, nbits), qcol_bytes(nbits, rows), sizeof(float)));
         const TileGeom t = make_tile_geom(rows, cols, nbits, tune.tile_gs, tune.tile_stage, tune.tile_threads);
-        if (!tile_geometry_forced(tune) && lanes_applicable<float>(rows, nbits, t.gs))
+        if (!tile_geometry_forced(tune) && lanes_applicable<float>(rows, cols, nbits, t.gs))
             return family_lanes_quantize(nbits, zt, s, ev, g, r_in, r_out, qc, make_lanes_geom<float>(rows, cols, nbits, t.gs));
         return family_tile_quantize(nbits, zt, s, ev, g, r_in, r_out, qc, t);
     }
@@ -1007,7 +1033,7 @@ inline hipError_t launch_stripe_reduce(hipStream_t s, LaunchEvents ev, const Str
     // Same tile geometry as launch_quantize would use for a matrix of this height, so that the statistics are summed in
     // the same order and the fused call gives the bytes of the reference's unquantize ... quantize call sequence.
     const TileGeom t = make_tile_geom(rows, cols, nbits, tune.tile_gs, tune.tile_stage, tune.tile_threads);
-    if (!tile_geometry_forced(tune) && lanes_stripe_applicable<float>(rows, cols, nbits, t.gs, src.workers))
+    if (!tile_geometry_forced(tune) && lanes_stripe_applicable<float>(rows, cols, nbits, t.gs, src.workers, tile_lds_bytes(t, src.workers)))
         return family_lanes_stripe(nbits, zt, s, ev, src, stripe_res, static_cast<char*>(q_out), agg_out, make_lanes_geom<float>(rows, cols, nbits, t.gs));
     return family_tile_stripe(nbits, zt, s, ev, src, stripe_res, static_cast<char*>(q_out), agg_out, t);
 }

@@ -303,7 +303,7 @@ inline hipError_t launch_quantize(hipStream_t s, LaunchEvents ev, const double* 
         const TileGeom t = make_tile_geom(rows, cols, nbits, tune.tile_gs);
         if (tile_lds_bytes(t, 0) > kMaxLdsBytes)
             return hipErrorInvalidValue;
-        if (!tile_geometry_forced(tune) && lanes_applicable<double>(rows, nbits, t.gs))
+        if (!tile_geometry_forced(tune) && lanes_applicable<double>(rows, cols, nbits, t.gs))
             return family_lanes_quantize(nbits, zt, s, ev, g, r_in, r_out, qc, make_lanes_geom<double>(rows, cols, nbits, t.gs));
         return dispatch_nbits64<TileLauncher>(nbits, zt, s, ev, g, r_in, r_out, qc, t);
     }
@@ -406,7 +406,7 @@ inline hipError_t launch_stripe_reduce(hipStream_t s, LaunchEvents ev, const Str
     const TileGeom t = make_tile_geom(rows, cols, nbits, tune.tile_gs);
     if (tile_lds_bytes(t, src.workers) > kMaxLdsBytes)
         return hipErrorInvalidValue;
-    if (!tile_geometry_forced(tune) && lanes_stripe_applicable<double>(rows, cols, nbits, t.gs, src.workers))
+    if (!tile_geometry_forced(tune) && lanes_stripe_applicable<double>(rows, cols, nbits, t.gs, src.workers, tile_lds_bytes(t, src.workers)))
         return family_lanes_stripe(nbits, zt, s, ev, src, stripe_res, static_cast<char*>(q_out), agg_out,
                                    make_lanes_geom<double>(rows, cols, nbits, t.gs));
     return dispatch_nbits64<StripeLauncher>(nbits, zt, s, ev, src, stripe_res, static_cast<char*>(q_out), agg_out, t);

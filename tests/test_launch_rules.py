@@ -167,3 +167,47 @@ def test_few_columns_of_a_set_that_registers_hold(nbits):
         assert member(5632, nbits, cols=cols)[0] == member(6144, nbits, cols=cols)[0] == REGISTERS_6
         assert member(6144, nbits, cols=cols)[1] <= SMALL_LDS
     assert member(6176, nbits, cols=32)[0] == STAGED
+
+
+def on_lanes(rows, n, nbits, workers=0, double=0):
+    L = cntk_amd.lib()
+    return bool((L.cntkq_debug_lanes_f64 if double else L.cntkq_debug_lanes)(rows, max(1, n // rows), nbits, workers))
+
+
+def test_quantize_on_lanes():
+    for nbits in (1, 2, 4, 8, 16):
+        for rows in (17, 33, 161, 512, 1023, 1280):
+            assert on_lanes(rows, 10 ** 4, nbits) and on_lanes(rows, 4 * 10 ** 7, nbits)
+        assert not on_lanes(16, 10 ** 6, nbits) and not on_lanes(1281, 10 ** 6, nbits)
+    assert not on_lanes(512, 10 ** 6, 32)
+    for nbits in (1, 2, 4, 8, 16, 32):  # doubles: 17 x 294117 at 16 bits 28.0 us with tiles, 30.2 on lanes
+        assert on_lanes(17, 10 ** 6, nbits, double=1) and on_lanes(32, 10 ** 7, nbits, double=1) and on_lanes(512, 10 ** 7, nbits, double=1)
+        assert on_lanes(31, 2 * 10 ** 6, nbits, double=1) == (nbits < 8) and not on_lanes(513, 10 ** 6, nbits, double=1)
+
+
+@pytest.mark.parametrize("rows,n,nbits,most", [
+    (64, 10 ** 6, 1, 16), (512, 10 ** 5, 1, 16), (576, 10 ** 6, 2, 12), (147, 10 ** 6, 4, 8), (1023, 10 ** 6, 8, 6), (512, 10 ** 5, 16, 6),
+    (63, 500000, 4, 8), (32, 500000, 8, 5), (31, 120000, 2, 8), (17, 120000, 16, 5), (512, 1100000, 1, 2), (63, 600000, 1, 2), (31, 140000, 1, 2)])
+def test_stripes_on_lanes_by_workers(rows, n, nbits, most):
+    """Up to this many workers (512 x 1953 at 4 bits: 1.17 times as fast with 8 workers, 0.95 with 16; 32 x 31250 0.87 and 0.74)."""
+    assert [k for k in range(1, 65) if on_lanes(rows, n, nbits, k)] == list(range(1, most + 1))
+
+
+def test_large_stripes_on_lanes():
+    """One and two workers above 1 M elements: with no fewer workgroups to a compute unit than tiles have (319 x 25078 at 16 bits: 28.8 us with tiles, 33.8 on
+    lanes), two of them at 4 bits and more with most of a lane's elements there (65 x 46153 at 8 bits: 14.3 and 15.1 us)."""
+    n = 8 * 10 ** 6
+    for nbits in (1, 2):
+        assert all(on_lanes(rows, n, nbits, k) for rows in (32, 65, 161, 512, 641) for k in (1, 2))
+    for rows, nbits in ((319, 8), (1279, 4), (513, 16), (129, 16)):
+        assert not on_lanes(rows, n, nbits, 1) and not on_lanes(rows, n, nbits, 2) and on_lanes(rows, 10 ** 6, nbits, 2)
+    for rows in (65, 161, 321, 641):
+        assert on_lanes(rows, n, 4, 1) and not on_lanes(rows, n, 4, 2)
+    assert on_lanes(256, n, 4, 2) and not on_lanes(31, 300000, 1, 1) and on_lanes(31, 250000, 1, 1)
+
+
+@pytest.mark.parametrize("rows,n,nbits,most", [
+    (32, 500000, 4, 8), (512, 10 ** 5, 8, 6), (512, 10 ** 5, 16, 4), (200, 500000, 32, 4), (24, 500000, 1, 4), (24, 60000, 1, 8), (23, 10 ** 5, 1, 2),
+    (512, 600000, 1, 2), (17, 10 ** 7, 32, 2)])
+def test_stripes_of_doubles_on_lanes_by_workers(rows, n, nbits, most):
+    assert [k for k in range(1, 65) if on_lanes(rows, n, nbits, k, double=1)] == list(range(1, most + 1))
