@@ -111,6 +111,7 @@ def lib():
             getattr(L, name).argtypes = [_vp, _sz, _sz, _sz, ctypes.c_int]
         L.cntkq_debug_set_tuning.argtypes = [_vp, ctypes.c_int, ctypes.c_uint, ctypes.c_uint, ctypes.c_int, ctypes.c_int]
         L.cntkq_debug_set_strip_spin_limit.argtypes = [_vp, ctypes.c_uint]
+        L.cntkq_debug_set_strip_scratch_limit.argtypes = [_vp, _sz]
         L.cntkq_debug_strip_max_strips.argtypes = [_vp, _sz, ctypes.c_int]
         L.cntkq_debug_strip_max_strips.restype = ctypes.c_uint
         L.cntkq_debug_strip_max_strips_f64.argtypes = [_vp, _sz, ctypes.c_int]
@@ -607,6 +608,9 @@ class MatrixQuantizerImpl:
 
     def _set_strip_spin_limit(self, limit):
         _check(lib().cntkq_debug_set_strip_spin_limit(self._h, limit))
+
+    def _set_strip_scratch_limit(self, nbytes):
+        _check(lib().cntkq_debug_set_strip_scratch_limit(self._h, nbytes))
 
     def _strip_max_strips(self, nbits, zero_threshold_for_1bit=False, dtype=torch.float32):
         """Most strips per column that the strip kernels take on this device at this bit width (0: none)."""

@@ -994,6 +994,15 @@ int cntkq_debug_set_strip_spin_limit(cntkq_quantizer* h, unsigned limit)
     return CNTKQ_OK;
 }
 
+// The largest scratch buffer of the strip kernels that the handle may allocate from now on (tests of what happens without memory)
+int cntkq_debug_set_strip_scratch_limit(cntkq_quantizer* h, size_t bytes)
+{
+    if (h == nullptr)
+        return fail(CNTKQ_INVALID_ARGUMENT, "cntkq_debug_set_strip_scratch_limit: null handle");
+    h->strip_scratch.limit = bytes;
+    return CNTKQ_OK;
+}
+
 unsigned cntkq_debug_strip_max_strips(cntkq_quantizer* h, size_t nbits, int zero_threshold_for_1bit)
 {
     if (h == nullptr || !valid_nbits(nbits) || nbits >= 32)

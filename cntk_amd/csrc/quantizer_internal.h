@@ -34,6 +34,10 @@ int cntkq_debug_set_tuning(cntkq_quantizer* h, int quantize_path, unsigned tile_
  * runs to its end: the way to test that error path. */
 int cntkq_debug_set_strip_spin_limit(cntkq_quantizer* h, unsigned limit);
 
+/* The largest scratch buffer of the strip kernels, in bytes, that the handle allocates from now on: a larger one is refused as if the
+ * device had no memory left. */
+int cntkq_debug_set_strip_scratch_limit(cntkq_quantizer* h, size_t bytes);
+
 /* The most strips per column that the strip kernels (path 6) take on the handle's device at this bit width: half of what
  * the device holds of the kernel, as the runtime's occupancy query tells (a column of more strips than half a die holds
  * has them on all eight dies), never more than 8 x 128 (0: unknown, or no strip kernel for the bit width). A strip is

@@ -58,6 +58,8 @@ struct StripScratchOwner
     bool captured = false;
     std::vector<char*> retired;
     uint32_t abandoned_seen = 0; // what the buffer's count of abandoned columns read when the host last looked
+    bool copies_refused = false; // there was no memory for copies of the records: not asked for again while the buffer stays
+    size_t limit = SIZE_MAX; // (tests: a larger buffer than this is refused as if the device's memory were used up)
 };
 
 struct LaunchTuning
@@ -578,8 +580,14 @@ inline bool strip_scratch_fits(const StripScratchOwner& o, size_t cols, size_t s
            sizeof(StripHeader) + o.groups_bytes + strip_records_bytes(cols, strips, records_each) <= o.bytes;
 }
 
+inline hipError_t strip_scratch_alloc(const StripScratchOwner& o, size_t bytes, void** p)
+{
+    return bytes > o.limit ? hipErrorOutOfMemory : hipMalloc(p, bytes);
+}
+
 // Makes the owner's buffer large enough for this launch (growing waits for the stream and clears the new buffer: the launch
-// count and every record's tag start at zero). Not possible while the stream is being captured.
+// count and every record's tag start at zero). Not possible while the stream is being captured. The old buffer is kept until the
+// larger one is there, and a failed call leaves it in use; where there is no memory for both, the new one is made without room to grow.
 inline hipError_t strip_scratch_for(StripScratchOwner& o, hipStream_t s, size_t cols, size_t strips, size_t records_each, StripScratch& out)
 {
     if (o.error_host == nullptr)
@@ -599,21 +607,17 @@ inline hipError_t strip_scratch_for(StripScratchOwner& o, hipStream_t s, size_t 
         hipError_t rc = hipStreamSynchronize(s);
         if (rc != hipSuccess)
             return rc;
-        if (o.dev != nullptr)
-        {
-            if (o.captured)
-                o.retired.push_back(o.dev); // a recorded launch may still be replayed on it
-            else
-                (void) hipFree(o.dev);
-        }
-        o.dev = nullptr;
-        o.bytes = 0;
-        o.captured = false;
-        o.abandoned_seen = 0;
         const size_t need = sizeof(StripHeader) + strip_records_bytes(cols, strips, records_each);
-        const size_t cap = std::max<size_t>((need * 2 + 8191) & ~(size_t) 4095, (size_t) 1 << 20);
+        const size_t least = (size_t) 1 << 20;
+        size_t cap = std::max((need * 2 + 8191) & ~(size_t) 4095, least);
         void* p = nullptr;
-        rc = hipMalloc(&p, cap);
+        rc = strip_scratch_alloc(o, cap, &p);
+        if (rc == hipErrorOutOfMemory)
+        {
+            (void) hipGetLastError();
+            cap = std::max((need + need / 255 + 8191) & ~(size_t) 4095, least); // (a 256th of the whole is for the finish counters)
+            rc = strip_scratch_alloc(o, cap, &p);
+        }
         if (rc != hipSuccess)
             return rc;
         rc = hipMemsetAsync(p, 0, cap, s);
@@ -624,6 +628,16 @@ inline hipError_t strip_scratch_for(StripScratchOwner& o, hipStream_t s, size_t 
             (void) hipFree(p);
             return rc;
         }
+        if (o.dev != nullptr)
+        {
+            if (o.captured)
+                o.retired.push_back(o.dev); // a recorded launch may still be replayed on it
+            else
+                (void) hipFree(o.dev);
+        }
+        o.captured = false;
+        o.copies_refused = false;
+        o.abandoned_seen = 0;
         o.dev = static_cast<char*>(p);
         o.bytes = cap;
         o.groups_bytes = (cap / 256 + 63) & ~(size_t) 63; // counters need 1/512 of what the records need
@@ -746,15 +760,17 @@ inline hipError_t launch_on_strips(hipStream_t s, size_t rows, size_t cols, size
     StripScratch scratch;
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     const bool capturing = hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
-    // (the copies of the records only where the buffer has or may get the room: without them it takes what it always took)
+    // The copies of the records only where the buffer has or may get the room; where there is no memory for them, one copy, in the buffer as
+    // it stands if that holds it.
     const uint32_t copy_shift = strip_copy_shift(c.strips);
     if (!passes && (strip_scratch_fits(o, cols, c.strips, strip_records<E>() * strip_copies(c.strips, copy_shift)) ||
-                    (tune.strip_may_allocate && !capturing)))
+                    (tune.strip_may_allocate && !capturing && !o.copies_refused)))
         c.copy_shift = copy_shift;
     hipError_t rc = strip_scratch_for(o, s, cols, c.strips, strip_records<E>() * strip_copies(c.strips, c.copy_shift), scratch);
     if (rc == hipErrorOutOfMemory && c.copy_shift != 31)
     {
         (void) hipGetLastError();
+        o.copies_refused = true;
         c.copy_shift = 31;
         rc = strip_scratch_for(o, s, cols, c.strips, strip_records<E>(), scratch);
     }

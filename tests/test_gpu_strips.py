@@ -4,6 +4,7 @@ Needs an MI355X."""
 import pytest
 import torch
 
+import cntk_amd
 import datagen
 from cntk_amd import Matrix, MatrixQuantizerImpl, QuantizedMatrix
 
@@ -76,3 +77,42 @@ def test_recorded_launch_without_room_for_copies(dtype, rows):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(Q.buffer, want[0]) and torch.equal(R.data.view(torch.uint8), want[1])
+
+
+@pytest.mark.parametrize("recorded", [False, True])
+@pytest.mark.parametrize("dtype,rows", [(F32, 102401), (F64, 51201)])
+def test_no_memory_for_copies(dtype, rows, recorded):
+    """7 strips x 4000 (2000) columns, whose records in one copy fit the starting buffer: where a larger one is refused, the launch takes that one copy in
+    the buffer it has, whether a recorded launch uses it or not; what does not fit it is refused and leaves the buffer in use."""
+    cols = 4000 if dtype == F32 else 2000
+    gen = torch.Generator(device="cuda:0")
+    gen.manual_seed(rows + 1)
+    g = torch.randn(rows * cols, generator=gen, device="cuda:0").to(dtype)
+    r = torch.zeros(rows * cols, dtype=dtype, device="cuda:0")
+    small = (rows, 40)
+    gs, rs = g[:rows * 40], r[:rows * 40]
+    want, want_small = (_quantize(MatrixQuantizerImpl.Create(0, False), *x, 1, dtype, False) for x in ((g, r, rows, cols), (gs, rs) + small))
+    qz = MatrixQuantizerImpl.Create(0, False)
+    G, R, Q = Matrix(*small, 0, gs, dtype=dtype), Matrix(*small, 0, rs.clone(), dtype=dtype), QuantizedMatrix(*small, 1, 0, dtype=dtype)
+    graph = torch.cuda.CUDAGraph()
+    if recorded:
+        with torch.cuda.graph(graph, stream=torch.cuda.Stream()):
+            qz.SetMainStream(torch.cuda.current_stream().cuda_stream)
+            qz.QuantizeAsync(G, R, Q, R, False)
+        qz.SetMainStream(torch.cuda.current_stream().cuda_stream)
+    qz._set_strip_scratch_limit(1 << 20)
+    for step in range(3):
+        got = _quantize(qz, g, r, rows, cols, 1, dtype, False)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1]), step
+        with pytest.raises(cntk_amd.QuantizerError):  # (twice the columns: more than the buffer holds even in one copy)
+            _quantize(qz, *(torch.zeros(rows * cols * 2, dtype=dtype, device="cuda:0") for _ in range(2)), rows, cols * 2, 1, dtype, False)
+        if recorded:
+            R.data.zero_()
+            Q.buffer.zero_()
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(Q.buffer, want_small[0]) and torch.equal(R.data.view(torch.uint8), want_small[1]), step
+    qz._set_strip_scratch_limit(1 << 40)
+    got = _quantize(qz, g, r, rows, cols, 1, dtype, False)
+    assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
