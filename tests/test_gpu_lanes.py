@@ -13,9 +13,12 @@ pytestmark = pytest.mark.gpu
 PATH_TILE = 1
 F32, F64 = torch.float32, torch.float64
 # heights: the first of its kernel, a column of fewer QWords than lanes, the edges of every number of lanes (160 / 161, 320 / 321, 640 / 641 floats;
-# 64 / 65, 128 / 129, 256 / 257 doubles) and of 4, 8, 16 and 20 elements per lane, the last one
+# 64 / 65, 128 / 129, 256 / 257 doubles) and of 4, 8, 16 and 20 elements per lane, the last odd one
 ROWS = {F32: [17, 31, 32, 33, 64, 65, 128, 129, 147, 160, 161, 256, 257, 320, 321, 511, 512, 513, 640, 641, 1023, 1025, 1279],
         F64: [17, 32, 33, 63, 64, 65, 127, 128, 129, 255, 256, 257, 511, 512]}
+# ... and the last height of all, every lane with 20 elements: only matrices off the 16-byte grid come here with it (an index in the list that is no multiple
+# of 4, so an offset that is none; as whole aligned pieces it is a column kernel's)
+UNALIGNED_ROWS = {F32: [1280], F64: []}
 # columns: a wavefront that is not full, workgroups with wavefronts beyond the last column, whole ones and one column more
 COLS = [1, 7, 33, 64, 65]
 CASES = [(F32, b, z) for b, z in ((1, False), (1, True), (2, False), (4, False), (8, False), (16, False))] + \
@@ -59,7 +62,7 @@ def test_quantize(dtype, nbits, zt):
     tile._set_tuning(quantize_path=PATH_TILE)
     gen = torch.Generator(device="cuda:0")
     gen.manual_seed(datagen.case_seed(nbits))
-    for n, rows in enumerate(ROWS[dtype]):
+    for n, rows in enumerate(ROWS[dtype] + UNALIGNED_ROWS[dtype]):
         for cols in COLS:
             g, r, ((Q1, R1), (Q2, R2)) = _pair(plain, tile, rows, cols, nbits, dtype, zt, gen, n % 4)
             torch.cuda.synchronize()
@@ -77,7 +80,7 @@ def test_stripe_reduce(dtype, nbits, zt, workers):
     tile._set_tuning(quantize_path=PATH_TILE)
     gen = torch.Generator(device="cuda:0")
     gen.manual_seed(datagen.case_seed(nbits) + workers)
-    for n, rows in enumerate(ROWS[dtype]):
+    for n, rows in enumerate(ROWS[dtype] + UNALIGNED_ROWS[dtype]):
         for cols in (1, 33, 65):
             kw = dict(dtype=dtype)
             stripes = []

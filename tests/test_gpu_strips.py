@@ -1,11 +1,14 @@
 """Tall columns in strips: ragged ends at every remainder, every number of copies of the strips' partial sums, and a launch whose scratch
-buffer has no room for copies. The strips in passes (nothing waits, one copy) add the same sums in the same order and are the oracle.
-Needs an MI355X."""
+buffer has no room for copies. The strips in passes (nothing waits, one copy) add the same sums in the same order and tell whether the exchange
+is right; they load a column as the single launch does, so the loads of the ragged ends are held against the CPU oracle. Needs an MI355X."""
+import numpy as np
 import pytest
 import torch
 
 import cntk_amd
 import datagen
+import oracle
+import parity
 from cntk_amd import Matrix, MatrixQuantizerImpl, QuantizedMatrix
 
 pytestmark = pytest.mark.gpu
@@ -23,6 +26,11 @@ def _quantize(qz, g, r, rows, cols, nbits, dtype, zt):
     qz.WaitQuantizeAsyncDone()
     torch.cuda.synchronize()
     return Q.buffer, R.data.view(torch.uint8)
+
+
+def _column(m, rows, j, dtype):
+    """Column j as the oracle takes it."""
+    return np.asfortranarray(m.view(dtype)[j * rows:(j + 1) * rows].cpu().numpy().reshape((rows, 1)))
 
 
 # strips per column: fewer than share a copy, the edges of 1, 2 and 3 copies, the edges of the pause before the first look (8, 27),
@@ -52,6 +60,39 @@ def test_strips_against_passes(dtype, nbits, zt):
                 qz._set_tuning(quantize_path=path)
                 outs.append(_quantize(qz, g, r, rows, cols, nbits, dtype, zt))
             assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1]), (strips, rows)
+            if strips <= 5:  # the last column, which is finite
+                packed, j = outs[0][0].cpu().numpy(), cols - 1
+                qcol = packed.size // cols
+                parity.check_quantize(_column(g, rows, j, dtype), _column(r, rows, j, dtype), packed[j * qcol:].copy(), _column(outs[0][1], rows, j, dtype), nbits, zt)
+
+
+@pytest.mark.parametrize("dtype,nbits,zt", [(F32, 1, False), (F32, 1, True), (F32, 2, False), (F32, 4, False), (F32, 8, False), (F32, 16, False),
+                                            (F64, 1, False), (F64, 4, False), (F64, 32, False)])
+def test_ragged_stripes_against_the_oracle(dtype, nbits, zt):
+    """The fused reduction of two workers' stripes of 11 strips (three copies of the records), at every kind of ragged end."""
+    qz = MatrixQuantizerImpl.Create(0, False)
+    words, per, cols, workers = WORDS[dtype][nbits], (32 if dtype == F32 else 64) // nbits, 2, 2
+    npdt = np.float32 if dtype == F32 else np.float64
+    for extra in (0, 1, 2, 3, 5, per, words * per - 1, words * per // 2 + 1):
+        rows = 10 * words * per + (extra if extra else words * per)
+        print(dtype, nbits, zt, "rows", rows, flush=True)
+        assert qz.StripeReduceTakes(rows, cols, nbits, zt, dtype)
+        zeros = np.zeros((rows, cols), npdt, order="F")
+        stripes, agg = [], None
+        for w in range(workers):
+            q, _ = oracle.quantize(datagen.normal(70 + w + extra, rows, cols, dtype=npdt), zeros, nbits, zt, threads=8)
+            Q = QuantizedMatrix(rows, cols, nbits, 0, dtype=dtype)
+            Q.from_numpy(q)
+            stripes.append(Q)
+            agg = oracle.unquantize(q, rows, cols, nbits, dtype=npdt, threads=8) if w == 0 else \
+                oracle.unquantize(q, rows, cols, nbits, out=agg, add=True, threads=8)
+        sres = datagen.normal(80 + extra, rows, cols, 0.002, dtype=npdt)
+        S, Out = Matrix.from_numpy(sres), QuantizedMatrix(rows, cols, nbits, 0, dtype=dtype)
+        Out.buffer.fill_(0xA5)
+        qz.StripeReduceAsync(stripes, 0, S, Out, zt)
+        qz.WaitStripeReduceDone()
+        torch.cuda.synchronize()
+        parity.check_quantize(agg, sres, Out.to_numpy(), S.to_numpy(), nbits, zt)
 
 
 @pytest.mark.parametrize("dtype,rows", [(F32, 102401), (F64, 51201)])
