@@ -606,8 +606,9 @@ class MatrixQuantizerImpl:
     def _set_tuning(self, quantize_path=0, tile_gs=0, unq_slots=0, unq_mode=0, tile_stage=-1):
         _check(lib().cntkq_debug_set_tuning(self._h, quantize_path, tile_gs, unq_slots, unq_mode, tile_stage))
 
-    def _set_strip_spin_limit(self, limit):
-        _check(lib().cntkq_debug_set_strip_spin_limit(self._h, limit))
+    def _set_strip_spin_limit(self, limit=None):
+        """None: as on a new handle."""
+        _check(lib().cntkq_debug_set_strip_spin_limit(self._h, 0xFFFFFFFF if limit is None else limit))
 
     def _set_strip_scratch_limit(self, nbytes):
         _check(lib().cntkq_debug_set_strip_scratch_limit(self._h, nbytes))

@@ -985,12 +985,12 @@ int cntkq_debug_set_tuning(cntkq_quantizer* h, int quantize_path, unsigned tile_
 }
 
 // How often a lane of a strip kernel polls for another workgroup's partial sum before it gives up (tests of the error path
-// set it to zero: every kernel still runs to its end).
+// set it to zero: every kernel still runs to its end; UINT_MAX: what a new handle has).
 int cntkq_debug_set_strip_spin_limit(cntkq_quantizer* h, unsigned limit)
 {
     if (h == nullptr)
         return fail(CNTKQ_INVALID_ARGUMENT, "cntkq_debug_set_strip_spin_limit: null handle");
-    h->tune.strip_spin_limit = limit;
+    h->tune.strip_spin_limit = limit == UINT32_MAX ? LaunchTuning().strip_spin_limit : limit;
     return CNTKQ_OK;
 }
 

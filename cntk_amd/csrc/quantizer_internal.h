@@ -30,7 +30,7 @@ int cntkq_debug_set_tuning(cntkq_quantizer* h, int quantize_path, unsigned tile_
                            int unq_mode, int tile_stage);
 
 /* How often a lane of a strip kernel (path 6) polls for another workgroup's partial sum before it gives up and raises the
- * error that the next cntkq_wait_quantize_done reports. Zero makes every exchange fail at once while every kernel still
+ * error that the next cntkq_wait_quantize_done reports (UINT_MAX: as often as on a new handle). Zero makes every exchange fail at once while every kernel still
  * runs to its end: the way to test that error path. */
 int cntkq_debug_set_strip_spin_limit(cntkq_quantizer* h, unsigned limit);
 

@@ -248,7 +248,7 @@ def test_tall_columns_that_never_wait():
     b.WaitQuantizeAsyncDone()
     torch.cuda.synchronize()
     assert np.array_equal(Q.to_numpy(), outs[0][0]) and parity.bits_equal(R.to_numpy(), outs[0][1])
-    b._set_strip_spin_limit(1 << 17)
+    b._set_strip_spin_limit()
     b.SetTallColumnsNeverWait(False)
     assert b.StripeReduceTakes(rows, cols, 1)
 
@@ -726,7 +726,7 @@ def test_strip_kernel_reports_workgroups_that_give_up(host_q):
     else:
         r_after = R.to_numpy()
         assert any(parity.bits_equal(r_after[:, j], r0[:, j]) for j in range(cols))
-    qz._set_strip_spin_limit(1 << 17)
+    qz._set_strip_spin_limit()
     R.data.zero_()
     qz.QuantizeAsync(G, R, Q, R, False)
     qz.WaitQuantizeAsyncDone()

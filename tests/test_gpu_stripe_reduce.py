@@ -424,7 +424,7 @@ def test_stripe_reduce_on_strips_reports_workgroups_that_give_up(dtype):
                               np.asfortranarray(s_after[:, j:j + 1]), nbits, False)
     say("   columns left untouched: %d of %d" % (untouched, n))
     assert untouched >= 1
-    qz._set_strip_spin_limit(1 << 17)
+    qz._set_strip_spin_limit()
     _, Out, S = run()
     qz.WaitStripeReduceDone()
     parity.check_quantize(agg_o, sres, Out.to_numpy(), S.to_numpy(), nbits, False)
