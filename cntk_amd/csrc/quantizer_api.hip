@@ -97,9 +97,8 @@ struct BatchAbi<float>
         return family_batch_reg_quantize(nbits, zt && nbits == 1, s, ev, de, db, members, blocks, lds, threads, wide);
     }
 
-    // Fills the geometry of a member of the quantize grid; false: the matrix gets a launch of its own. any_lds: the grid is resident as a whole
-    // whatever LDS its members take.
-    static bool quantize_member(const QItem& it, size_t nbits, QEntry& e, size_t& lds, uint64_t& blocks, bool any_lds)
+    // Fills the geometry of a member of the quantize grid; false: the matrix gets a launch of its own.
+    static bool quantize_member(const QItem& it, size_t nbits, QEntry& e, size_t& lds, uint64_t& blocks, const SetGrid& grid)
     {
         const int path = quantize_auto_path(it.in, it.res_in, it.res_out, it.qbuf, it.rows, nbits);
         if (path == kPathTile && short_applicable(it.rows, it.cols, qwords_per_col(it.rows, nbits)))
@@ -113,7 +112,7 @@ struct BatchAbi<float>
         if (path == kPathTile)
         {
             const TileGeom t = make_tile_geom(it.rows, it.cols, nbits, 0, -1, 0);
-            if (lanes_member<float>(it.rows, it.cols, nbits, t.gs, tile_lds_bytes(t, 0), any_lds))
+            if (lanes_member<float>(it.rows, it.cols, nbits, t.gs, tile_lds_bytes(t, 0), grid))
             {
                 e.kind = 14;
                 e.l = make_lanes_geom<float>(it.rows, it.cols, nbits, t.gs);
@@ -486,7 +485,24 @@ int quantize_batch_noalloc_impl(cntkq_quantizer* h, const cntkq_quantize_item* i
         static_assert(sizeof(Entry) == CNTKQ_NOALLOC_ENTRY_BYTES, "the public header states the size of a table entry");
         static_assert(CNTKQ_NOALLOC_MAX_ITEMS * (sizeof(Entry) + sizeof(uint32_t)) + 2 * sizeof(uint32_t) <= kNoAllocScratchBytes,
                       "a list of the largest permitted size fits the fixed array");
-        // pass 1: count the members, so that the two classes can be laid out one after the other
+        // pass 1: what stands beside the short members
+        SetGrid grid;
+        for (size_t i = 0; i < count; ++i)
+        {
+            const cntkq_quantize_item& it = items[i];
+            if (it.rows == 0 || it.cols == 0)
+                continue;
+            Entry e;
+            std::memset(&e, 0, sizeof e);
+            size_t lds = 0;
+            uint64_t blocks = 0;
+            if (!A::quantize_member(it, nbits, e, lds, blocks, SetGrid()))
+                continue;
+            const bool staged = A::first_in_grid(e);
+            grid.staged = grid.staged || staged;
+            grid.elements += staged ? 0 : it.rows * it.cols;
+        }
+        // pass 2: count the members, so that the two classes can be laid out one after the other
         size_t members[2] = {0, 0};
         for (size_t i = 0; i < count; ++i)
         {
@@ -497,7 +513,7 @@ int quantize_batch_noalloc_impl(cntkq_quantizer* h, const cntkq_quantize_item* i
             std::memset(&e, 0, sizeof e);
             size_t lds = 0;
             uint64_t blocks = 0;
-            if (A::quantize_member(it, nbits, e, lds, blocks, false))
+            if (A::quantize_member(it, nbits, e, lds, blocks, grid))
                 members[lds <= kBatchSmallLds ? 0 : 1]++;
         }
         const bool single = members[0] + members[1] == 1; // a grid of its own is nothing to share: plain launch
@@ -527,7 +543,7 @@ int quantize_batch_noalloc_impl(cntkq_quantizer* h, const cntkq_quantize_item* i
                 std::memset(&en, 0, sizeof en);
                 size_t lds = 0;
                 uint64_t blocks = 0;
-                if (!A::quantize_member(it, nbits, en, lds, blocks, false) || (lds <= kBatchSmallLds ? 0 : 1) != cls)
+                if (!A::quantize_member(it, nbits, en, lds, blocks, grid) || (lds <= kBatchSmallLds ? 0 : 1) != cls)
                     continue;
                 en.g = it.in;
                 en.r_in = it.res_in;
@@ -554,7 +570,7 @@ int quantize_batch_noalloc_impl(cntkq_quantizer* h, const cntkq_quantize_item* i
             Entry en;
             size_t lds = 0;
             uint64_t blocks = 0;
-            if (single || !A::quantize_member(it, nbits, en, lds, blocks, false))
+            if (single || !A::quantize_member(it, nbits, en, lds, blocks, grid))
                 st.own[st.own_count++] = i;
         }
         st.entries_bytes = entries_bytes;
@@ -1045,6 +1061,11 @@ int cntkq_debug_lanes(size_t rows, size_t cols, size_t nbits, size_t workers)
     const TileGeom t = make_tile_geom(rows, cols, nbits, 0, -1, 0);
     return (workers == 0 ? lanes_applicable<float>(rows, cols, nbits, t.gs)
                          : lanes_stripe_applicable<float>(rows, cols, nbits, t.gs, workers, tile_lds_bytes(t, (uint32_t) workers))) ? 1 : 0;
+}
+
+int cntkq_debug_lanes_beside_staged(size_t rows, size_t elements)
+{
+    return lanes_beside_staged(rows, elements) ? 1 : 0;
 }
 
 size_t cntkq_debug_staged_max_rows(size_t nbits)

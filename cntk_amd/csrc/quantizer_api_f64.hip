@@ -56,7 +56,7 @@ struct BatchAbi<double>
 
     // members of the general grid are runs of column tiles, small matrices of the element-wise register kernel among them, which run the
     // tile body (the same bytes); columns on 1024 threads are members of the register grid below, the rest gets launches of its own
-    static bool quantize_member(const QItem& it, size_t nbits, QEntry& e, size_t& lds, uint64_t& blocks, bool any_lds)
+    static bool quantize_member(const QItem& it, size_t nbits, QEntry& e, size_t& lds, uint64_t& blocks, const SetGrid& grid)
     {
         const int path = f64::quantize_auto_path(it.in, it.res_in, it.res_out, it.rows, nbits);
         if (path != kPathTile && !(path == kPathRegScalar && it.rows * it.cols < kOwnLaunchElements))
@@ -66,7 +66,7 @@ struct BatchAbi<double>
         if (lds > f64::kMaxLdsBytes)
             return false;
         blocks = (e.t.cols + e.t.cols_per_tile - 1) / e.t.cols_per_tile;
-        if (path == kPathTile && lanes_member<double>(it.rows, it.cols, nbits, e.t.gs, lds, any_lds))
+        if (path == kPathTile && lanes_member<double>(it.rows, it.cols, nbits, e.t.gs, lds, grid))
         {
             e.kind = 14;
             e.l = make_lanes_geom<double>(it.rows, it.cols, nbits, e.t.gs);

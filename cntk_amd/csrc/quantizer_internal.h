@@ -54,6 +54,9 @@ int cntkq_debug_short_columns_f64(size_t rows, size_t cols, size_t nbits);
 int cntkq_debug_decoder(size_t rows, size_t cols, size_t nbits, int packed_on_host);
 int cntkq_debug_decoder_f64(size_t rows, size_t cols, size_t nbits, int packed_on_host);
 
+/* Whether a short member of a set may be on lanes beside a column staged in memory and this many elements of other members. Needs no device. */
+int cntkq_debug_lanes_beside_staged(size_t rows, size_t elements);
+
 /* Whether an aligned stripe of a set is a member of the register grids, and the height up to which few tall columns of a set stay
  * staged in memory rather than have a register grid launched for them. Need no device. */
 int cntkq_debug_stripe_shares_register_grid(size_t rows, size_t cols, size_t nbits, size_t workers);

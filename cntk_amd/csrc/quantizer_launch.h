@@ -266,16 +266,33 @@ inline bool lanes_stripe_applicable(size_t rows, size_t cols, size_t nbits, uint
     return n <= (rows >= 32 ? 512 * K : 128 * K) && workers <= (nbits <= 4 ? 8u : 5u);
 }
 
+// What a set's grid is to a short member of it
+struct SetGrid
+{
+    bool resident = false; // all its workgroups are on the device at once, whatever LDS its members take
+    bool staged = false;   // with a column staged in memory, whose three passes take long,
+    size_t elements = 0;   // ... and so many elements of other members beside it
+};
+
+// Beside a column staged in memory, which the grid waits for at its end, the loads of lanes, all at once, hold that column up: until the other
+// members take longer than it does, they are the better the more slowly they load. Tiles / lanes at 1 and 2 bits beside 1 x 6592 and 3 x 8000 rows: 142 and
+// 300 rows 0.93 to 0.98 at 2 M elements, 0.85 to 0.93 at 4.5 M, 0.85 to 0.98 at 6 and 8 M, 0.98 to 1.1 at 10 M; 48, 64, 512, 900 rows 0.92 to 1.0, 0.91 to
+// 1.0, 0.89 to 1.06, 0.93 to 1.24; up to 32 rows 0.94 to 1.06, 0.98 to 1.42, 0.97 to 1.56, 1.1 to 1.8.
+inline bool lanes_beside_staged(size_t rows, size_t elements)
+{
+    return rows <= 32 || elements >= (size_t) (rows >= 128 && rows <= 400 ? 8 : 5) << 20;
+}
+
 // Short columns of a set to be quantized: all workgroups of a grid are given the LDS of its largest member, and members above 20 KB may
 // cost a launch of their own. The records in LDS, which the tile kernels need at 1 and 2 bits only, take many heights across that
 // line (147 rows at 4 bits 19.1 -> 21.6 KB, 512 at 8 bits 16.7 -> 20.6, 147 at 16 bits 19.1 -> 28.6). There the member is a tile, unless all
-// of the grid is resident at once anyway (any_lds). Lanes everywhere / by this rule, us: ResNet-50 at 4, 8, 16 bits 57.0 / 57.0, 60.6 / 59.1, 71.6 / 63.3,
+// of the grid is resident at once anyway. Lanes everywhere / by this rule, us: ResNet-50 at 4, 8, 16 bits 57.0 / 57.0, 60.6 / 59.1, 71.6 / 63.3,
 // without allocation 63.2 / 56.4, 63.7 / 57.3, 70.3 / 62.0; the stripes of one worker 53.1 / 53.6, 60.9 / 58.7, 75.8 / 66.1.
 template <typename E>
-inline bool lanes_member(size_t rows, size_t cols, size_t nbits, uint32_t lanes, size_t tile_lds, bool any_lds)
+inline bool lanes_member(size_t rows, size_t cols, size_t nbits, uint32_t lanes, size_t tile_lds, const SetGrid& grid)
 {
-    return lanes_applicable<E>(rows, cols, nbits, lanes) &&
-           (any_lds || lds_workgroups(lanes_lds_bytes<E>(make_lanes_geom<E>(rows, cols, nbits, lanes), 0)) >= lds_workgroups(tile_lds));
+    return lanes_applicable<E>(rows, cols, nbits, lanes) && (!grid.staged || lanes_beside_staged(rows, grid.elements)) &&
+           (grid.resident || lds_workgroups(lanes_lds_bytes<E>(make_lanes_geom<E>(rows, cols, nbits, lanes), 0)) >= lds_workgroups(tile_lds));
 }
 
 // ... of a set's stripes, among which a stripe's size says little about how full the device is: a single worker's (ResNet-50's at 1

@@ -193,6 +193,13 @@ def test_stripes_on_lanes_by_workers(rows, n, nbits, most):
     assert [k for k in range(1, 65) if on_lanes(rows, n, nbits, k)] == list(range(1, most + 1))
 
 
+def test_short_members_beside_a_staged_column():
+    """142 x 31690 at 1 bit beside 3 columns of 8000 rows staged in memory (4.5 M elements): 16.8 us with tiles, 19.3 on lanes; 10 M 26.8 and 26.3."""
+    L = cntk_amd.lib()
+    for rows, least in ((17, 0), (32, 0), (33, 5), (127, 5), (128, 8), (400, 8), (401, 5), (1279, 5)):
+        assert L.cntkq_debug_lanes_beside_staged(rows, least << 20) and not (least and L.cntkq_debug_lanes_beside_staged(rows, (least << 20) - 1))
+
+
 def test_large_stripes_on_lanes():
     """One and two workers above 1 M elements: with no fewer workgroups to a compute unit than tiles have (319 x 25078 at 16 bits: 28.8 us with tiles, 33.8 on
     lanes), two of them at 4 bits and more with most of a lane's elements there (65 x 46153 at 8 bits: 14.3 and 15.1 us)."""
