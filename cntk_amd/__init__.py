@@ -121,7 +121,7 @@ def lib():
         L.cntkq_debug_decoder.argtypes = L.cntkq_debug_decoder_f64.argtypes = [_sz, _sz, _sz, ctypes.c_int]
         L.cntkq_debug_lanes.argtypes = L.cntkq_debug_lanes_f64.argtypes = [_sz, _sz, _sz, _sz]
         L.cntkq_debug_lanes_beside_staged.argtypes = [_sz, _sz]
-        L.cntkq_debug_set_member.argtypes = L.cntkq_debug_set_member_f64.argtypes = [_sz, _sz, _sz, _sz, ctypes.POINTER(_sz)]
+        L.cntkq_debug_set_member.argtypes = L.cntkq_debug_set_member_f64.argtypes = [_sz, _sz, _sz, _sz, ctypes.c_int, ctypes.POINTER(_sz)]
         L.cntkq_debug_stripe_shares_register_grid.argtypes = [_sz, _sz, _sz, _sz]
         L.cntkq_debug_staged_max_rows.argtypes = [_sz]
         L.cntkq_debug_staged_max_rows.restype = _sz

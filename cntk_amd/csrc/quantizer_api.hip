@@ -1049,10 +1049,10 @@ int cntkq_debug_stripe_shares_register_grid(size_t rows, size_t cols, size_t nbi
 }
 
 // The kind of member (QuantizeBatchEntry, StripeBatchEntry) that a matrix or stripe of whole aligned pieces is in the general grids, and its LDS;
-// -1: none of them. workers 0: quantized.
-int cntkq_debug_set_member(size_t rows, size_t cols, size_t nbits, size_t workers, size_t* lds)
+// -1: none of them. workers 0: quantized. resident: all of the grid's workgroups are on the device at once.
+int cntkq_debug_set_member(size_t rows, size_t cols, size_t nbits, size_t workers, int resident, size_t* lds)
 {
-    return debug_set_member<float>(rows, cols, nbits, workers, lds);
+    return debug_set_member<float>(rows, cols, nbits, workers, resident != 0, lds);
 }
 
 // Whether a plain call that the tile kernels could take runs on lanes (workers 0: quantize)

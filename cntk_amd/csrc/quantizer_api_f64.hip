@@ -219,9 +219,9 @@ int cntkq_debug_lanes_f64(size_t rows, size_t cols, size_t nbits, size_t workers
                          : lanes_stripe_applicable<double>(rows, cols, nbits, t.gs, workers, f64::tile_lds_bytes(t, (uint32_t) workers))) ? 1 : 0;
 }
 
-int cntkq_debug_set_member_f64(size_t rows, size_t cols, size_t nbits, size_t workers, size_t* lds)
+int cntkq_debug_set_member_f64(size_t rows, size_t cols, size_t nbits, size_t workers, int resident, size_t* lds)
 {
-    return debug_set_member<double>(rows, cols, nbits, workers, lds);
+    return debug_set_member<double>(rows, cols, nbits, workers, resident != 0, lds);
 }
 
 size_t cntkq_qwords_per_col_f64(size_t rows, size_t nbits)

@@ -296,12 +296,17 @@ inline bool lanes_member(size_t rows, size_t cols, size_t nbits, uint32_t lanes,
 }
 
 // ... of a set's stripes, among which a stripe's size says little about how full the device is: a single worker's (ResNet-50's at 1
-// bit with one worker 50.9 -> 49.2 us, at 4 bits with eight 92 -> 96)
+// bit with one worker 50.9 -> 49.2 us, at 4 bits with eight 92 -> 96). Where all of the grid is resident the LDS costs nothing, however large the
+// stripe (300 x 3685, 7425 x 4 and 512 x 512 at 4 bits 21.2 us with 300 rows as tiles, 17.7 on lanes).
 template <typename E>
 inline bool lanes_stripe_member(size_t rows, size_t cols, size_t nbits, uint32_t lanes, size_t workers, size_t tile_lds, bool any_lds)
 {
-    return workers == 1 && lanes_stripe_applicable<E>(rows, cols, nbits, lanes, workers, tile_lds) &&
-           (any_lds || lds_workgroups(lanes_lds_bytes<E>(make_lanes_geom<E>(rows, cols, nbits, lanes), workers)) >= lds_workgroups(tile_lds));
+    if (workers != 1 || (sizeof(E) == 4 && rows < 32 && rows * cols > 256 * 1024))
+        return false;
+    if (any_lds)
+        return lanes_hold<E>(rows, nbits, lanes);
+    return lanes_stripe_applicable<E>(rows, cols, nbits, lanes, workers, tile_lds) &&
+           lds_workgroups(lanes_lds_bytes<E>(make_lanes_geom<E>(rows, cols, nbits, lanes), workers)) >= lds_workgroups(tile_lds);
 }
 
 inline uint32_t lanes_blocks(const LanesGeom& t)

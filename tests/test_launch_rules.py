@@ -120,11 +120,11 @@ TILES, COLUMNS, STAGED, REGISTERS_6, LANES = 0, 1, 5, 7, 14
 SMALL_LDS = 20480  # eight workgroups in a compute unit; a set's members above it may get a launch of their own
 
 
-def member(rows, nbits, workers=0, double=0, cols=100):
-    """(kind, bytes of LDS) of a member of a set's general grid."""
+def member(rows, nbits, workers=0, double=0, cols=100, resident=0):
+    """(kind, bytes of LDS) of a member of a set's general grid, one that fills the device or one that is resident as a whole."""
     L = cntk_amd.lib()
     lds = ctypes.c_size_t()
-    kind = (L.cntkq_debug_set_member_f64 if double else L.cntkq_debug_set_member)(rows, cols, nbits, workers, ctypes.byref(lds))
+    kind = (L.cntkq_debug_set_member_f64 if double else L.cntkq_debug_set_member)(rows, cols, nbits, workers, resident, ctypes.byref(lds))
     return kind, lds.value
 
 
@@ -158,6 +158,17 @@ def test_short_members_on_lanes():
     lanes = {rows: [b for b in (1, 2, 4, 8, 16) if member(rows, b)[0] == LANES] for rows in (33, 64, 128, 147, 256, 512, 576)}
     assert lanes == {33: [1, 2, 4, 8, 16], 64: [1, 2, 4, 8, 16], 128: [1, 2, 4], 147: [1, 2], 256: [1, 2, 4], 512: [1, 2, 4], 576: [1, 2]}
     assert [b for b in (1, 2, 4, 8, 16) if member(147, b, 1)[0] == LANES] == [1, 2] and member(147, 1, 2)[0] == TILES
+
+
+@pytest.mark.parametrize("workers", [0, 1])
+def test_short_members_of_a_resident_grid(workers):
+    """Their LDS costs nothing: on lanes whatever it is, also stripes of more than 1 M elements (300 x 3685 at 4 bits)."""
+    for nbits in (1, 2, 4, 8, 16):
+        for rows, cols in ((17, 1000), (147, 100), (300, 3685), (512, 512), (576, 2000), (1023, 1500)):
+            assert member(rows, nbits, workers, cols=cols, resident=1)[0] == LANES
+            assert member(min(rows, 512), nbits, workers, double=1, cols=cols, resident=1)[0] == LANES
+    assert member(300, 4, 1, cols=3685)[0] == TILES and member(31, 1, 1, cols=10000, resident=1)[0] == TILES
+    assert member(300, 4, 2, cols=100, resident=1)[0] == TILES
 
 
 @pytest.mark.parametrize("nbits", [1, 2, 4, 8, 16])
